@@ -8,8 +8,8 @@
 // Layout (row-major, no strides): q/out [B,S,H,D], k/v [B,S,KV,D], lengths u32[B].
 //
 // Three kernels:
-//   attn_scalar      one wavefront per (token, head); any D <= 256. Routes "attention" and
-//                    "attention_f16_scalar".
+//   attn_scalar      one wavefront per (token, head); any D <= 256. Route "attention_f16_scalar",
+//                    and route "attention" where attn_f32x3 does not take the head size.
 //   attn_f32_ring    fp32 MFMA (v_mfma_f32_32x32x2_f32) tiles on an LDS DMA ring, D in {32,64};
 //   attn_f32_split   the same fp32 MFMA arithmetic for D = 128, keys split over two wavefronts
 //                    per row block and merged in fixed order; any S.
@@ -1539,15 +1539,22 @@ struct X3Args {
   const uint32_t* lengths;
   float* out;
   int B, S, H, KV;
-  float scale_log2;
+  float scale_log2, scale_log2_lo;  // scale * log2(e) as the sum of two floats
   int bidi;
   F16Shape shp;
 };
 
-template <int D>
+// fp32 attention on bf16 MFMA, the split products summed by size: one accumulator for the leading
+// ones and one for the smaller ones, so that only the leading products round at the magnitude of
+// the result. SEP: P V too (its smaller products in ol), and two leading accumulators per score at
+// D > 32. Error against float64 (normal inputs, S 24 / 41 / 63 at D 128 / 32 / 64): 0.96, 1.5 and
+// 1.6e-7 with SEP, 1.5, 2.6 and 2.6e-7 with every product in one chain; attn_scalar 0.95, 1.8 and
+// 2.1e-7.
+template <int D, bool SEP>
 __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   static_assert(D == 32 || D == 64 || D == 128, "the split-bf16 fp32 kernel serves D = 32, 64, 128");
   // KT keys per tile: every tile is 8 KiB of fp32 per tensor, 8 channels of one row per thread
+  constexpr int NH = SEP && D > 32 ? 2 : 1;
   constexpr int KT = 2048 / D, NKB = KT / 16, NS = D / 32, NDT = D / 16, CPR = D / 8;
   constexpr int TILE = KT * D;                       // elements per K or V tile
   constexpr int SPLIT_BYTES = 2 * 2 * 3 * TILE * 2;  // [buffer][K, V][plane] bf16
@@ -1561,7 +1568,6 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   const Sched sc = schedule(a.lengths, a.B, a.S, a.KV, a.shp.kv, a.shp.wpp, a.shp.serp);
   const Geom16 g = geom16_of(sc, a.bidi, wave, a.shp);
   const int S = a.S, H = a.H, KV = a.KV;
-  const float scale_log2 = a.scale_log2;
   int tid = static_cast<int>(threadIdx.x);
   asm volatile("" : "+v"(tid));
   const int lane = tid & 63, r = lane & 15, gq = lane >> 4;
@@ -1615,8 +1621,15 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   bf16x8 q1[NS], q2[NS], q3[NS];
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const floatx4 x0 = *reinterpret_cast<const floatx4*>(qrow + qoff + 32 * s);
-    const floatx4 x1 = *reinterpret_cast<const floatx4*>(qrow + qoff + 32 * s + 4);
+    floatx4 x0 = *reinterpret_cast<const floatx4*>(qrow + qoff + 32 * s);
+    floatx4 x1 = *reinterpret_cast<const floatx4*>(qrow + qoff + 32 * s + 4);
+    // q * scale * log2(e), rounded once: the scores come out as base-2 exponents, with no product
+    // per score and without the rounding error of the constant, which every score would share
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x0[j] = fmaf(x0[j], a.scale_log2, x0[j] * a.scale_log2_lo);
+      x1[j] = fmaf(x1[j], a.scale_log2, x1[j] * a.scale_log2_lo);
+    }
     uint4v w1, w2, w3;
     split3x8(x0, x1, w1, w2, w3);
     q1[s] = __builtin_bit_cast(bf16x8, w1);
@@ -1625,9 +1638,12 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   }
   // Rows past S read row S - 1 (finite data) and are never stored.
 
-  floatx4 o[NDT];
+  floatx4 o[NDT], ol[SEP ? NDT : 1];  // ol: the smaller products of P and V
 #pragma unroll
-  for (int dt = 0; dt < NDT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < NDT; ++dt) {
+    o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    if constexpr (SEP) ol[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
   float m_run = -INFINITY, l_run = 0.0f;
 
   auto rescale = [&](float d) {
@@ -1635,7 +1651,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
     const float corr = __builtin_amdgcn_exp2f(d);
     l_run *= corr;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) o[dt] *= corr;
+    for (int dt = 0; dt < NDT; ++dt) {
+      o[dt] *= corr;
+      if constexpr (SEP) ol[dt] *= corr;
+    }
   };
 
   // tile kt from split buffer buf; sc[kb][j] is key 16 kb + 4g + j of the tile
@@ -1644,7 +1663,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
     floatx4 sc[NKB];
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
-      floatx4 acc[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+      // the leading products in one accumulator (SEP: two, where D has several k-steps), the five
+      // smaller ones in another: their sums do not round at the magnitude of the score
+      floatx4 hi[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+      floatx4 lo = {0.f, 0.f, 0.f, 0.f};
       const int row = 16 * kb + r, rbase = row * D, ksw = ksw_x3<D>(row);
 #pragma unroll
       for (int s = 0; s < NS; ++s) {
@@ -1652,16 +1674,20 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
         const bf16x8 k1 = *reinterpret_cast<const bf16x8*>(k1p + off);
         const bf16x8 k2 = *reinterpret_cast<const bf16x8*>(k1p + TILE + off);
         const bf16x8 k3 = *reinterpret_cast<const bf16x8*>(k1p + 2 * TILE + off);
-        floatx4& c = acc[(s + kb) & 1];
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q1[s], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q2[s], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q1[s], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q3[s], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q2[s], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k3, q1[s], c, 0, 0, 0);
+        floatx4& h = hi[NH > 1 && 2 * s >= NS ? 1 : 0];
+        h = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q1[s], h, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k3, q1[s], lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q2[s], lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q3[s], lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q1[s], lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q2[s], lo, 0, 0, 0);
       }
-      mfma_result_fence(acc[0], acc[1]);
-      sc[kb] = acc[0] + acc[1];
+      mfma_result_fence(hi[0], lo);
+      if constexpr (NH > 1) {
+        mfma_result_fence(hi[1]);
+        hi[0] += hi[1];
+      }
+      sc[kb] = hi[0] + lo;
     }
     if (kt * KT + KT > g.limit_min) {
 #pragma unroll
@@ -1674,7 +1700,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
 #pragma unroll
     for (int kb = 1; kb < NKB; ++kb)
       mx = fmaxf(mx, fmaxf(fmaxf(sc[kb][0], sc[kb][1]), fmaxf(sc[kb][2], sc[kb][3])));
-    const float mloc = rowmax4(mx) * scale_log2;
+    const float mloc = rowmax4(mx);
     const bool grow = mloc > m_run + kMaxSlack;
     // every row sees key 0 in its first tile (L >= 1), so m_new is finite from tile 0 on
     const float m_new = grow ? mloc : m_run;
@@ -1689,7 +1715,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
       uint32_t u0[4], u1[4], u2[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        pf[j] = __builtin_amdgcn_exp2f(fmaf(sc[kb][j], scale_log2, -m_new));
+        pf[j] = __builtin_amdgcn_exp2f(sc[kb][j] - m_new);
         u0[j] = __float_as_uint(pf[j]);
         const float r1 = pf[j] - __uint_as_float(u0[j] & 0xffff0000u);
         u1[j] = __float_as_uint(r1);
@@ -1734,8 +1760,9 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
         const bf16x8 a31 =
             __builtin_bit_cast(bf16x8, __builtin_shufflevector(vt, vt, 0, 1, 2, 3, 4, 5, 6, 7));
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a12, bp11, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a12, bp22, o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a31, bp13, o[dt], 0, 0, 0);
+        floatx4& lo = SEP ? ol[dt] : o[dt];
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a31, bp13, lo, 0, 0, 0);
+        lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a12, bp22, lo, 0, 0, 0);
       }
     }
   };
@@ -1761,7 +1788,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
     if (kt + 1 < ntiles) step(kt + 1, Stage<1>{});
   }
   wait_lgkmcnt<0>();
-  const float inv = __builtin_amdgcn_rcpf(rowsum4(l_run));
+  const float l_row = rowsum4(l_run), inv = __builtin_amdgcn_rcpf(l_row);
   stage_barrier();
 
   // ---- epilogue: fragments -> row-major rows in LDS -> full-row stores (as attn_f16_mfma) ----
@@ -1772,8 +1799,17 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   {
     char* const orow = ob + r * RS;
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt)
-      *reinterpret_cast<floatx4*>(orow + 4 * (16 * dt + 4 * gq)) = o[dt] * inv;
+    for (int dt = 0; dt < NDT; ++dt) {
+      if constexpr (SEP) o[dt] += ol[dt];
+      // o / l (SEP: the estimate's quotient corrected by its remainder)
+      floatx4 q;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        q[j] = o[dt][j] * inv;
+        if constexpr (SEP) q[j] = fmaf(fmaf(-q[j], l_row, o[dt][j]), inv, q[j]);
+      }
+      *reinterpret_cast<floatx4*>(orow + 4 * (16 * dt + 4 * gq)) = q;
+    }
   }
   const int lo = lane / OCH, hmask = (1 << g.hsh) - 1;
   const uint32_t voff =
@@ -1845,10 +1881,20 @@ bool attention_scalar_fits(uint64_t B, uint64_t S, uint64_t H) {
   return B * S * H * 64 < (1ull << 32);
 }
 
+static bool attention_f32x3_fits(int B, int S, int H, int KV, int D);
+
 hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   if (!attention_scalar_fits(a.B, a.S, a.H)) return hipErrorInvalidValue;
   const unsigned grid = static_cast<unsigned>(a.B * a.S * a.H);
   if (!grid) return hipSuccess;
+  // fp32 rows of a head size that attn_f32x3 tiles (32, 64, 128) run there from 16 keys on:
+  // attn_scalar's keys are a serial chain of wave reductions, about 1.25 us each whatever the
+  // batch (24 tokens of 16 heads 30.9 against 8.0 us, 16 x 41 tokens of 12 heads 39.6 against
+  // 9.1 us per launch). Under 16 keys the chain is as short as the tile's latency.
+  if (a.S >= 16 && !a.in_f16 && !a.out_f16 &&
+      attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D) &&
+      attention_f32_fits(a.B, a.S, a.H, a.KV))
+    return launch_attention_f32(a, st);
   const float scale = a.scale;
   if (!a.in_f16 && !a.out_f16)
     attn_scalar<float, float><<<grid, 64, 0, st>>>(
@@ -1930,19 +1976,27 @@ hipError_t launch_attention_f32(const AttnArgs& a, hipStream_t st) {
     x.S = a.S;
     x.H = a.H;
     x.KV = a.KV;
-    x.scale_log2 = sl2;
+    const double c = static_cast<double>(a.scale) * 1.4426950408889634073599;
+    x.scale_log2 = static_cast<float>(c);
+    x.scale_log2_lo = static_cast<float>(c - static_cast<double>(x.scale_log2));
     x.bidi = a.bidi;
     x.shp = f16_shape(a.B, a.S, a.H, a.KV);
     const dim3 grid = sched_grid(a.B, a.KV, (x.shp.nwb + 3) / 4);
     switch (a.D) {
       case 32:
-        attn_f32x3<32><<<grid, 256, 0, st>>>(x);
+        attn_f32x3<32, true><<<grid, 256, 0, st>>>(x);
         break;
       case 64:
-        attn_f32x3<64><<<grid, 256, 0, st>>>(x);
+        attn_f32x3<64, true><<<grid, 256, 0, st>>>(x);
         break;
       default:
-        attn_f32x3<128><<<grid, 256, 0, st>>>(x);
+        // short rows (the calls that ran on attn_scalar) keep the smaller products of P and V
+        // in accumulators of their own, at 184 registers (two workgroups per CU) against 152
+        // (three), which long rows need: 67 against 83 us at 8 x 512
+        if (a.S < 64)
+          attn_f32x3<128, true><<<grid, 256, 0, st>>>(x);
+        else
+          attn_f32x3<128, false><<<grid, 256, 0, st>>>(x);
         break;
     }
     return hipGetLastError();

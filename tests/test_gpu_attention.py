@@ -95,6 +95,25 @@ def test_bge_small_c1_through_route(runtime):
     assert got.reshape(2, 16, 384).shape == (2, 16, 384)
 
 
+@pytest.mark.parametrize("dim,heads,kv", [(32, 12, 12), (64, 4, 2), (128, 16, 8), (128, 3, 1),
+                                          (96, 4, 2)])
+@pytest.mark.parametrize("bidirectional", [False, True])
+@pytest.mark.parametrize("seq,length_pair", [(1, (1, 1)), (2, (2, 1)), (15, (15, 7)), (16, (1, 16)),
+                                             (17, (17, 16)), (41, (33, 41)), (63, (63, 32))])
+def test_short_sequences_on_the_scalar_route(runtime, dim, heads, kv, bidirectional, seq,
+                                             length_pair):
+    """Route "attention" at the tile edges of the MFMA kernel that serves head sizes 32, 64 and 128
+    there from 16 keys on (16, 32, 64 keys a tile), below that, and a head size it does not take."""
+    rng = np.random.default_rng(seq * 131 + dim)
+    q = rng.normal(size=(2, seq, heads, dim)).astype(np.float32)
+    k, v = [rng.normal(size=(2, seq, kv, dim)).astype(np.float32) for _ in range(2)]
+    lengths = np.array(length_pair, np.uint32)
+    got = run(runtime, "attention", [q, k, v, lengths], q.shape, threads=2 * seq * heads * 32,
+              group_size=32, seq=seq, heads=heads, kv_heads=kv, dim=dim, scale=dim**-0.5,
+              bidirectional=bidirectional)
+    check_f32(got, ref.attention(q, k, v, lengths, bidirectional=bidirectional))
+
+
 @pytest.mark.parametrize("dim", [32, 128])
 @pytest.mark.parametrize("bidirectional", [False, True])
 @pytest.mark.parametrize(
