@@ -80,19 +80,27 @@ hipError_t launch_norm_rope_f16(const _Float16* x, _Float16* y, const uint16_t* 
                                 const uint32_t* lengths, int B, int S, int heads, int D,
                                 float eps, bool split, hipStream_t st);
 
-// uint4 affine group-64 projection, fp32 activations, bf16 scale/bias (tessery linear4 family,
-// kernels.metal:11-19, 32-51, 489-605, 655-684, 733-773). Computes rows [row0, row1).
-// With few output tiles and a scratch buffer, K is split over workgroups (partial sums added in a
-// fixed order by a second kernel), as for the dense projections.
-hipError_t launch_linear4_f32(const float* x, const uint32_t* w, const uint16_t* scales,
-                              const uint16_t* biases, float* out, int row0, int row1, int cols,
-                              int k, float* scratch, size_t scratch_floats, hipStream_t st);
-// Gate and up projections of rows [row0, row1) with out = silu(gate) * up (tessery gated4,
-// kernels.metal:609-656, 687-731), bit-identical to linear4 + linear4 + silu_gate.
-hipError_t launch_gated4_f32(const float* x, const uint32_t* w, const uint16_t* scales,
-                             const uint16_t* biases, const uint32_t* uw, const uint16_t* uscales,
-                             const uint16_t* ubiases, float* out, int row0, int row1, int cols,
-                             int k, float* scratch, size_t scratch_floats, hipStream_t st);
+// One uint4 affine group-64 projection, fp32 activations, bf16 scale/bias (tessery linear4 family,
+// kernels.metal:11-19, 32-51, 489-605, 655-684, 733-773): rows [row0, row1) of out = x W^T, x and
+// out being whole matrices (row 0 first).
+struct Linear4Job {
+  const float* x;
+  const uint32_t* w;
+  const uint16_t* scales;
+  const uint16_t* biases;
+  float* out;
+  int row0, row1, cols, k;
+};
+hipError_t launch_linear4_f32(const Linear4Job& job, float* scratch, size_t scratch_floats,
+                              hipStream_t st);
+// Whether launch_linear4_f32 runs the job on linear4_rows, whose results depend neither on the rows
+// of the launch nor on the projections beside it.
+bool linear4_on_rows(const Linear4Job& job, const float* scratch, size_t scratch_floats);
+// One to three projections of the same rows of one x in one linear4_rows launch, with the bits of
+// separate ones. With `gated` (two jobs of equal width: gate, up): out of the gate takes
+// silu(gate) * up (tessery gated4, kernels.metal:609-656, 687-731), out of the up projection, when
+// not null, its own values, as linear4 + linear4 + silu_gate leave them.
+hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated, hipStream_t st);
 // The same projection for M >= kLinear4HiloRows rows on fp16 MFMA: rows scaled by powers of two
 // and split into hi + lo fp16 halves (about 22 bits), exact codes, fp32 sums. scratch holds the M
 // row scales. x and y start at row 0 of the range; N % 128 == 0, K % 64 == 0.

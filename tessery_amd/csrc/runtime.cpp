@@ -9,6 +9,7 @@
 // from the reference thread formula and checks every buffer size before it may be queued.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <cstdlib>
@@ -653,6 +654,44 @@ bool attention_args(Runtime* rt, const Op& op, tessery::AttnArgs* out) {
   return true;
 }
 
+bool is_linear4(Route r) {
+  return r == R_LINEAR4 || r == R_LINEAR4_TILED || r == R_LINEAR4_TAIL || r == R_LINEAR4_16X32 ||
+         r == R_LINEAR4_32X32 || r == R_LINEAR4_SMALL3;
+}
+
+bool is_gated4(Route r) { return r == R_GATED4_16X32 || r == R_GATED4_8X32; }
+
+// The projection of a linear4 op (buffers x, w, scales, biases, out).
+bool linear4_job(const Op& op, tessery::Linear4Job* job) {
+  RowRange rr;
+  if (!is_linear4(op.route) || !linear4_range(op.route, op.p, op.threads, op.group, &rr))
+    return false;
+  *job = {static_cast<const float*>(op.ptr[0]),    static_cast<const uint32_t*>(op.ptr[1]),
+          static_cast<const uint16_t*>(op.ptr[2]), static_cast<const uint16_t*>(op.ptr[3]),
+          static_cast<float*>(op.ptr[4]),          static_cast<int>(rr.r0),
+          static_cast<int>(rr.r1),                 static_cast<int>(op.p.cols),
+          static_cast<int>(op.p.k)};
+  return true;
+}
+
+// Gate and up projections of a gated4 op (buffers x, w, s, b, up w, up s, up b, out).
+bool gated4_jobs(const Op& op, tessery::Linear4Job* jobs) {
+  RowRange rr;
+  if (!is_gated4(op.route) || !gated4_range(op.route, op.p, op.threads, op.group, &rr))
+    return false;
+  for (int i = 0; i < 2; ++i)
+    jobs[i] = {static_cast<const float*>(op.ptr[0]),
+               static_cast<const uint32_t*>(op.ptr[1 + 3 * i]),
+               static_cast<const uint16_t*>(op.ptr[2 + 3 * i]),
+               static_cast<const uint16_t*>(op.ptr[3 + 3 * i]),
+               i == 0 ? static_cast<float*>(op.ptr[7]) : nullptr,
+               static_cast<int>(rr.r0),
+               static_cast<int>(rr.r1),
+               static_cast<int>(op.p.cols),
+               static_cast<int>(op.p.k)};
+  return true;
+}
+
 hipError_t launch(Runtime* rt, const Op& op) {
   hipStream_t st = rt->stream;
   const Params& p = op.p;
@@ -700,28 +739,17 @@ hipError_t launch(Runtime* rt, const Op& op) {
     case R_LINEAR4_16X32:
     case R_LINEAR4_32X32:
     case R_LINEAR4_SMALL3: {
-      RowRange rr;
-      if (!linear4_range(op.route, p, op.threads, op.group, &rr)) return hipErrorInvalidValue;
-      return tessery::launch_linear4_f32(
-          static_cast<const float*>(op.ptr[0]), static_cast<const uint32_t*>(op.ptr[1]),
-          static_cast<const uint16_t*>(op.ptr[2]), static_cast<const uint16_t*>(op.ptr[3]),
-          static_cast<float*>(op.ptr[4]), static_cast<int>(rr.r0), static_cast<int>(rr.r1),
-          static_cast<int>(p.cols), static_cast<int>(p.k), rt->dense_scratch, kDenseScratchFloats,
-          st);
+      tessery::Linear4Job job;
+      if (!linear4_job(op, &job)) return hipErrorInvalidValue;
+      return tessery::launch_linear4_f32(job, rt->dense_scratch, kDenseScratchFloats, st);
     }
     case R_QKV4_F16:
       return tessery::launch_qkv4_f16(qkv4_args(op), st);
     case R_GATED4_16X32:
     case R_GATED4_8X32: {
-      RowRange rr;
-      if (!gated4_range(op.route, p, op.threads, op.group, &rr)) return hipErrorInvalidValue;
-      return tessery::launch_gated4_f32(
-          static_cast<const float*>(op.ptr[0]), static_cast<const uint32_t*>(op.ptr[1]),
-          static_cast<const uint16_t*>(op.ptr[2]), static_cast<const uint16_t*>(op.ptr[3]),
-          static_cast<const uint32_t*>(op.ptr[4]), static_cast<const uint16_t*>(op.ptr[5]),
-          static_cast<const uint16_t*>(op.ptr[6]), static_cast<float*>(op.ptr[7]),
-          static_cast<int>(rr.r0), static_cast<int>(rr.r1), static_cast<int>(p.cols),
-          static_cast<int>(p.k), rt->dense_scratch, kDenseScratchFloats, st);
+      tessery::Linear4Job jobs[2];
+      if (!gated4_jobs(op, jobs)) return hipErrorInvalidValue;
+      return tessery::launch_linear4_rows(jobs, 2, true, st);
     }
     case R_SILU_GATE:
       return tessery::launch_silu_gate_f32(static_cast<float*>(op.ptr[0]),
@@ -938,7 +966,6 @@ int mi_dispatch(void* runtime, const char* name, void** buffers, uint32_t count,
   return queue_op(rt, op) ? 0 : 1;
 }
 
-bool is_linear4(Route r);
 hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
 
 // Pairs of queued launches that one kernel runs with the same bits (the second op of a pair is
@@ -1052,11 +1079,6 @@ hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b) {
   return hipErrorNotReady;
 }
 
-bool is_linear4(Route r) {
-  return r == R_LINEAR4 || r == R_LINEAR4_TILED || r == R_LINEAR4_TAIL || r == R_LINEAR4_16X32 ||
-         r == R_LINEAR4_32X32 || r == R_LINEAR4_SMALL3;
-}
-
 // The gated MLP as the reference's unfused form queues it (metal.py:501-530): linear4(x -> g),
 // linear4(x -> u) over the same rows, then silu_gate(g, u). When both projections cover all rows
 // of their outputs and would run the fp16-MFMA kernel, one launch computes both from one staging
@@ -1104,30 +1126,132 @@ hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated) 
   return e == hipErrorInvalidValue ? hipErrorNotReady : e;
 }
 
-// Launches ops [first, last) in order, running as one kernel the triples launch_fused_gated takes
-// and the pairs launch_fused_pair takes; the fusions made are added to *fc. Under stream capture
+// A uint4 projection over a run of queued ops: ops[first, end) are launches of one projection (the
+// same buffers and shape) over consecutive row ranges, as linear4_plan partitions its rows.
+struct Linear4Run {
+  tessery::Linear4Job job;
+  size_t end;
+};
+
+// The run that starts at op `first`; false unless linear4_rows runs it. Its results depend on no
+// launch's rows, so one launch over the joined rows leaves the bits of the separate ones; a
+// projection that fp16 MFMA takes (linear4_hilo) stays as queued.
+bool linear4_run(Runtime* rt, size_t first, size_t last, Linear4Run* run) {
+  if (!linear4_job(rt->ops[first], &run->job) ||
+      !tessery::linear4_on_rows(run->job, rt->dense_scratch, kDenseScratchFloats))
+    return false;
+  run->end = first + 1;
+  // a launch reads x and the weights that an output over them would have changed by then
+  const Op& a = rt->ops[first];
+  for (int i = 0; i < 4; ++i)
+    if (a.ptr[i] == a.ptr[4]) return true;
+  for (; run->end < last; ++run->end) {
+    const Op& b = rt->ops[run->end];
+    tessery::Linear4Job next;
+    if (!linear4_job(b, &next) || b.p.rows != a.p.rows || next.cols != run->job.cols ||
+        next.k != run->job.k || next.row0 != run->job.row1 ||
+        !std::equal(a.ptr.begin(), a.ptr.begin() + 5, b.ptr.begin()) ||
+        !tessery::linear4_on_rows(next, rt->dense_scratch, kDenseScratchFloats))
+      break;
+    run->job.row1 = next.row1;
+  }
+  return true;
+}
+
+// The linear4_rows launch that starts at op `first`: up to three projections of the same rows of
+// one x queued one after the other (q, k and v), two of them with the silu_gate that follows
+// (gate and up), each over its whole run of row ranges, or the row ranges of a gated4 projection.
+// *taken: the ops it ran. hipErrorNotReady: op `first` is no such projection.
+hipError_t launch_linear4_runs(Runtime* rt, size_t first, size_t last, size_t* taken) {
+  const Op& a = rt->ops[first];
+  if (is_gated4(a.route)) {
+    tessery::Linear4Job jobs[2], next[2];
+    if (!gated4_jobs(a, jobs)) return hipErrorInvalidValue;
+    size_t end = first + 1;
+    bool apart = true;  // the output is none of the inputs
+    for (int i = 0; i < 7; ++i) apart = apart && a.ptr[i] != a.ptr[7];
+    for (; apart && end < last; ++end) {
+      const Op& b = rt->ops[end];
+      if (!gated4_jobs(b, next) || a.ptr != b.ptr || b.p.rows != a.p.rows ||
+          next[0].cols != jobs[0].cols || next[0].k != jobs[0].k || next[0].row0 != jobs[0].row1)
+        break;
+      jobs[0].row1 = jobs[1].row1 = next[0].row1;
+    }
+    *taken = end - first;
+    return tessery::launch_linear4_rows(jobs, 2, true, rt->stream);
+  }
+  Linear4Run run;
+  if (!is_linear4(a.route) || !linear4_run(rt, first, last, &run)) return hipErrorNotReady;
+  tessery::Linear4Job jobs[3] = {run.job};
+  size_t ends[3] = {run.end, 0, 0};
+  int count = 1;
+  while (count < 3 && ends[count - 1] < last &&
+         linear4_run(rt, ends[count - 1], last, &run)) {
+    const tessery::Linear4Job& j = run.job;
+    bool joins = j.x == jobs[0].x && j.k == jobs[0].k && j.row0 == jobs[0].row0 &&
+                 j.row1 == jobs[0].row1 && static_cast<const void*>(j.out) != j.x;
+    // no output is an input or output of another projection of the launch
+    for (int i = 0; i < count && joins; ++i) {
+      const tessery::Linear4Job& o = jobs[i];
+      for (const void* in : {static_cast<const void*>(j.x), static_cast<const void*>(j.w),
+                             static_cast<const void*>(j.scales),
+                             static_cast<const void*>(j.biases), static_cast<const void*>(j.out)})
+        joins = joins && in != o.out;
+      for (const void* in : {static_cast<const void*>(o.w), static_cast<const void*>(o.scales),
+                             static_cast<const void*>(o.biases)})
+        joins = joins && in != j.out;
+    }
+    if (!joins) break;
+    jobs[count] = j;
+    ends[count++] = run.end;
+  }
+  // gate, up, silu_gate(gate, up) over every row
+  if (count >= 2 && ends[1] < last && jobs[0].cols == jobs[1].cols && jobs[0].row0 == 0) {
+    const Op& c = rt->ops[ends[1]];
+    if (c.route == R_SILU_GATE && c.ptr[0] == jobs[0].out && c.ptr[1] == jobs[1].out &&
+        static_cast<uint64_t>(c.p.n) ==
+            static_cast<uint64_t>(jobs[0].row1) * static_cast<uint64_t>(jobs[0].cols)) {
+      *taken = ends[1] + 1 - first;
+      return tessery::launch_linear4_rows(jobs, 2, true, rt->stream);
+    }
+  }
+  *taken = ends[count - 1] - first;
+  return tessery::launch_linear4_rows(jobs, count, false, rt->stream);
+}
+
+// Launches op `first` and those after it (before op `last`) that run inside the same kernel: the
+// runs launch_linear4_runs takes, the triples of launch_fused_gated and the pairs of
+// launch_fused_pair (the last two counted in *fc). *taken: the ops launched.
+hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, FusionCount* fc) {
+  const hipError_t rows = launch_linear4_runs(rt, first, last, taken);
+  if (rows != hipErrorNotReady) return rows;
+  const hipError_t gated =
+      first + 2 < last
+          ? launch_fused_gated(rt, rt->ops[first], rt->ops[first + 1], rt->ops[first + 2])
+          : hipErrorNotReady;
+  if (gated != hipErrorNotReady) {
+    fc->gated += gated == hipSuccess;
+    *taken = 3;
+    return gated;
+  }
+  const hipError_t pair = first + 1 < last
+                              ? launch_fused_pair(rt, rt->ops[first], rt->ops[first + 1])
+                              : hipErrorNotReady;
+  if (pair != hipErrorNotReady) {
+    fc->pairs += pair == hipSuccess;
+    *taken = 2;
+    return pair;
+  }
+  *taken = 1;
+  return launch(rt, rt->ops[first]);
+}
+
+// Launches ops [first, last) in order; the fusions made are added to *fc. Under stream capture
 // nothing runs yet, so the caller decides where the count goes (the runtime's totals for direct
 // launches, the cached graph for a capture).
 hipError_t launch_range(Runtime* rt, size_t first, size_t last, FusionCount* fc) {
-  for (size_t i = first; i < last; ++i) {
-    const hipError_t gated =
-        i + 2 < last ? launch_fused_gated(rt, rt->ops[i], rt->ops[i + 1], rt->ops[i + 2])
-                     : hipErrorNotReady;
-    if (gated == hipSuccess) {
-      ++fc->gated;
-      i += 2;
-      continue;
-    }
-    if (gated != hipErrorNotReady) return gated;
-    const hipError_t fused =
-        i + 1 < last ? launch_fused_pair(rt, rt->ops[i], rt->ops[i + 1]) : hipErrorNotReady;
-    if (fused == hipSuccess) {
-      ++fc->pairs;
-      ++i;
-      continue;
-    }
-    if (fused != hipErrorNotReady) return fused;
-    const hipError_t e = launch(rt, rt->ops[i]);
+  for (size_t i = first, taken = 0; i < last; i += taken) {
+    const hipError_t e = launch_next(rt, i, last, &taken, fc);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -1225,37 +1349,26 @@ int mi_finish(void* runtime) {
     }
     if (!failed && launch_direct(rt, i, n) != hipSuccess) failed = 1;
   }
-  if (rt->profiling) rt->profile_fused.assign(n, 0);
-  for (size_t i = 0; rt->profiling && i < n && !failed; ++i) {
-    if (rt->profiling && hipEventRecord(rt->prof_events[2 * i], rt->stream) != hipSuccess) failed = 1;
-    // a fused triple or pair runs inside the first op's events; the others' events enclose no
-    // work
-    const hipError_t gated =
-        failed || i + 2 >= n ? hipErrorNotReady
-                             : launch_fused_gated(rt, rt->ops[i], rt->ops[i + 1], rt->ops[i + 2]);
-    if (!failed && gated != hipErrorNotReady && gated != hipSuccess) failed = 1;
-    const hipError_t fused =
-        failed || gated == hipSuccess || i + 1 >= n
-            ? hipErrorNotReady
-            : launch_fused_pair(rt, rt->ops[i], rt->ops[i + 1]);
-    if (!failed && fused != hipErrorNotReady && fused != hipSuccess) failed = 1;
-    if (!failed && gated == hipErrorNotReady && fused == hipErrorNotReady &&
-        launch(rt, rt->ops[i]) != hipSuccess)
-      failed = 1;
-    if (!failed && rt->profiling &&
-        hipEventRecord(rt->prof_events[2 * i + 1], rt->stream) != hipSuccess)
-      failed = 1;
-    const size_t extra = !failed && gated == hipSuccess ? 2 : (!failed && fused == hipSuccess ? 1 : 0);
-    rt->fused_gated += extra == 2;
-    rt->fused_pairs += extra == 1;
-    rt->profile_fused[i] = 0;
-    for (size_t e = 0; e < extra && !failed; ++e) {
-      ++i;
-      rt->profile_fused[i] = 1;
-      if (rt->profiling && (hipEventRecord(rt->prof_events[2 * i], rt->stream) != hipSuccess ||
-                            hipEventRecord(rt->prof_events[2 * i + 1], rt->stream) != hipSuccess))
+  if (rt->profiling) {
+    // ops that run inside the kernel of one before them: the first one's events enclose that
+    // kernel, the others' enclose no work
+    rt->profile_fused.assign(n, 0);
+    FusionCount fc;
+    for (size_t i = 0, taken = 0; i < n && !failed; i += taken) {
+      if (hipEventRecord(rt->prof_events[2 * i], rt->stream) != hipSuccess ||
+          launch_next(rt, i, n, &taken, &fc) != hipSuccess ||
+          hipEventRecord(rt->prof_events[2 * i + 1], rt->stream) != hipSuccess) {
         failed = 1;
+        break;
+      }
+      for (size_t j = i + 1; j < i + taken && !failed; ++j) {
+        rt->profile_fused[j] = 1;
+        if (hipEventRecord(rt->prof_events[2 * j], rt->stream) != hipSuccess ||
+            hipEventRecord(rt->prof_events[2 * j + 1], rt->stream) != hipSuccess)
+          failed = 1;
+      }
     }
+    if (!failed) count_fusions(rt, fc);
   }
   if (hipEventRecord(rt->ev_end, rt->stream) != hipSuccess) failed = 1;
   if (hipStreamSynchronize(rt->stream) != hipSuccess) failed = 1;
