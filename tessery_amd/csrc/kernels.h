@@ -52,7 +52,7 @@ hipError_t launch_attention_f16(const AttnArgs& a, hipStream_t st);
 
 // tessery rms_norm (kernels.metal:53-63): rows x cols fp32, bf16 weight, out may alias x.
 hipError_t launch_rms_norm_f32(const float* x, const uint16_t* w, float* out, int rows, int cols,
-                               float eps, hipStream_t st);
+                               float eps, void* planes, hipStream_t st);
 // RoPE tables [S, D/2] of cos / sin(pos * theta^(-2j/D)), evaluated in float64 on the device
 // and rounded once to float32.
 bool rope_tables_fit(int S, int D);
@@ -64,7 +64,8 @@ hipError_t launch_rope_f32(float* x, const float* cos_tab, const float* sin_tab,
 // launch_add_f32(x, r, x) followed by launch_rms_norm_f32(x, w, y) as one pass with the same bits;
 // hipErrorNotReady unless cols % 4 == 0 and x, r, y are 16-byte aligned.
 hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, float* y,
-                                   int rows, int cols, float eps, hipStream_t st);
+                                   int rows, int cols, float eps, void* planes,
+                                   hipStream_t st);
 // launch_rms_norm_f32 in place (x == out) followed by launch_rope_f32 on the same rows, as one
 // kernel with the same bits; hipErrorNotReady when the shape is not covered (8 | dim <= 256, x
 // 16-byte aligned) and the two launches must run instead.
@@ -91,16 +92,26 @@ struct Linear4Job {
   float* out;
   int row0, row1, cols, k;
 };
+// Scratch of linear4_rows: `in` takes the planes (planes.h) of the activations it reads, `out` those
+// of a gated output; each of `bytes`, 16-byte aligned.
+struct PlanesScratch {
+  void *in, *out;
+  size_t bytes;
+};
 hipError_t launch_linear4_f32(const Linear4Job& job, float* scratch, size_t scratch_floats,
-                              hipStream_t st);
+                              const PlanesScratch& planes, hipStream_t st);
 // Whether launch_linear4_f32 runs the job on linear4_rows, whose results depend neither on the rows
 // of the launch nor on the projections beside it.
 bool linear4_on_rows(const Linear4Job& job, const float* scratch, size_t scratch_floats);
 // One to three projections of the same rows of one x in one linear4_rows launch, with the bits of
 // separate ones. With `gated` (two jobs of equal width: gate, up): out of the gate takes
 // silu(gate) * up (tessery gated4, kernels.metal:609-656, 687-731), out of the up projection, when
-// not null, its own values, as linear4 + linear4 + silu_gate leave them.
-hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated, hipStream_t st);
+// not null, its own values, as linear4 + linear4 + silu_gate leave them. prepared: scratch.in holds
+// the planes of x already (row0 = 0); else they are made first. keep (gated, row0 = 0): scratch.out
+// takes the planes of the gated output. Both need planes that fit the scratch.
+hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated,
+                               const PlanesScratch& scratch, bool prepared, bool keep,
+                               hipStream_t st);
 // The same projection for M >= kLinear4HiloRows rows on fp16 MFMA: rows scaled by powers of two
 // and split into hi + lo fp16 halves (about 22 bits), exact codes, fp32 sums. scratch holds the M
 // row scales. x and y start at row 0 of the range; N % 128 == 0, K % 64 == 0.

@@ -20,6 +20,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "lds_dma.h"
+#include "planes.h"
 
 namespace tessery {
 
@@ -37,15 +38,13 @@ namespace {
 // K order: eight partitions of consecutive groups (partition p: groups [p G / 8, (p + 1) G / 8)),
 // each summed on its own, then added as a balanced tree.
 //
-// Layout: 8 wavefronts = WC column blocks of 32 x WK slots of 8 / WK consecutive partitions; a
-// workgroup makes a tile of 32 rows x 32 WC columns. The WC wavefronts of a slot stage one group
-// of x at a time (32 x 64 floats -> three bf16 planes in LDS, the next group's x and weights in
-// registers meanwhile); the slots' sums meet in LDS at the end, so no partial sums leave the
-// workgroup. Bound: with few rows the latency of one pass over K (loads, split, MFMA chain, the
-// sum over slots) and the splitting of x, which every workgroup repeats; with many rows the VALU
-// (split, decode, fold), about as many cycles as the MFMAs at WC = 4.
-// LDS planes are rows of 128 bytes, 16-byte chunk c of row r at c ^ ((r >> 1) & 7): the 16 rows one
-// read group takes land on different banks, and 8 lanes write one row.
+// x comes as planes (planes.h), so no workgroup splits it again. linear4_rows (few tiles): operands go
+// straight from L1 to registers, with no LDS and no barrier before the end; a workgroup makes a
+// tile of 32 x 32 with one partition a wavefront, and their sums meet in LDS, so no partial sums
+// leave it. Bound: the loads. A wavefront reads 12 KiB of x for a group and fetches whole lines of
+// weights and scales, which is why it takes four groups of those at a time. Measured, the o
+// projection (K = 2048) of 24 rows: 7.4 us, 9.3 us with every workgroup splitting x itself; down
+// (K = 3072) 9.2 and 12.8 us.
 constexpr int kL4Parts = 8;
 constexpr int kRedRow = 40;  // floats per staged result row: the lane halves' rows r, r + 4 on
                              // opposite halves of the banks
@@ -61,15 +60,18 @@ struct L4Set {
 // Up to three projections of the same x, or (GATED) gate and up of equal width: out of set 0 takes
 // silu(gate) * up, out of set 1 (may be null) the up projection.
 struct L4Args {
-  const float* x;
+  Planes x;  // of rows row0 .. row1 - 1
   L4Set set[3];
   int row0, row1, k;
-  int vec;  // every out 16-byte aligned and every width a multiple of 4
+  int vec;      // every out 16-byte aligned and every width a multiple of 4
+  Planes next;  // GATED: the planes of the output (terms null: none), row0 = 0
 };
 
 // (c - 8) / 16 of the eight codes of a weight word as bf16, in natural order
 __device__ __forceinline__ bf16x8 decode_centred(uint32_t word) {
-  const uint32_t even = word ^ 0x88888888u, odd = even >> 4;
+  const uint32_t even = word ^ 0x88888888u;
+  uint32_t odd = even >> 4;
+  asm("" : "+v"(odd));  // its bytes are then operand selects of the conversions, not shifts
   uint4v r;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
@@ -80,95 +82,308 @@ __device__ __forceinline__ bf16x8 decode_centred(uint32_t word) {
   return __builtin_bit_cast(bf16x8, r);
 }
 
-struct Split3 {
-  uint32_t t[3];  // the three bf16 terms, each in the upper half of its word
-};
-__device__ __forceinline__ Split3 split3(float x) {
-  Split3 r;
-  r.t[0] = __float_as_uint(x);
-  const float r1 = x - __uint_as_float(r.t[0] & 0xffff0000u);
-  r.t[1] = __float_as_uint(r1);
-  r.t[2] = __float_as_uint(r1 - __uint_as_float(r.t[1] & 0xffff0000u));
-  return r;
-}
-__device__ __forceinline__ uint32_t upper_pair(uint32_t first, uint32_t second) {
-  return __builtin_amdgcn_perm(second, first, 0x07060302u);
+// Planes of rows row0 .. of x: a workgroup splits one row tile's group, thread (row tid / 8, chunk
+// tid % 8) 8 inputs; the 8 rows of a wavefront make 128-byte pieces.
+__global__ __launch_bounds__(256) void split_planes(const float* __restrict__ x, Planes p,
+                                                    int row0, int row1, int k) {
+  const int groups = k >> 6, g = blockIdx.y, row = threadIdx.x >> 3, c = threadIdx.x & 7;
+  const int at = static_cast<int>(blockIdx.x) * kPlaneRows + row;
+  if (row0 + at >= row1) return;
+  const float* const src = x + static_cast<size_t>(row0 + at) * k + 64 * g + 8 * c;
+  const floatx4 u = *reinterpret_cast<const floatx4*>(src);
+  const floatx4 v = *reinterpret_cast<const floatx4*>(src + 4);
+  const size_t tile = static_cast<size_t>(blockIdx.x) * groups + g;
+  const int lane = row + 32 * (c >> 2);
+  uint4v t[3];
+  split3x8(u, v, t[0], t[1], t[2]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    *reinterpret_cast<uint4v*>(p.terms + tile * kPlaneGroup + i * kPlaneTerm + (c & 3) * 512 +
+                               lane * 8) = t[i];
+  float sum = ((u[0] + u[1]) + (u[2] + u[3])) + ((v[0] + v[1]) + (v[2] + v[3]));
+  sum += __shfl_xor(sum, 1);
+  sum += __shfl_xor(sum, 2);
+  if ((c & 3) == 0) p.sums[tile * kPlaneSums + lane] = sum;
 }
 
-template <int WC, int WK, bool GATED>
-__global__ __launch_bounds__(512, WC == 1 ? 2 : 4) void linear4_rows(L4Args a) {
-  static_assert(WC * WK == 8 && kL4Parts % WK == 0 && (!GATED || WC > 1), "eight wavefronts");
-  constexpr int NP = kL4Parts / WK;     // partitions of a slot
-  constexpr int NBUF = WC == 4 ? 2 : 1;  // x stages of a slot
-  constexpr int CPT = 4 / WC;           // 8-float chunks of x a thread stages per group
-  constexpr int PLANE = 32 * 64;
-  constexpr int STAGE = NBUF * WK * 3 * PLANE * 2, RED = 8 * 32 * kRedRow * 4;
-  __shared__ __attribute__((aligned(1024))) char mem[STAGE > RED ? STAGE : RED];
-  __shared__ float xg[NBUF][WK][2][32];  // sums of 32 inputs (half a group) per row
-  uint16_t* const planes = reinterpret_cast<uint16_t*>(mem);
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+__device__ __forceinline__ rsrc_t resource(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+
+// Weight words, scales and biases of a lane's column for N consecutive groups: a column's groups lie
+// side by side, so four of them fill the line that one would fetch. Scales and biases are 2-byte
+// words at any parity: whole dwords from the aligned one below, shifted by the lane. Groups past
+// the last one read the next column's, or zero past the end (the caller uses none of them).
+template <int N>
+struct Words {
+  uint4v w[N];
+  uint32_t s[N / 2 + 1], b[N / 2 + 1];
+};
+struct ColumnWords {
+  rsrc_t wres, sres, bres;
+  uint32_t woff, soff, groups;
+
+  __device__ __forceinline__ ColumnWords(const L4Set& set, int n, int hh, int K) {
+    const uint32_t half = static_cast<uint32_t>(K >> 1), cols = static_cast<uint32_t>(set.cols);
+    groups = static_cast<uint32_t>(K >> 6);
+    // scales and biases in whole dwords: an odd count is followed by padding of its allocation
+    const uint32_t bytes = (cols * groups * 2u + 3u) & ~3u;
+    wres = resource(set.w, cols * half);
+    sres = resource(set.s, bytes);
+    bres = resource(set.b, bytes);
+    woff = static_cast<uint32_t>(n) * half + 16u * static_cast<uint32_t>(hh);
+    soff = static_cast<uint32_t>(n) * groups * 2u;
+  }
+  template <int N>
+  __device__ __forceinline__ void load(Words<N>& r, int at) const {
+    const uint32_t g = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      r.w[j] = __builtin_amdgcn_raw_buffer_load_b128(wres, woff + 32u * j, 32u * g, 0);
+    const uint32_t off = (soff + 2u * g) & ~3u;
+    if constexpr (N == 4) {
+      const uint3v s = __builtin_amdgcn_raw_buffer_load_b96(sres, off, 0, 0);
+      const uint3v b = __builtin_amdgcn_raw_buffer_load_b96(bres, off, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) r.s[j] = s[j], r.b[j] = b[j];
+    } else {
+      static_assert(N == 2, "two or four groups");
+      const uint2v s = __builtin_amdgcn_raw_buffer_load_b64(sres, off, 0, 0);
+      const uint2v b = __builtin_amdgcn_raw_buffer_load_b64(bres, off, 0, 0);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) r.s[j] = s[j], r.b[j] = b[j];
+    }
+  }
+  // the words as loaded for `at` -> scales and biases of groups 2 i, 2 i + 1 in s[i] and b[i]
+  template <int N>
+  __device__ __forceinline__ void align(Words<N>& r, int at) const {
+    const uint32_t shift = ((soff + 2u * static_cast<uint32_t>(at)) & 2u) * 8u;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      r.s[i] = __builtin_amdgcn_alignbit(r.s[i + 1], r.s[i], shift);
+      r.b[i] = __builtin_amdgcn_alignbit(r.b[i + 1], r.b[i], shift);
+    }
+  }
+};
+
+// Column tile t of a launch -> the weight set it belongs to and the tile's place in it.
+__device__ __forceinline__ void column_tile(const L4Args& a, int width, int& tile, int& set) {
+  while (set < 2 && tile >= (a.set[set].cols + width - 1) / width) {
+    tile -= (a.set[set].cols + width - 1) / width;
+    ++set;
+  }
+}
+
+// What a 32-column block needs of one group's words: the codes, the bias operand (b' in the lane's
+// k-slots, against the terms of its half-group sum) and the scale.
+struct Prepared {
+  bf16x8 codes[4], bias;
+  float s16;
+};
+// of group j (a constant after unrolling) of aligned words
+template <int N>
+__device__ __forceinline__ Prepared prepare_group(const Words<N>& words, int j) {
+  auto upper = [&](uint32_t v) { return __uint_as_float(j & 1 ? v & 0xffff0000u : v << 16); };
+  const float scale = upper(words.s[j / 2]), bias = upper(words.b[j / 2]);
+  Prepared r;
+#pragma unroll
+  for (int s4 = 0; s4 < 4; ++s4) r.codes[s4] = decode_centred(words.w[j][s4]);
+  const Split3 bs = split3(fmaf(8.0f, scale, bias));
+  const uint32_t b12 = upper_pair(bs.t[0], bs.t[1]);
+  r.bias = __builtin_bit_cast(bf16x8, uint4v{b12, b12, upper_pair(bs.t[2], bs.t[0]), 0u});
+  r.s16 = 16.0f * scale;
+  return r;
+}
+
+// acc += the group's products for one 32 x 32 tile; x(t, s4): the operand of term t, k-step s4.
+template <typename X>
+__device__ __forceinline__ void multiply_group(const Prepared& w, X x, float xsum, floatx16& acc) {
+  // bias term: six products of the terms of the lane's half-group sum and b'
+  const Split3 xs = split3(xsum);
+  const bf16x8 xa = __builtin_bit_cast(
+      bf16x8, uint4v{upper_pair(xs.t[0], xs.t[0]), upper_pair(xs.t[1], xs.t[1]),
+                     upper_pair(xs.t[0], xs.t[2]), 0u});
+  acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, w.bias, acc, 0, 0, 0);
+  floatx16 p;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) p[e] = 0.0f;
+#pragma unroll
+  for (int t = 2; t >= 0; --t)  // the smallest terms first
+#pragma unroll
+    for (int s4 = 0; s4 < 4; ++s4)
+      p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x(t, s4), w.codes[s4], p, 0, 0, 0);
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = fmaf(w.s16, p[e], acc[e]);
+}
+
+// The end of a tile of BLOCKS column blocks (GATED: the gate's, then the up projection's), one a
+// wavefront: the sums of the SLOTS slots meet in LDS (`red`, free by now), then whole-row stores.
+template <int BLOCKS, int SLOTS, bool GATED>
+__device__ __forceinline__ void store_tile(const L4Args& a, float* red,
+                                           const floatx16& total, int slot, int own, int first,
+                                           int tile, int rbase) {
+  constexpr int TC = GATED ? 16 * BLOCKS : 32 * BLOCKS, THREADS = 64 * SLOTS * BLOCKS;
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+#pragma unroll
+  for (int e = 0; e < 16; ++e)
+    red[((slot * BLOCKS + own) * 32 + 8 * (e >> 2) + 4 * hh + (e & 3)) * kRedRow + l32] = total[e];
+  wait_lgkmcnt<0>();
+  stage_barrier();
+  auto sum4 = [&](int block, int row, int col) {
+    auto at = [&](int s) {
+      return *reinterpret_cast<const floatx4*>(
+          &red[((s * BLOCKS + block) * 32 + row) * kRedRow + col]);
+    };
+    auto add = [](const floatx4& u, const floatx4& v) {
+      return floatx4{u[0] + v[0], u[1] + v[1], u[2] + v[2], u[3] + v[3]};
+    };
+    if constexpr (SLOTS == 8)
+      return add(add(add(at(0), at(1)), add(at(2), at(3))),
+                 add(add(at(4), at(5)), add(at(6), at(7))));
+    else if constexpr (SLOTS == 4)
+      return add(add(at(0), at(1)), add(at(2), at(3)));
+    else
+      return add(at(0), at(1));
+  };
+  auto store = [&](const L4Set& set, int row, int c0, const floatx4& y) {
+    float* const dst = set.out + static_cast<size_t>(row) * set.cols + c0;
+    if (a.vec && c0 + 4 <= set.cols) {
+      *reinterpret_cast<floatx4*>(dst) = y;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (c0 + j < set.cols) dst[j] = y[j];
+    }
+  };
+  for (int i = tid; i < 32 * TC / 4; i += THREADS) {
+    const int row = i / (TC / 4), c = 4 * (i % (TC / 4)), block = c >> 5;
+    if (rbase + row >= a.row1) break;  // rows ascend with i
+    floatx4 y = sum4(block, row, c & 31);
+    if constexpr (GATED) {
+      const floatx4 up = sum4(block + BLOCKS / 2, row, c & 31);
+      if (a.set[1].out) store(a.set[1], rbase + row, tile * TC + c, up);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = silu_times(y[j], up[j]);
+      if (a.next.terms && tile * TC + c < a.set[0].cols)
+        store_planes4(a.next, rbase + row, tile * TC + c, a.set[0].cols >> 6, y);
+    }
+    store(a.set[GATED ? 0 : first], rbase + row, tile * TC + c, y);
+  }
+}
+
+// A 32 x 32 tile, one partition a wavefront.
+__global__ __launch_bounds__(512, 2) void linear4_rows(L4Args a) {
+  __shared__ __attribute__((aligned(16))) float red[8 * 32 * kRedRow];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int groups = a.k >> 6;
+  const int rbase = a.row0 + static_cast<int>(blockIdx.x) * kPlaneRows;
+  int tile = blockIdx.y, first = 0;
+  column_tile(a, 32, tile, first);
+  // clamped columns aren't stored
+  const ColumnWords column(a.set[first], min(tile * 32 + l32, a.set[first].cols - 1), hh, a.k);
+
+  // Rows past the last one, and a group past the wavefront's last one, are asked for at kNowhere,
+  // out of the resource's range: no memory access, and no branch around the loads, which keeps the
+  // compiler's waits exact.
+  constexpr uint32_t kNowhere = 0xc0000000u;
+  const uint32_t norow = rbase + l32 < a.row1 ? 0u : kNowhere;
+  const size_t xtile = static_cast<size_t>(blockIdx.x) * groups;
+  const rsrc_t xres = resource(a.x.terms + xtile * kPlaneGroup,
+                               static_cast<uint32_t>(groups) * (kPlaneGroup * 2u));
+  const rsrc_t xsres = resource(a.x.sums + xtile * kPlaneSums,
+                                static_cast<uint32_t>(groups) * (kPlaneSums * 4u));
+  struct Group {
+    bf16x8 x[3][4];
+    float sum;
+  };
+  int g = wave * groups / kL4Parts;
+  const int end = (wave + 1) * groups / kL4Parts;
+  auto load = [&](Group& r, int at) {
+    const uint32_t past = at < end ? norow : kNowhere;
+    const uint32_t gx = __builtin_amdgcn_readfirstlane(at < end ? at : 0);
+    r.sum = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                          xsres, (4u * lane) | past, 4u * kPlaneSums * gx, 0));
+#pragma unroll
+    for (int t = 2; t >= 0; --t)
+#pragma unroll
+      for (int s4 = 0; s4 < 4; ++s4)
+        r.x[t][s4] = __builtin_bit_cast(
+            bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+                        xres, ((16u * lane) | past) + 1024u * s4,
+                        2u * kPlaneGroup * gx + 2u * kPlaneTerm * t, 0));
+    asm volatile("" ::: "memory");  // issued here, before the product that runs meanwhile
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // every sum started from +0, as in the other tile shape
+  floatx16 total;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) total[e] = 0.0f;
+  if (g < end) {
+    Group x[2];
+    Words<4> words;
+    column.load(words, g);
+    load(x[0], g);
+    bool more = true;
+    while (more) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j == 0) column.align(words, g);
+        const Prepared w = prepare_group(words, j);
+        if (j == 3) column.load(words, g + 4);
+        load(x[(j + 1) & 1], g + j + 1);
+        const Group& r = x[j & 1];
+        multiply_group(w, [&](int t, int s4) { return r.x[t][s4]; }, r.sum, total);
+        if (g + j + 1 >= end) {
+          more = false;
+          break;
+        }
+      }
+      g += 4;
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 16; ++e) total[e] += 0.0f;
+  store_tile<1, 8, false>(a, red, total, wave, 0, first, tile, rbase);
+}
+
+// The same with x shared: 8 wavefronts = WC column blocks of 32 x WK slots of 8 / WK partitions
+// (GATED: half of the blocks are the gate's columns, half the up projection's). One group of x a
+// slot at a time is copied to LDS (two stages, the copy of the next group under way while this one
+// is multiplied) and read by the slot's WC wavefronts. Bound: the issue of VALU instructions
+// (decoding and folding, about 110 beside 13 MFMAs) and a step's barrier and waits. Measured: q, k
+// and v of 308 rows 18.1 us, gate and up 20.9; with x split in every workgroup 22 and 26.
+template <int WC, bool GATED>
+__global__ __launch_bounds__(512, WC == 4 ? 4 : 2) void linear4_rows_shared(L4Args a) {
+  constexpr int WK = 8 / WC, NP = kL4Parts / WK;  // partitions of a slot
+  constexpr int TC = GATED ? 16 * WC : 32 * WC;   // columns of a tile in each of its sets
+  constexpr int STAGES = 2 * WK * kPlaneGroup * 2, RED = 8 * 32 * kRedRow * 4;
+  __shared__ __attribute__((aligned(1024))) char mem[STAGES > RED ? STAGES : RED];
 
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
   const int wc = wave % WC, slot = wave / WC;
-  const int K = a.k, groups = K >> 6;
-  const int rbase = a.row0 + static_cast<int>(blockIdx.x) * 32;
-
-  // column tile -> weight set and the wavefront's first column in it
-  constexpr int TC = GATED ? 16 * WC : 32 * WC;  // columns of a tile in each of its sets
+  const int groups = a.k >> 6;
+  const int rbase = a.row0 + static_cast<int>(blockIdx.x) * kPlaneRows;
   int tile = blockIdx.y, first = 0;
-  if constexpr (!GATED)
-    while (first < 2 && tile >= (a.set[first].cols + TC - 1) / TC) {
-      tile -= (a.set[first].cols + TC - 1) / TC;
-      ++first;
-    }
-  const L4Set& mine = a.set[GATED ? (wc >= WC / 2) : first];
-  const int cblock = GATED ? wc % (WC / 2) : wc;
-  const int n = min(tile * TC + 32 * cblock + l32, mine.cols - 1);  // clamped columns aren't stored
-  // wave-uniform bases, 32-bit lane offsets (cols, K <= 65536)
-  const uint32_t woff = static_cast<uint32_t>(n) * static_cast<uint32_t>(K >> 3) + 4u * hh;
-  const uint32_t soff = static_cast<uint32_t>(n) * static_cast<uint32_t>(groups);
+  if constexpr (!GATED) column_tile(a, TC, tile, first);
+  const L4Set set = a.set[GATED ? (wc >= WC / 2) : first];
+  const int n = tile * TC + 32 * (GATED ? wc % (WC / 2) : wc) + l32;
+  const ColumnWords column(set, min(n, set.cols - 1), hh, a.k);  // clamped columns aren't stored
+  const size_t xtile = static_cast<size_t>(blockIdx.x) * groups;
 
-  // staging role: chunk (row, c) = floats 8c .. 8c + 7 of the group
-  const int st = wc * 64 + lane, srow = st >> 3, sc = st & 7;
-  const float* const xbase = a.x + static_cast<size_t>(rbase) * K;
-  uint32_t xoff[CPT];
-#pragma unroll
-  for (int i = 0; i < CPT; ++i)
-    xoff[i] = static_cast<uint32_t>(min(srow + 8 * WC * i, a.row1 - 1 - rbase)) *
-                  static_cast<uint32_t>(K) + 8u * sc;
-
-  floatx4 xr[CPT][2];
-  uint4v wd;
-  uint16_t sw, bw;
-  auto load = [&](int g) {
-    wd = *reinterpret_cast<const uint4v*>(mine.w + 8 * g + woff);
-    sw = (mine.s + g)[soff];
-    bw = (mine.b + g)[soff];
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const floatx4* src = reinterpret_cast<const floatx4*>(xbase + 64 * g + xoff[i]);
-      xr[i][0] = src[0];
-      xr[i][1] = src[1];
-    }
-  };
-  // the group in xr -> planes and half-group sums of stage buf
   auto stage = [&](int buf) {
-    uint16_t* const dst = planes + (buf * WK + slot) * 3 * PLANE;
+    return reinterpret_cast<_Float16*>(mem) + (buf * WK + slot) * kPlaneGroup;
+  };
+  float sum;
+  auto load = [&](int buf, int g) {
+    sum = a.x.sums[(xtile + g) * kPlaneSums + lane];
+    const uint16_t* const src = a.x.terms + (xtile + g) * kPlaneGroup;
 #pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const floatx4 u = xr[i][0], v = xr[i][1];
-      const int row = srow + 8 * WC * i;
-      uint4v p1, p2, p3;
-      split3x8(u, v, p1, p2, p3);
-      const int at = row * 64 + 8 * (sc ^ ((row >> 1) & 7));
-      *reinterpret_cast<uint4v*>(dst + at) = p1;
-      *reinterpret_cast<uint4v*>(dst + PLANE + at) = p2;
-      *reinterpret_cast<uint4v*>(dst + 2 * PLANE + at) = p3;
-      // a half group is one lane quad: DPP quad permutations (lane ^ 1, then lane ^ 2)
-      float sum = ((u[0] + u[1]) + (u[2] + u[3])) + ((v[0] + v[1]) + (v[2] + v[3]));
-      sum += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum), 0xB1, 0xf, 0xf, false));
-      sum += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(sum), 0x4E, 0xf, 0xf, false));
-      xg[buf][slot][sc >> 2][row] = sum;  // the quad's lanes hold the same sum
+    for (int i = 0; i < 12 / WC; ++i) {
+      const int piece = wc * (12 / WC) + i;
+      dma16_at(src + piece * 512, 16u * lane, stage(buf) + piece * 512);
     }
   };
 
@@ -178,7 +393,7 @@ __global__ __launch_bounds__(512, WC == 1 ? 2 : 4) void linear4_rows(L4Args a) {
   const int p0 = slot * NP;
   auto bound = [&](int p) { return p * groups / kL4Parts; };
   int g = bound(p0), part = 0, pend = bound(p0 + 1);
-  const int gend = bound(p0 + NP);
+  const int end = bound(p0 + NP);
   // closes partition `part` of the slot: balanced-tree sums, every one started from +0
   auto close = [&]() {
 #pragma unroll
@@ -199,150 +414,85 @@ __global__ __launch_bounds__(512, WC == 1 ? 2 : 4) void linear4_rows(L4Args a) {
 #pragma unroll
   for (int s = 0; s < WK; ++s) steps = max(steps, bound((s + 1) * NP) - bound(s * NP));
 
-  if (g < gend) load(g);
-  for (int step = 0; step < steps; ++step, ++g) {
-    const int buf = NBUF == 2 ? step & 1 : 0;
-    const bool live = g < gend;
-    if (NBUF == 1 && WC > 1 && step) stage_barrier();  // the group before has been read
-    uint4v wcur = wd;
-    const float scale = bf16_to_float(sw), bias = bf16_to_float(bw);
-    if (live) stage(buf);
-    if (g + 1 < gend) load(g + 1);
-    if constexpr (WC > 1) {
-      wait_lgkmcnt<0>();
+  constexpr int N = WC == 4 ? 2 : 4;  // registers: 128 at WC = 4, for two workgroups on a CU
+  Words<N> words;
+  column.load(words, g);
+  if (g < end) load(0, g);
+  for (int step = 0; step < steps; step += N, g += N) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (step + j >= steps) break;
+      // this step's copy and words have landed; every wavefront is done with the other stage
+      wait_vmcnt<0>();
       stage_barrier();
-    } else {
-      __builtin_amdgcn_wave_barrier();
+      if (j == 0) column.align(words, g);
+      const Prepared w = prepare_group(words, j);
+      const float xsum = sum;
+      if (j == N - 1) column.load(words, g + N);
+      if (g + j + 1 < end) load((j + 1) & 1, g + j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (g + j >= end) continue;
+      while (part + 1 < NP && g + j >= pend) close();
+      const _Float16* const src = stage(j & 1) + lane * 8;
+      multiply_group(w,
+                     [&](int t, int s4) {
+                       return *reinterpret_cast<const bf16x8*>(src + t * kPlaneTerm + s4 * 512);
+                     },
+                     xsum, acc);
     }
-    if (!live) continue;
-    while (part + 1 < NP && g >= pend) close();
-    const uint16_t* const src = planes + (buf * WK + slot) * 3 * PLANE;
-    const int arow = l32 * 64;
-    // bias term: the lane's half-group sum X and b', six products of their terms in the lane's
-    // k-slots
-    const Split3 xs = split3(xg[buf][slot][hh][l32]), bs = split3(fmaf(8.0f, scale, bias));
-    const uint32_t b12 = upper_pair(bs.t[0], bs.t[1]);
-    const bf16x8 xa = __builtin_bit_cast(
-        bf16x8, uint4v{upper_pair(xs.t[0], xs.t[0]), upper_pair(xs.t[1], xs.t[1]),
-                       upper_pair(xs.t[0], xs.t[2]), 0u});
-    const bf16x8 xb =
-        __builtin_bit_cast(bf16x8, uint4v{b12, b12, upper_pair(bs.t[2], bs.t[0]), 0u});
-    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, xb, acc, 0, 0, 0);
-    floatx16 p;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) p[e] = 0.0f;
-    bf16x8 bq[4];
-#pragma unroll
-    for (int s4 = 0; s4 < 4; ++s4) bq[s4] = decode_centred(wcur[s4]);
-#pragma unroll
-    for (int plane = 2; plane >= 0; --plane)  // the smallest terms first
-#pragma unroll
-      for (int s4 = 0; s4 < 4; ++s4) {
-        const bf16x8 av = *reinterpret_cast<const bf16x8*>(
-            src + plane * PLANE + arow + 8 * ((4 * hh + s4) ^ ((l32 >> 1) & 7)));
-        p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bq[s4], p, 0, 0, 0);
-      }
-    const float s16 = 16.0f * scale;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[e] = fmaf(s16, p[e], acc[e]);
-    if constexpr (WC == 1) __builtin_amdgcn_wave_barrier();
   }
   while (part < NP) close();
-
-  // ---- sum over the slots in LDS, then whole-row stores ----
+  wait_vmcnt<0>();
   wait_lgkmcnt<0>();
-  stage_barrier();  // the x stages are free
-  float* const red = reinterpret_cast<float*>(mem);
-#pragma unroll
-  for (int e = 0; e < 16; ++e)
-    red[(wave * 32 + 8 * (e >> 2) + 4 * hh + (e & 3)) * kRedRow + l32] = total[e];
-  wait_lgkmcnt<0>();
-  stage_barrier();
-  // V consecutive columns of a row from column block cb
-  constexpr int V = TC * 32 / 512 < 4 ? TC * 32 / 512 : 4;
-  auto sum_slots = [&](int cb, int row, int col, float (&y)[V]) {
-    auto at = [&](int s, int j) { return red[((s * WC + cb) * 32 + row) * kRedRow + col + j]; };
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      if constexpr (WK == 8)
-        y[j] = ((at(0, j) + at(1, j)) + (at(2, j) + at(3, j))) +
-               ((at(4, j) + at(5, j)) + (at(6, j) + at(7, j)));
-      else if constexpr (WK == 4)
-        y[j] = (at(0, j) + at(1, j)) + (at(2, j) + at(3, j));
-      else
-        y[j] = at(0, j) + at(1, j);
-    }
-  };
-  auto store = [&](const L4Set& set, int row, int c0, const float (&y)[V]) {
-    float* const dst = set.out + static_cast<size_t>(row) * set.cols + c0;
-    if (a.vec && V == 4 && c0 + V <= set.cols) {
-      *reinterpret_cast<floatx4*>(dst) = floatx4{y[0], y[1], y[V > 2 ? 2 : 0], y[V > 2 ? 3 : 0]};
-    } else if (a.vec && V == 2 && c0 + V <= set.cols) {
-      *reinterpret_cast<float2v*>(dst) = float2v{y[0], y[1]};
-    } else {
-#pragma unroll
-      for (int j = 0; j < V; ++j)
-        if (c0 + j < set.cols) dst[j] = y[j];
-    }
-  };
-#pragma unroll
-  for (int i = 0; i < TC * 32 / (512 * V); ++i) {
-    const int at = V * (tid + 512 * i), row = at / TC, c = at % TC;
-    if (rbase + row >= a.row1) continue;
-    float y[V];
-    sum_slots(c >> 5, row, c & 31, y);
-    if constexpr (GATED) {
-      float up[V];
-      sum_slots((c >> 5) + WC / 2, row, c & 31, up);
-      if (a.set[1].out) store(a.set[1], rbase + row, tile * TC + c, up);
-#pragma unroll
-      for (int j = 0; j < V; ++j) y[j] = silu_times(y[j], up[j]);
-    }
-    store(a.set[GATED ? 0 : first], rbase + row, tile * TC + c, y);
-  }
+  stage_barrier();  // the stages are free
+  store_tile<WC, WK, GATED>(a, reinterpret_cast<float*>(mem), total, slot, wc, first, tile, rbase);
 }
 
-// Column blocks per workgroup for `tiles` 32 x 32 output tiles.
-int l4_blocks(int64_t tiles) { return tiles >= 2048 ? 4 : tiles >= 512 ? 2 : 1; }
+template <int WIDTH>
+dim3 l4_grid(const L4Args& a, int sets) {
+  unsigned tiles = 0;
+  for (int i = 0; i < sets; ++i)
+    tiles += static_cast<unsigned>((a.set[i].cols + WIDTH - 1) / WIDTH);
+  return dim3(static_cast<unsigned>((a.row1 - a.row0 + kPlaneRows - 1) / kPlaneRows), tiles);
+}
+
+void run_rows(const L4Args& a, int sets, hipStream_t st) {
+  linear4_rows<<<l4_grid<32>(a, sets), 512, 0, st>>>(a);
+}
 
 template <int WC, bool GATED>
-void run_rows(const L4Args& a, int sets, hipStream_t st) {
-  constexpr int TC = GATED ? 16 * WC : 32 * WC;
-  unsigned tiles = 0;
-  for (int i = 0; i < (GATED ? 1 : sets); ++i)
-    tiles += static_cast<unsigned>((a.set[i].cols + TC - 1) / TC);
-  const dim3 grid(static_cast<unsigned>((a.row1 - a.row0 + 31) / 32), tiles);
-  linear4_rows<WC, 8 / WC, GATED><<<grid, 512, 0, st>>>(a);
+void run_shared(const L4Args& a, int sets, hipStream_t st) {
+  linear4_rows_shared<WC, GATED>
+      <<<l4_grid<GATED ? 16 * WC : 32 * WC>(a, GATED ? 1 : sets), 512, 0, st>>>(a);
 }
 
-hipError_t launch_rows(const Linear4Job* jobs, int count, bool gated, hipStream_t st) {
-  const Linear4Job& j = jobs[0];
+hipError_t launch_rows(const Linear4Job* jobs, int count, bool gated, const Planes& x, int row0,
+                       int row1, const Planes& next, hipStream_t st) {
   L4Args a{};
-  a.x = j.x;
-  a.row0 = j.row0;
-  a.row1 = j.row1;
-  a.k = j.k;
+  a.x = x;
+  a.row0 = row0;
+  a.row1 = row1;
+  a.k = jobs[0].k;
   a.vec = 1;
+  a.next = next;
   int64_t tiles = 0;
   for (int i = 0; i < count; ++i) {
     a.set[i] = L4Set{jobs[i].w, jobs[i].scales, jobs[i].biases, jobs[i].out, jobs[i].cols};
     if (jobs[i].cols % 4 || (reinterpret_cast<uintptr_t>(jobs[i].out) & 15)) a.vec = 0;
     tiles += (jobs[i].cols + 31) / 32;
   }
-  tiles *= (j.row1 - j.row0 + 31) / 32;
-  const int wc = l4_blocks(tiles);
-  if (gated) {
-    if (wc == 4)
-      run_rows<4, true>(a, count, st);
-    else
-      run_rows<2, true>(a, count, st);
-  } else if (wc == 4) {
-    run_rows<4, false>(a, count, st);
-  } else if (wc == 2) {
-    run_rows<2, false>(a, count, st);
-  } else {
-    run_rows<1, false>(a, count, st);
-  }
+  tiles *= (row1 - row0 + kPlaneRows - 1) / kPlaneRows;
+  // the widest tile that still has a workgroup for (nearly) every CU: one 32 x 32 tile each up to
+  // 256 (q, k and v of 48 rows 6.0 us, 8.1 with two blocks), two up to 512 (o of 308 rows 12.1 us,
+  // 14.3 with one and 18.8 with four), else four (gate and up of 1000 rows 55 us, 86 with two)
+  if (tiles > 512)
+    gated ? run_shared<4, true>(a, count, st) : run_shared<4, false>(a, count, st);
+  else if (gated)
+    run_shared<2, true>(a, count, st);
+  else if (tiles > 256)
+    run_shared<2, false>(a, count, st);
+  else
+    run_rows(a, count, st);
   return hipGetLastError();
 }
 
@@ -369,25 +519,54 @@ bool linear4_on_rows(const Linear4Job& j, const float* scratch, size_t scratch_f
   return !runs_hilo(j, scratch, scratch_floats);
 }
 
-hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated, hipStream_t st) {
+hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated,
+                               const PlanesScratch& scratch, bool prepared, bool keep,
+                               hipStream_t st) {
   if (count < 1 || count > 3 || (gated && (count != 2 || jobs[0].cols != jobs[1].cols)))
     return hipErrorInvalidValue;
+  const Linear4Job& j = jobs[0];
   for (int i = 0; i < count; ++i)
-    if (jobs[i].x != jobs[0].x || jobs[i].row0 != jobs[0].row0 || jobs[i].row1 != jobs[0].row1 ||
-        jobs[i].k != jobs[0].k || jobs[i].cols <= 0 || jobs[i].k <= 0 || jobs[i].k % 64)
+    if (jobs[i].x != j.x || jobs[i].row0 != j.row0 || jobs[i].row1 != j.row1 ||
+        jobs[i].k != j.k || jobs[i].cols <= 0 || j.k <= 0 || j.k % 64 || j.k > 65536)
       return hipErrorInvalidValue;
-  if (jobs[0].row1 <= jobs[0].row0) return hipSuccess;
-  return launch_rows(jobs, count, gated, st);
+  if (j.row1 <= j.row0) return hipSuccess;
+  const int rows = j.row1 - j.row0;
+  Planes next{};
+  if (keep) {
+    if (!gated || j.row0 || j.cols % 64 || planes_bytes(rows, j.cols) > scratch.bytes)
+      return hipErrorInvalidValue;
+    next = planes_at(scratch.out, rows, j.cols);
+  }
+  if (prepared) {
+    if (j.row0 || planes_bytes(rows, j.k) > scratch.bytes) return hipErrorInvalidValue;
+    return launch_rows(jobs, count, gated, planes_at(scratch.in, rows, j.k), 0, j.row1, next, st);
+  }
+  // x in ranges of whole row tiles whose planes fit the scratch (one range for most shapes; an
+  // output kept as planes is within it)
+  const size_t tile_bytes = planes_bytes(kPlaneRows, j.k);
+  const int64_t fit = static_cast<int64_t>(scratch.bytes / tile_bytes);
+  if (fit < 1) return hipErrorInvalidValue;
+  const int step = static_cast<int>(std::min<int64_t>(fit * kPlaneRows, 1 << 20));
+  if (keep && step < rows) return hipErrorInvalidValue;
+  for (int r = j.row0; r < j.row1; r += std::min(step, j.row1 - r)) {
+    const int end = r + std::min(step, j.row1 - r);
+    const Planes x = planes_at(scratch.in, end - r, j.k);
+    const dim3 grid((end - r + kPlaneRows - 1) / kPlaneRows, j.k / 64);
+    split_planes<<<grid, 256, 0, st>>>(j.x, x, r, end, j.k);
+    const hipError_t e = launch_rows(jobs, count, gated, x, r, end, next, st);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_linear4_f32(const Linear4Job& j, float* scratch, size_t scratch_floats,
-                              hipStream_t st) {
+                              const PlanesScratch& planes, hipStream_t st) {
   if (j.row1 <= j.row0 || j.cols <= 0) return hipSuccess;
   if (runs_hilo(j, scratch, scratch_floats))
     return launch_linear4_hilo_f32(j.x + static_cast<size_t>(j.row0) * j.k, j.w, j.scales, j.biases,
                                    j.out + static_cast<size_t>(j.row0) * j.cols, j.row1 - j.row0,
                                    j.cols, j.k, scratch, scratch_floats, st);
-  return launch_linear4_rows(&j, 1, false, st);
+  return launch_linear4_rows(&j, 1, false, planes, false, false, st);
 }
 
 hipError_t launch_silu_gate_f32(float* gate, const float* up, uint32_t n, hipStream_t st) {

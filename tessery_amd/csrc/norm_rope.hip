@@ -11,6 +11,7 @@
 // (seq, D, theta); the allocation-free entry point rebuilds it in its scratch on every call.
 #include "common.h"
 #include "kernels.h"
+#include "planes.h"
 
 namespace tessery {
 
@@ -31,10 +32,12 @@ __device__ __forceinline__ float rope_second(float a, float b, float cv, float s
 }
 
 // One wavefront per row, 4 rows per 256-thread workgroup. out may alias x. With VEC (cols a
-// multiple of 4, x and out 16-byte aligned) rows are read and written as float4.
-template <bool VEC>
+// multiple of 4, x and out 16-byte aligned) rows are read and written as float4. With PLANES (VEC,
+// cols a multiple of 64) the result also goes out as planes.h's terms, for the projections after it.
+template <bool VEC, bool PLANES>
 __global__ __launch_bounds__(256) void rms_norm_f32(const float* x, const uint16_t* __restrict__ w,
-                                                    float* out, int rows, int cols, float eps) {
+                                                    float* out, int rows, int cols, float eps,
+                                                    Planes planes) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;  // row-uniform: the whole wavefront leaves together
@@ -57,6 +60,7 @@ __global__ __launch_bounds__(256) void rms_norm_f32(const float* x, const uint16
 #pragma unroll
       for (int j = 0; j < 4; ++j) r[j] = v[j] * inv * bf16_to_float(w[4 * c + j]);
       y4[c] = r;
+      if constexpr (PLANES) store_planes4(planes, row, 4 * c, cols >> 6, r);
     }
     return;
   }
@@ -193,22 +197,30 @@ __global__ __launch_bounds__(256) void norm_rope_f16(const _Float16* __restrict_
 }
 
 hipError_t launch_rms_norm_f32(const float* x, const uint16_t* w, float* out, int rows, int cols,
-                               float eps, hipStream_t st) {
+                               float eps, void* planes, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
   const bool vec = (cols & 3) == 0 &&
                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-  if (vec)
-    rms_norm_f32<true><<<(rows + 3) / 4, 256, 0, st>>>(x, w, out, rows, cols, eps);
+  if (planes && (!vec || cols % 64)) return hipErrorInvalidValue;
+  const dim3 grid((rows + 3) / 4);
+  if (planes)
+    rms_norm_f32<true, true><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps,
+                                                   planes_at(planes, rows, cols));
+  else if (vec)
+    rms_norm_f32<true, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{});
   else
-    rms_norm_f32<false><<<(rows + 3) / 4, 256, 0, st>>>(x, w, out, rows, cols, eps);
+    rms_norm_f32<false, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{});
   return hipGetLastError();
 }
 
 // add(x, r -> x) followed by rms_norm(x -> y), one wavefront per row, float4 pieces: the sum
 // is stored to x, and y takes the bits of the separate float4 rms_norm (same order of squares).
+// PLANES: as in rms_norm_f32.
+template <bool PLANES>
 __global__ __launch_bounds__(256) void add_rms_norm_f32(float* x, const float* __restrict__ r,
                                                         const uint16_t* __restrict__ w, float* y,
-                                                        int rows, int cols, float eps) {
+                                                        int rows, int cols, float eps,
+                                                        Planes planes) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -234,17 +246,25 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32(float* x, const float* _
 #pragma unroll
     for (int j = 0; j < 4; ++j) o[j] = v[j] * inv * bf16_to_float(w[4 * c + j]);
     y4[c] = o;
+    if constexpr (PLANES) store_planes4(planes, row, 4 * c, cols >> 6, o);
   }
 }
 
 hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, float* y,
-                                   int rows, int cols, float eps, hipStream_t st) {
+                                   int rows, int cols, float eps, void* planes,
+                                   hipStream_t st) {
   if (rows <= 0) return hipSuccess;
+  if (planes && cols % 64) return hipErrorInvalidValue;
   if (cols <= 0 || cols % 4 ||
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(r) |
         reinterpret_cast<uintptr_t>(y)) & 15))
     return hipErrorNotReady;  // the separate launches run instead
-  add_rms_norm_f32<<<(rows + 3) / 4, 256, 0, st>>>(x, r, w, y, rows, cols, eps);
+  const dim3 grid((rows + 3) / 4);
+  if (planes)
+    add_rms_norm_f32<true><<<grid, 256, 0, st>>>(x, r, w, y, rows, cols, eps,
+                                                 planes_at(planes, rows, cols));
+  else
+    add_rms_norm_f32<false><<<grid, 256, 0, st>>>(x, r, w, y, rows, cols, eps, Planes{});
   return hipGetLastError();
 }
 

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "kernels.h"
+#include "planes.h"
 #include "tessery_hip.h"
 
 using tessery::Params;
@@ -158,6 +159,7 @@ struct Runtime {
   uint64_t graph_launches = 0, graph_builds = 0;
   uint64_t fused_pairs = 0, fused_gated = 0;  // launch-time fusions (diagnostics)
   float* dense_scratch = nullptr;  // split-K partial sums of small-batch projections
+  void* planes[2] = {};  // planes of the activations uint4 projections read, and of their output
   std::vector<Segment> segments;
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_end = nullptr;
@@ -559,9 +561,19 @@ bool ensure_rope(Runtime* rt, uint32_t seq, uint32_t dim, float theta) {
   return true;
 }
 
+bool is_linear4(Route r) {
+  return r == R_LINEAR4 || r == R_LINEAR4_TILED || r == R_LINEAR4_TAIL || r == R_LINEAR4_16X32 ||
+         r == R_LINEAR4_32X32 || r == R_LINEAR4_SMALL3;
+}
+
+bool is_gated4(Route r) { return r == R_GATED4_16X32 || r == R_GATED4_8X32; }
+
 // Scratch of the split-K projection paths (dense and uint4), allocated once per runtime on first
 // use (its address never changes, so a captured graph keeps pointing at it).
 constexpr size_t kDenseScratchFloats = size_t{8} << 20;  // 32 MiB
+// Each of the two planes scratches: 1023 rows (more run on linear4_hilo) of 3072 inputs, Qwen3's
+// widest, in 18.4 MiB. Others go through it in row ranges.
+constexpr size_t kPlanesBytes = size_t{20} << 20;
 
 bool prepare(Runtime* rt, Route r, const Params& p) {
   switch (r) {
@@ -587,6 +599,11 @@ bool prepare(Runtime* rt, Route r, const Params& p) {
         rt->dense_scratch = nullptr;
         return false;
       }
+      for (void*& p : rt->planes)
+        if ((is_linear4(r) || is_gated4(r)) && !p && hipMalloc(&p, kPlanesBytes) != hipSuccess) {
+          p = nullptr;
+          return false;
+        }
       return true;
     default:
       return true;
@@ -654,13 +671,6 @@ bool attention_args(Runtime* rt, const Op& op, tessery::AttnArgs* out) {
   return true;
 }
 
-bool is_linear4(Route r) {
-  return r == R_LINEAR4 || r == R_LINEAR4_TILED || r == R_LINEAR4_TAIL || r == R_LINEAR4_16X32 ||
-         r == R_LINEAR4_32X32 || r == R_LINEAR4_SMALL3;
-}
-
-bool is_gated4(Route r) { return r == R_GATED4_16X32 || r == R_GATED4_8X32; }
-
 // The projection of a linear4 op (buffers x, w, scales, biases, out).
 bool linear4_job(const Op& op, tessery::Linear4Job* job) {
   RowRange rr;
@@ -692,7 +702,13 @@ bool gated4_jobs(const Op& op, tessery::Linear4Job* jobs) {
   return true;
 }
 
-hipError_t launch(Runtime* rt, const Op& op) {
+// `in` is the planes scratch `slot`, `out` the other one.
+tessery::PlanesScratch planes_scratch(Runtime* rt, int slot) {
+  return {rt->planes[slot], rt->planes[1 - slot], kPlanesBytes};
+}
+
+// planes: where a rms_norm also leaves its output as planes (null: nowhere).
+hipError_t launch(Runtime* rt, const Op& op, void* planes) {
   hipStream_t st = rt->stream;
   const Params& p = op.p;
   switch (op.route) {
@@ -725,7 +741,7 @@ hipError_t launch(Runtime* rt, const Op& op) {
       return tessery::launch_rms_norm_f32(
           static_cast<const float*>(op.ptr[0]), static_cast<const uint16_t*>(op.ptr[1]),
           static_cast<float*>(op.ptr[2]), static_cast<int>(op.threads / 32),
-          static_cast<int>(p.cols), p.eps, st);
+          static_cast<int>(p.cols), p.eps, planes, st);
     case R_ROPE: {
       const RopeTable* t = rope_of(rt, p);
       if (!t) return hipErrorInvalidValue;
@@ -741,7 +757,8 @@ hipError_t launch(Runtime* rt, const Op& op) {
     case R_LINEAR4_SMALL3: {
       tessery::Linear4Job job;
       if (!linear4_job(op, &job)) return hipErrorInvalidValue;
-      return tessery::launch_linear4_f32(job, rt->dense_scratch, kDenseScratchFloats, st);
+      return tessery::launch_linear4_f32(job, rt->dense_scratch, kDenseScratchFloats,
+                                         planes_scratch(rt, 0), st);
     }
     case R_QKV4_F16:
       return tessery::launch_qkv4_f16(qkv4_args(op), st);
@@ -749,7 +766,7 @@ hipError_t launch(Runtime* rt, const Op& op) {
     case R_GATED4_8X32: {
       tessery::Linear4Job jobs[2];
       if (!gated4_jobs(op, jobs)) return hipErrorInvalidValue;
-      return tessery::launch_linear4_rows(jobs, 2, true, st);
+      return tessery::launch_linear4_rows(jobs, 2, true, planes_scratch(rt, 0), false, false, st);
     }
     case R_SILU_GATE:
       return tessery::launch_silu_gate_f32(static_cast<float*>(op.ptr[0]),
@@ -877,6 +894,8 @@ void mi_destroy(void* runtime) {
     (void)hipFree(kv.second.sin);
   }
   if (rt->dense_scratch) (void)hipFree(rt->dense_scratch);
+  for (void* p : rt->planes)
+    if (p) (void)hipFree(p);
   release_profile_events(rt);
   if (rt->ev_start) (void)hipEventDestroy(rt->ev_start);
   if (rt->ev_end) (void)hipEventDestroy(rt->ev_end);
@@ -984,7 +1003,7 @@ hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
 //     same shape and lengths, neither writing a buffer of the other -> the attention launch with
 //     the prologue in extra workgroups.
 // Returns the launch status, or hipErrorNotReady when ops[i], ops[i + 1] are not such a pair.
-hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b) {
+hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes) {
   hipStream_t st = rt->stream;
   if (is_linear4(a.route)) return launch_fused_dual(rt, a, b, false);
   const bool projection = a.route == R_MATMUL || a.route == R_MATMUL_TILED ||
@@ -1017,7 +1036,7 @@ hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b) {
     return tessery::launch_add_rms_norm_f32(
         static_cast<float*>(a.ptr[0]), static_cast<const float*>(a.ptr[1]),
         static_cast<const uint16_t*>(b.ptr[1]), static_cast<float*>(b.ptr[2]),
-        static_cast<int>(b.threads / 32), static_cast<int>(b.p.cols), b.p.eps, st);
+        static_cast<int>(b.threads / 32), static_cast<int>(b.p.cols), b.p.eps, planes, st);
   }
   if (a.route == R_QKV4_F16 && b.route == R_NORM_ROPE_F16 && b.ptr[0] == a.ptr[5] &&
       b.p.dim == 128 && static_cast<uint64_t>(b.p.heads) * 128 == a.p.n &&
@@ -1158,41 +1177,53 @@ bool linear4_run(Runtime* rt, size_t first, size_t last, Linear4Run* run) {
   return true;
 }
 
-// The linear4_rows launch that starts at op `first`: up to three projections of the same rows of
-// one x queued one after the other (q, k and v), two of them with the silu_gate that follows
-// (gate and up), each over its whole run of row ranges, or the row ranges of a gated4 projection.
-// *taken: the ops it ran. hipErrorNotReady: op `first` is no such projection.
-hipError_t launch_linear4_runs(Runtime* rt, size_t first, size_t last, size_t* taken) {
+// A linear4_rows launch over ops [first, end).
+struct Projection {
+  tessery::Linear4Job jobs[3];
+  int count;
+  bool gated;
+  size_t end;
+};
+
+// The launch that starts at op `first`: up to three projections of the same rows of one x queued one
+// after the other (q, k and v), two of them with the silu_gate that follows (gate and up), each
+// over its whole run of row ranges, or the row ranges of a gated4 projection. False: op `first`
+// is no projection that linear4_rows runs.
+bool find_projection(Runtime* rt, size_t first, size_t last, Projection* p) {
   const Op& a = rt->ops[first];
   if (is_gated4(a.route)) {
-    tessery::Linear4Job jobs[2], next[2];
-    if (!gated4_jobs(a, jobs)) return hipErrorInvalidValue;
-    size_t end = first + 1;
+    tessery::Linear4Job next[2];
+    if (!gated4_jobs(a, p->jobs)) return false;
+    p->count = 2;
+    p->gated = true;
+    p->end = first + 1;
     bool apart = true;  // the output is none of the inputs
     for (int i = 0; i < 7; ++i) apart = apart && a.ptr[i] != a.ptr[7];
-    for (; apart && end < last; ++end) {
-      const Op& b = rt->ops[end];
+    for (; apart && p->end < last; ++p->end) {
+      const Op& b = rt->ops[p->end];
       if (!gated4_jobs(b, next) || a.ptr != b.ptr || b.p.rows != a.p.rows ||
-          next[0].cols != jobs[0].cols || next[0].k != jobs[0].k || next[0].row0 != jobs[0].row1)
+          next[0].cols != p->jobs[0].cols || next[0].k != p->jobs[0].k ||
+          next[0].row0 != p->jobs[0].row1)
         break;
-      jobs[0].row1 = jobs[1].row1 = next[0].row1;
+      p->jobs[0].row1 = p->jobs[1].row1 = next[0].row1;
     }
-    *taken = end - first;
-    return tessery::launch_linear4_rows(jobs, 2, true, rt->stream);
+    return true;
   }
   Linear4Run run;
-  if (!is_linear4(a.route) || !linear4_run(rt, first, last, &run)) return hipErrorNotReady;
-  tessery::Linear4Job jobs[3] = {run.job};
+  if (!is_linear4(a.route) || !linear4_run(rt, first, last, &run)) return false;
+  p->jobs[0] = run.job;
+  p->gated = false;
+  p->count = 1;
   size_t ends[3] = {run.end, 0, 0};
-  int count = 1;
-  while (count < 3 && ends[count - 1] < last &&
-         linear4_run(rt, ends[count - 1], last, &run)) {
+  while (p->count < 3 && ends[p->count - 1] < last &&
+         linear4_run(rt, ends[p->count - 1], last, &run)) {
     const tessery::Linear4Job& j = run.job;
-    bool joins = j.x == jobs[0].x && j.k == jobs[0].k && j.row0 == jobs[0].row0 &&
-                 j.row1 == jobs[0].row1 && static_cast<const void*>(j.out) != j.x;
+    const tessery::Linear4Job& lead = p->jobs[0];
+    bool joins = j.x == lead.x && j.k == lead.k && j.row0 == lead.row0 && j.row1 == lead.row1 &&
+                 static_cast<const void*>(j.out) != j.x;
     // no output is an input or output of another projection of the launch
-    for (int i = 0; i < count && joins; ++i) {
-      const tessery::Linear4Job& o = jobs[i];
+    for (int i = 0; i < p->count && joins; ++i) {
+      const tessery::Linear4Job& o = p->jobs[i];
       for (const void* in : {static_cast<const void*>(j.x), static_cast<const void*>(j.w),
                              static_cast<const void*>(j.scales),
                              static_cast<const void*>(j.biases), static_cast<const void*>(j.out)})
@@ -1202,58 +1233,115 @@ hipError_t launch_linear4_runs(Runtime* rt, size_t first, size_t last, size_t* t
         joins = joins && in != j.out;
     }
     if (!joins) break;
-    jobs[count] = j;
-    ends[count++] = run.end;
+    p->jobs[p->count] = j;
+    ends[p->count++] = run.end;
   }
   // gate, up, silu_gate(gate, up) over every row
-  if (count >= 2 && ends[1] < last && jobs[0].cols == jobs[1].cols && jobs[0].row0 == 0) {
+  if (p->count >= 2 && ends[1] < last && p->jobs[0].cols == p->jobs[1].cols &&
+      p->jobs[0].row0 == 0) {
     const Op& c = rt->ops[ends[1]];
-    if (c.route == R_SILU_GATE && c.ptr[0] == jobs[0].out && c.ptr[1] == jobs[1].out &&
+    if (c.route == R_SILU_GATE && c.ptr[0] == p->jobs[0].out && c.ptr[1] == p->jobs[1].out &&
         static_cast<uint64_t>(c.p.n) ==
-            static_cast<uint64_t>(jobs[0].row1) * static_cast<uint64_t>(jobs[0].cols)) {
-      *taken = ends[1] + 1 - first;
-      return tessery::launch_linear4_rows(jobs, 2, true, rt->stream);
+            static_cast<uint64_t>(p->jobs[0].row1) * static_cast<uint64_t>(p->jobs[0].cols)) {
+      p->count = 2;
+      p->gated = true;
+      p->end = ends[1] + 1;
+      return true;
     }
   }
-  *taken = ends[count - 1] - first;
-  return tessery::launch_linear4_rows(jobs, count, false, rt->stream);
+  p->end = ends[p->count - 1];
+  return true;
+}
+
+// What the launch before left for the next one: the planes of x [rows, k], in a planes scratch.
+struct Ready {
+  const void* x = nullptr;
+  uint64_t rows = 0, k = 0;
+  int slot = 0;
+};
+
+// Launches of one pass over the queue: their fusions, and what the last one left behind.
+struct Pass {
+  FusionCount fused;
+  Ready ready;
+};
+
+// Whether op `at` starts a projection that reads all of x [rows, k] as planes the scratch holds.
+bool reads_planes(Runtime* rt, size_t at, size_t last, const void* x, uint64_t rows, uint64_t k) {
+  Projection p;
+  return at < last && find_projection(rt, at, last, &p) && p.jobs[0].x == x &&
+         p.jobs[0].row0 == 0 && static_cast<uint64_t>(p.jobs[0].row1) == rows &&
+         static_cast<uint64_t>(p.jobs[0].k) == k && p.jobs[0].out != x &&
+         tessery::planes_bytes(p.jobs[0].row1, p.jobs[0].k) <= kPlanesBytes;
 }
 
 // Launches op `first` and those after it (before op `last`) that run inside the same kernel: the
-// runs launch_linear4_runs takes, the triples of launch_fused_gated and the pairs of
-// launch_fused_pair (the last two counted in *fc). *taken: the ops launched.
-hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, FusionCount* fc) {
-  const hipError_t rows = launch_linear4_runs(rt, first, last, taken);
-  if (rows != hipErrorNotReady) return rows;
+// projections find_projection takes, the triples of launch_fused_gated and the pairs of
+// launch_fused_pair (the last two counted). A kernel whose output the next launch projects leaves
+// its planes too. *taken: the ops launched.
+hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pass* pass) {
+  const Ready ready = pass->ready;
+  pass->ready = {};
+  const Op& op = rt->ops[first];
+  Projection p;
+  if (find_projection(rt, first, last, &p)) {
+    const tessery::Linear4Job& j = p.jobs[0];
+    const bool prepared = ready.x && ready.x == j.x && j.row0 == 0 &&
+                          ready.rows == static_cast<uint64_t>(j.row1) &&
+                          ready.k == static_cast<uint64_t>(j.k);
+    const int slot = prepared ? ready.slot : 0;
+    *taken = p.end - first;
+    const bool keep = p.gated && j.row0 == 0 && j.out != j.x &&
+                      tessery::planes_bytes(j.row1, j.k) <= kPlanesBytes &&
+                      reads_planes(rt, p.end, last, j.out, j.row1, j.cols);
+    if (keep)
+      pass->ready = {j.out, static_cast<uint64_t>(j.row1), static_cast<uint64_t>(j.cols), 1 - slot};
+    return tessery::launch_linear4_rows(p.jobs, p.count, p.gated, planes_scratch(rt, slot),
+                                        prepared, keep, rt->stream);
+  }
   const hipError_t gated =
-      first + 2 < last
-          ? launch_fused_gated(rt, rt->ops[first], rt->ops[first + 1], rt->ops[first + 2])
-          : hipErrorNotReady;
+      first + 2 < last ? launch_fused_gated(rt, op, rt->ops[first + 1], rt->ops[first + 2])
+                       : hipErrorNotReady;
   if (gated != hipErrorNotReady) {
-    fc->gated += gated == hipSuccess;
+    pass->fused.gated += gated == hipSuccess;
     *taken = 3;
     return gated;
   }
-  const hipError_t pair = first + 1 < last
-                              ? launch_fused_pair(rt, rt->ops[first], rt->ops[first + 1])
-                              : hipErrorNotReady;
-  if (pair != hipErrorNotReady) {
-    fc->pairs += pair == hipSuccess;
-    *taken = 2;
-    return pair;
+  // the planes of a rms_norm (alone, or after the add it runs with) that projections read
+  auto norm_ready = [&](size_t at) {
+    const Op& n = rt->ops[at];
+    const uint64_t rows = n.threads / 32;
+    if (n.route == R_RMS_NORM && reads_planes(rt, at + 1, last, n.ptr[2], rows, n.p.cols))
+      return Ready{n.ptr[2], rows, n.p.cols, 0};
+    return Ready{};
+  };
+  if (first + 1 < last) {
+    const Ready after = op.route == R_ADD ? norm_ready(first + 1) : Ready{};
+    const hipError_t pair = launch_fused_pair(rt, op, rt->ops[first + 1],
+                                              after.x ? rt->planes[after.slot] : nullptr);
+    if (pair != hipErrorNotReady) {
+      pass->fused.pairs += pair == hipSuccess;
+      pass->ready = after;
+      *taken = 2;
+      return pair;
+    }
   }
   *taken = 1;
-  return launch(rt, rt->ops[first]);
+  pass->ready = norm_ready(first);
+  return launch(rt, op, pass->ready.x ? rt->planes[pass->ready.slot] : nullptr);
 }
 
 // Launches ops [first, last) in order; the fusions made are added to *fc. Under stream capture
 // nothing runs yet, so the caller decides where the count goes (the runtime's totals for direct
 // launches, the cached graph for a capture).
 hipError_t launch_range(Runtime* rt, size_t first, size_t last, FusionCount* fc) {
+  Pass pass;
   for (size_t i = first, taken = 0; i < last; i += taken) {
-    const hipError_t e = launch_next(rt, i, last, &taken, fc);
+    const hipError_t e = launch_next(rt, i, last, &taken, &pass);
     if (e != hipSuccess) return e;
   }
+  fc->pairs += pass.fused.pairs;
+  fc->gated += pass.fused.gated;
   return hipSuccess;
 }
 
@@ -1353,10 +1441,10 @@ int mi_finish(void* runtime) {
     // ops that run inside the kernel of one before them: the first one's events enclose that
     // kernel, the others' enclose no work
     rt->profile_fused.assign(n, 0);
-    FusionCount fc;
+    Pass pass;
     for (size_t i = 0, taken = 0; i < n && !failed; i += taken) {
       if (hipEventRecord(rt->prof_events[2 * i], rt->stream) != hipSuccess ||
-          launch_next(rt, i, n, &taken, &fc) != hipSuccess ||
+          launch_next(rt, i, n, &taken, &pass) != hipSuccess ||
           hipEventRecord(rt->prof_events[2 * i + 1], rt->stream) != hipSuccess) {
         failed = 1;
         break;
@@ -1368,7 +1456,7 @@ int mi_finish(void* runtime) {
           failed = 1;
       }
     }
-    if (!failed) count_fusions(rt, fc);
+    if (!failed) count_fusions(rt, pass.fused);
   }
   if (hipEventRecord(rt->ev_end, rt->stream) != hipSuccess) failed = 1;
   if (hipStreamSynchronize(rt->stream) != hipSuccess) failed = 1;

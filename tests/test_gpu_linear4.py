@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from oracle import quant4 as ref
-from tessery_amd.workloads import bf16_words
+from tessery_amd.workloads import bf16_values, bf16_words
 from tests.conftest import GOLDEN
 from tests.test_gpu_attention import run
 
@@ -155,3 +155,82 @@ def test_large_batch_fp16_mfma_path(runtime, m, n, k):
     err = np.abs(got - want)
     assert np.all(err <= 2e-6 * bound + 1e-37), float((err / (bound + 1e-300)).max())
     assert not np.any(got[0])
+
+
+# Rows and columns at the edges of the 32 x 32 tiles, one to four of them a workgroup (up to 256
+# tiles, up to 512, more), and K of 1, 3, 7, 17 and 48 groups: fewer than the eight partitions,
+# uneven ones, odd counts (scales and biases at both parities of a dword).
+@pytest.mark.parametrize("m,n,k", [(1, 8, 64), (31, 33, 192), (32, 96, 448), (33, 160, 1088),
+                                   (65, 1056, 1088), (257, 1024, 3072), (255, 1031, 64),
+                                   (289, 2080, 448), (1023, 128, 192), (1030, 1056, 192)])
+def test_split_bf16_rows_kernel_at_its_edges(runtime, m, n, k):
+    """Every output within 1e-6 of sum_k |x| |w| of float64 (fp32 sums of exact products: an error
+    of a few 2^-24 a partial sum, at most 96 of them), rows past the range untouched; row
+    magnitudes spread over 2^-20 .. 2^20."""
+    x, packed, scales, biases = make(55 + m + k, m, n, k)
+    x *= np.exp2(np.random.default_rng(m).integers(-20, 21, m)).astype(np.float32)[:, None]
+    got = project(runtime, [x, packed, scales, biases], m, n, k,
+                  out=np.full((m + 1, n), np.nan, np.float32))
+    assert np.isnan(got[m:]).all()
+    w = ref.dequantize(packed, scales, biases, k)
+    err = np.abs(got[:m] - x.astype(np.float64) @ w.T)
+    bound = 1e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    assert np.all(err <= bound), float((err / bound).max())
+
+
+@pytest.mark.parametrize("m,seq_of_ops", [(24, "norm"), (77, "norm"), (24, "add"), (308, "add"),
+                                          (37, "gated"), (24, "gated"), (200, "gated")])
+def test_projections_beside_each_other_keep_their_bits(runtime, m, seq_of_ops):
+    """q, k and v (and gate, up, silu_gate, down) queued in one command, after the norm that makes
+    their input, run as fewer launches than queued one by one, on activations that the launch
+    before split; every buffer holds the bits of separate commands."""
+    hidden, inter = 1024, 3072
+    rng = np.random.default_rng(m)
+    x, r = [rng.normal(size=(m, hidden)).astype(np.float32) for _ in range(2)]
+    gamma = bf16_words(rng.uniform(0.5, 1.5, hidden))
+
+    def weights(n, k):
+        return [ref.pack(rng.integers(0, 16, size=(n, k), dtype=np.uint32)),
+                bf16_words(rng.uniform(0.01, 0.2, size=(n, k // 64)) / 8),
+                bf16_words(rng.uniform(-1, 0.1, size=(n, k // 64)) / 8)]
+
+    sets = ([weights(inter, hidden), weights(inter, hidden), weights(hidden, inter)]
+            if seq_of_ops == "gated" else [weights(n, hidden) for n in (2048, 1024, 1024)])
+    results = []
+    for separate in (False, True):
+        bufs = [runtime.upload(a) for a in (x, r, gamma)]
+        wb = [[runtime.upload(a) for a in w] for w in sets]
+        h = runtime.buffer(x.nbytes)
+        outs = [runtime.buffer(m * w[0].shape[0] * 4) for w in sets]
+        steps = []
+        if seq_of_ops == "add":
+            steps.append(lambda: runtime._dispatch("add", [bufs[0], bufs[1], bufs[0]],
+                                                   threads=x.size, n=x.size))
+        steps.append(lambda: runtime._dispatch("rms_norm", [bufs[0], bufs[2], h], threads=m * 32,
+                                               group_size=32, cols=hidden, eps=1e-6))
+        if seq_of_ops == "gated":
+            steps.append(lambda: runtime._gated4([h, *wb[0], *wb[1], outs[0], outs[1]], rows=m,
+                                                 cols=inter, k=hidden))
+            steps.append(lambda: runtime._linear4([outs[0], *wb[2], outs[2]], rows=m, cols=hidden,
+                                                  k=inter))
+        else:
+            for w, out, a in zip(wb, outs, sets):
+                steps.append(lambda w=w, out=out, a=a: runtime._linear4(
+                    [h, *w, out], rows=m, cols=a[0].shape[0], k=hidden))
+        if separate:
+            for step in steps:
+                with runtime.command():
+                    step()
+        else:
+            with runtime.command():
+                for step in steps:
+                    step()
+        results.append([runtime.read(h, x.shape), *(runtime.read(o, (m, a[0].shape[0]))
+                                                    for o, a in zip(outs, sets))])
+        for b in [*bufs, *(b for w in wb for b in w), h, *outs]:
+            b.close()
+    for together, alone in zip(*results):
+        np.testing.assert_array_equal(together, alone)
+    xs = x.astype(np.float64) + (r if seq_of_ops == "add" else 0)
+    want = xs / np.sqrt((xs * xs).mean(-1, keepdims=True) + 1e-6) * bf16_values(gamma)
+    np.testing.assert_allclose(results[0][0], want, atol=1e-5, rtol=1e-5)
