@@ -11,6 +11,7 @@
 
 #include "common.h"
 #include "kernels.h"
+#include "lds_dma.h"
 
 namespace tessery {
 
@@ -150,8 +151,7 @@ __global__ __launch_bounds__(256) void matmul_f32(const float* __restrict__ a,
     }
 }
 
-// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA for large shapes (K % 32 == 0, N % 128
-// == 0, at least 256 tiles): a and bt are split exactly into three bf16 planes each (split3x8)
+// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are split exactly into three bf16 planes each (split3x8)
 // and every fp32 product is taken as the six terms b_i c_j with i + j <= 4 on
 // v_mfma_f32_32x32x16_bf16 in fp32 (the bf16 rate is 16x the fp32 one, so six products cost well
 // under half the fp32 instructions). Tile 64 rows x 128 columns; wavefront w
@@ -279,6 +279,205 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
   }
 }
 
+// ---- the same product with operands split beforehand (K % 32 == 0, K <= 512) ----
+//
+// split_dense makes the three bf16 terms of x and of the weights once, laid out as MFMA operands, for
+// all the projections of one x in one launch:
+// [row tile of 32][k-step of 16][term][lane][8], lane = row % 32 + 32 h holding inputs
+// 16 step + 8 h .. + 7. matmul_planes then only copies operands to LDS (global_load_lds_dwordx4:
+// whole KiB pieces, read back by lane, no bank conflicts) and multiplies, all of K in one workgroup:
+// no partial sums, and q, k and v in one launch. Measured, q, k and v of 656 rows: 3.4 + 12.3 us, 42
+// as three split-K launches of matmul_f32 with their reductions; of 4096: 5 + 28 us, 76 on matmul_x3.
+//
+// K order: two halves, each with its leading products in one sum and the five smaller ones in
+// another (only the leading ones round at the magnitude of the result), added at the end. It is
+// the same for every tile shape, so a row's bits depend on no other row and on no projection
+// beside it.
+constexpr int kDenseStep = 3 * 64 * 8;  // bf16 words of a row tile's k-step
+
+struct SplitArgs {
+  const float* src[4];  // x, then up to three weight matrices, rows of k floats
+  int row0[4], rows[4], tiles[4];
+  int count, k;
+  uint16_t* planes;  // the operands' planes, one after the other
+};
+
+// A workgroup splits 32 rows x 64 inputs of one operand: thread (row tid / 8, chunk tid % 8) 8 of
+// them. Rows past the last one repeat it.
+__global__ __launch_bounds__(256) void split_dense(SplitArgs a) {
+  int tile = blockIdx.x, which = 0;
+  size_t base = 0;
+  while (which + 1 < a.count && tile >= a.tiles[which]) {
+    tile -= a.tiles[which];
+    base += a.tiles[which];
+    ++which;
+  }
+  const int row = threadIdx.x >> 3, c = threadIdx.x & 7, kk = 64 * blockIdx.y + 8 * c;
+  if (kk >= a.k) return;
+  const int at = min(32 * tile + row, a.rows[which] - 1);
+  const float* const src = a.src[which] + static_cast<size_t>(a.row0[which] + at) * a.k + kk;
+  const floatx4 u = *reinterpret_cast<const floatx4*>(src);
+  const floatx4 v = *reinterpret_cast<const floatx4*>(src + 4);
+  uint4v t[3];
+  split3x8(u, v, t[0], t[1], t[2]);
+  uint16_t* const dst = a.planes + ((base + tile) * (a.k >> 4) + (kk >> 4)) * kDenseStep +
+                        (row + 32 * (c & 1)) * 8;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) *reinterpret_cast<uint4v*>(dst + i * 512) = t[i];
+}
+
+struct PlanesSet {
+  const float* bias;  // null: none
+  float* out;
+  int cols;
+  int tile0;  // first 32-column tile of its weights
+};
+struct PlanesArgs {
+  const uint16_t* x;
+  const uint16_t* w;
+  PlanesSet set[3];
+  int count, row0, row1, k;
+};
+
+// Tile 64 x 64, KS slots (one a half of K; KS = 1 takes them in turn) of 4 wavefronts of 32 x 32 each.
+// Two LDS stages of a 32-input chunk. While a chunk's products run, its wavefront reads the
+// operands of the next one from LDS and copies those of the one after, one instruction between two
+// products (issued together they cost as much as the products). Bound: few tiles, the issue and
+// latency of a chunk's copies; many, L2 (13 TB/s at 16384 rows). Tiles of 64 x 128 and 128 x 128,
+// which ask L2 for less, or more stages leave too few wavefronts on a CU to hide either: 16384 x
+// 1152 outputs 97 and 194 us, 130 with three stages, against 94. Workgroups are numbered so that
+// an XCD takes all columns of a row tile in turn, from its own L2.
+template <int KS, bool GELU>
+__global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(PlanesArgs a,
+                                                                          int row_tiles,
+                                                                          int col_tiles) {
+  constexpr int STAGE = 24 * 512;  // bf16 words: 12 KiB of x, then 12 KiB of weights
+  constexpr int COPIES = 6, READS = 12;
+  __shared__ __attribute__((aligned(1024))) uint16_t mem[2 * KS * STAGE];
+  const int block = blockIdx.x, turn = block >> 3;
+  const int rt = (block & 7) + 8 * (turn / col_tiles);
+  if (rt >= row_tiles) return;
+  int ct = turn % col_tiles, which = 0;
+  while (which + 1 < a.count && ct >= (a.set[which].cols + 63) / 64) {
+    ct -= (a.set[which].cols + 63) / 64;
+    ++which;
+  }
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
+  const int slot = wave >> 2, w4 = wave & 3, wr = w4 >> 1, wc = w4 & 1;
+  const int ksteps = a.k >> 4, chunks = a.k >> 5, half = chunks >> 1;
+  // A wavefront copies the 6 KiB of one operand tile: row tiles 0 and 1, column tiles 0 and 1.
+  // Row tiles past the last one read it again (their rows aren't stored).
+  const int last = (a.row1 - a.row0 - 1) >> 5;
+  const int from = w4 < 2 ? min(2 * rt + w4, last) : a.set[which].tile0 + 2 * ct + w4 - 2;
+  const uint16_t* const src =
+      (w4 < 2 ? a.x : a.w) + static_cast<size_t>(from) * ksteps * kDenseStep;
+  auto copy = [&](int i, int buf, int chunk) {
+    dma16_at(src + static_cast<size_t>(chunk) * (2 * kDenseStep) + i * 512, 16u * lane,
+             reinterpret_cast<_Float16*>(mem + (buf * KS + slot) * STAGE + (6 * w4 + i) * 512));
+  };
+  struct Operands {
+    bf16x8 x[2][3], y[2][3];
+  };
+  // read i of a chunk's operands, in the order the products need them: terms (2, 0), (1, 1), (0, 2)
+  auto read = [&](Operands& f, int i, int buf) {
+    const uint16_t* const at = mem + (buf * KS + slot) * STAGE + lane * 8;
+    const int t = i / 4, ks = (i >> 1) & 1;
+    if (i & 1)
+      f.y[ks][t] = *reinterpret_cast<const bf16x8*>(at + ((2 + wc) * 6 + ks * 3 + t) * 512);
+    else
+      f.x[ks][2 - t] = *reinterpret_cast<const bf16x8*>(at + (wr * 6 + ks * 3 + 2 - t) * 512);
+  };
+
+  floatx16 hi, lo, first;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) hi[e] = lo[e] = first[e] = 0.0f;
+  const int begin = slot ? half : 0, end = KS == 2 && !slot ? half : chunks;
+  const int steps = KS == 2 ? chunks - half : chunks;  // of the longer slot
+  Operands even, odd;
+  if (begin < end) {
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy(i, 0, begin);
+  }
+  wait_vmcnt<0>();
+  stage_barrier();
+  if (begin + 1 < end) {
+#pragma unroll
+    for (int i = 0; i < COPIES; ++i) copy(i, 1, begin + 1);
+  }
+#pragma unroll
+  for (int i = 0; i < READS; ++i) read(even, i, 0);
+  // chunk begin + step from `now`; `next` takes the one after
+  auto chunk = [&](int step, int buf, const Operands& now, Operands& next) {
+    // the next chunk's copy has landed, and every wavefront has read this one's stage
+    wait_vmcnt<0>();
+    wait_lgkmcnt<0>();
+    stage_barrier();
+    if (begin + step >= end) return;
+    const bool more = begin + step + 2 < end;
+    constexpr int term[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+#pragma unroll
+    for (int i = 0; i < 12; ++i) {
+      const int ks = i & 1, t = i >> 1;
+      floatx16& c = t < 5 ? lo : hi;
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][term[t][0]], now.y[ks][term[t][1]], c,
+                                                  0, 0, 0);
+      read(next, i, buf ^ 1);  // stale data after the last chunk, unused
+      if (more && (i & 1)) copy(i >> 1, buf, begin + step + 2);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (KS == 1 && step + 1 == half) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        first[e] = hi[e] + lo[e];
+        hi[e] = lo[e] = 0.0f;
+      }
+    }
+  };
+  for (int step = 0; step < steps; step += 2) {
+    chunk(step, 0, even, odd);
+    if (step + 1 < steps) chunk(step + 1, 1, odd, even);
+  }
+  floatx16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = hi[e] + lo[e];
+  // the last chunk's reads ahead have landed before the kernel ends or reuses their stage
+  wait_lgkmcnt<0>();
+
+  if constexpr (KS == 2) {
+    // the second half's sums through LDS to the first slot
+    stage_barrier();  // the stages are free
+    floatx4* const sums = reinterpret_cast<floatx4*>(mem) + w4 * 256 + lane;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (slot) sums[q * 64] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+    wait_lgkmcnt<0>();
+    stage_barrier();
+    if (slot) return;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 second = sums[q * 64];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        first[4 * q + j] = acc[4 * q + j];
+        acc[4 * q + j] = second[j];
+      }
+    }
+  }
+  const PlanesSet set = a.set[which];
+  const int col = ct * 64 + 32 * wc + l32;
+  if (col >= set.cols) return;
+  const float bias = set.bias ? set.bias[col] : 0.0f;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int r = a.row0 + rt * 64 + 32 * wr + 8 * (e >> 2) + 4 * hh + (e & 3);
+    if (r >= a.row1) continue;
+    float y = first[e] + acc[e];
+    if (set.bias) y += bias;
+    set.out[static_cast<size_t>(r) * set.cols + col] = GELU ? gelu_value(y) : y;
+  }
+}
+
 // Split-K epilogue: out[r][n] = sum over z in order of part[z][r - row0][n] (+ bias, GELU).
 template <bool BIAS, bool GELU>
 __global__ __launch_bounds__(256) void dense_reduce(const float* __restrict__ part,
@@ -394,25 +593,114 @@ int dense_splits(int rows, int cols, int k, size_t scratch_floats) {
   return splits;
 }
 
-// Workgroups along K for the split-bf16 kernel: 1 from 512 tiles of 64 x 128; from 64 tiles, enough
-// splits of at least two 32-wide chunks for about 768 workgroups when the partial sums fit the
-// scratch; 0 (the fp32 kernel) otherwise. Every split holds at least one chunk.
+// Workgroups along K for matmul_x3: 1 from 512 tiles of 64 x 128; from 64 tiles, enough splits of at
+// least two 32-wide chunks for about 768 workgroups; fewer tiles, for about 256 workgroups of at
+// least four chunks (656 x 384 outputs of K = 1536: 17.3 us with 7 to 12 splits, 20.8 with 4, 21.8
+// with 24, and 24.9 on matmul_f32); 0 (the fp32 kernel) where the partial sums do not fit the
+// scratch or K is short. Every split holds at least one chunk.
 static int x3_split_count(int rows, int cols, int k, int tiles, size_t scratch_floats) {
   if (tiles >= 512) return 1;
   const int chunks32 = k / 32;
-  if (tiles < 64 || chunks32 < 4) return 0;
-  int splits = std::min(chunks32 / 2, (768 + tiles - 1) / tiles);
+  if (tiles < 1 || chunks32 < (tiles < 64 ? 8 : 4)) return 0;
+  int splits = tiles < 64 ? std::min(chunks32 / 4, 256 / tiles)
+                          : std::min(chunks32 / 2, (768 + tiles - 1) / tiles);
   const int per = (chunks32 + splits - 1) / splits;
   splits = (chunks32 + per - 1) / per;
   if (splits < 2 || static_cast<size_t>(splits) * rows * cols > scratch_floats) return 0;
   return splits;
 }
 
-hipError_t launch_matmul_f32(const float* a, const float* bt, const float* bias, float* out,
-                             int row0, int row1, int cols, int k, bool gelu, float* scratch,
-                             size_t scratch_floats, hipStream_t st) {
-  if (row1 <= row0 || cols <= 0) return hipSuccess;
-  if (k <= 0) return hipErrorInvalidValue;
+template <int KS>
+static void run_planes(const PlanesArgs& a, bool gelu, hipStream_t st) {
+  const int row_tiles = (a.row1 - a.row0 + 63) / 64;
+  int col_tiles = 0;
+  for (int i = 0; i < a.count; ++i) col_tiles += (a.set[i].cols + 63) / 64;
+  const unsigned grid = 8u * static_cast<unsigned>((row_tiles + 7) / 8) *
+                        static_cast<unsigned>(col_tiles);
+  if (gelu)
+    matmul_planes<KS, true><<<grid, 256 * KS, 0, st>>>(a, row_tiles, col_tiles);
+  else
+    matmul_planes<KS, false><<<grid, 256 * KS, 0, st>>>(a, row_tiles, col_tiles);
+}
+
+static size_t dense_planes_bytes(int64_t rows, int k) {
+  return static_cast<size_t>((rows + 31) / 32) * static_cast<size_t>(k / 16) * kDenseStep * 2;
+}
+
+// K % 32 == 0 and 16-byte rows. Up to K = 512: beyond, one workgroup's walk over K is longer than
+// split-K launches and their reduction (656 x 384 outputs of K = 1536: 4.6 + 22 us against 17). Up
+// to 512 tiles of 64 x 128, where matmul_x3 fills the chip without split K and splits nothing
+// beforehand (16384 x 384 outputs of K = 384: 16 + 35 us against 40, 4096 x 1536: 8 + 38 against 42).
+bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
+  const int64_t tiles = static_cast<int64_t>((j.row1 - j.row0 + 63) / 64) * ((j.cols + 127) / 128);
+  return scratch.planes && j.k > 0 && j.k % 32 == 0 && j.k <= 512 && j.cols > 0 && tiles < 512 &&
+         dense_planes_bytes(64, j.k) * static_cast<size_t>((j.row1 - j.row0 + 63) / 64 + 3 * ((j.cols + 63) / 64)) <=
+             scratch.planes_bytes &&
+         ((reinterpret_cast<uintptr_t>(j.a) | reinterpret_cast<uintptr_t>(j.bt)) & 15) == 0;
+}
+
+hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
+                                const DenseScratch& scratch, hipStream_t st) {
+  if (count < 1 || count > 3) return hipErrorInvalidValue;
+  const DenseJob& j = jobs[0];
+  for (int i = 0; i < count; ++i)
+    if (jobs[i].a != j.a || jobs[i].row0 != j.row0 || jobs[i].row1 != j.row1 ||
+        jobs[i].k != j.k || !matmul_on_planes(jobs[i], scratch))
+      return hipErrorInvalidValue;
+  if (j.row1 <= j.row0) return hipSuccess;
+  const int rows = j.row1 - j.row0;
+  // every job fits the scratch with three times its own weights, so three of equal width do
+  size_t bytes = dense_planes_bytes((rows + 31) / 32 * 32, j.k);
+  for (int i = 0; i < count; ++i) bytes += dense_planes_bytes((jobs[i].cols + 63) / 64 * 64, j.k);
+  if (bytes > scratch.planes_bytes) {
+    for (int i = 0; i < count; ++i) {
+      const hipError_t e = launch_matmul_planes(jobs + i, 1, gelu, scratch, st);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
+  SplitArgs s{};
+  PlanesArgs p{};
+  s.k = p.k = j.k;
+  s.planes = static_cast<uint16_t*>(scratch.planes);
+  p.x = s.planes;
+  p.row0 = j.row0;
+  p.row1 = j.row1;
+  p.count = count;
+  s.count = count + 1;
+  const int xtiles = (rows + 31) / 32;
+  s.src[0] = j.a;
+  s.row0[0] = j.row0;
+  s.rows[0] = rows;
+  s.tiles[0] = xtiles;
+  p.w = s.planes + static_cast<size_t>(xtiles) * (j.k / 16) * kDenseStep;
+  int wtiles = 0;
+  for (int i = 0; i < count; ++i) {
+    s.src[i + 1] = jobs[i].bt;
+    s.rows[i + 1] = jobs[i].cols;
+    s.tiles[i + 1] = (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles
+    p.set[i] = PlanesSet{jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
+    wtiles += s.tiles[i + 1];
+  }
+  split_dense<<<dim3(static_cast<unsigned>(xtiles + wtiles), (j.k + 63) / 64), 256, 0, st>>>(s);
+  // under 128 tiles the CUs are not full: both halves of K at once (656 x 384 outputs 8.5 us, 10.1 in
+  // turn; 656 x 1152, 198 tiles, 16.1 and 12.3)
+  if (static_cast<int64_t>((rows + 63) / 64) * (wtiles / 2) < 128)
+    run_planes<2>(p, gelu, st);
+  else
+    run_planes<1>(p, gelu, st);
+  return hipGetLastError();
+}
+
+hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& dense,
+                             hipStream_t st) {
+  if (j.row1 <= j.row0 || j.cols <= 0) return hipSuccess;
+  if (j.k <= 0) return hipErrorInvalidValue;
+  if (matmul_on_planes(j, dense)) return launch_matmul_planes(&j, 1, gelu, dense, st);
+  const float *a = j.a, *bt = j.bt, *bias = j.bias;
+  float *out = j.out, *scratch = dense.sums;
+  const int row0 = j.row0, row1 = j.row1, cols = j.cols, k = j.k;
+  const size_t scratch_floats = dense.sums_floats;
   const int rows = row1 - row0, chunks = (k + 63) / 64;
   // large shapes on bf16 MFMA (split x3), with 16-byte rows: at least two tiles per CU, or K
   // split over workgroups into partial sums (about 768 workgroups) from 64 tiles

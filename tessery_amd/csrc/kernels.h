@@ -136,11 +136,27 @@ hipError_t launch_silu_gate_f32(float* gate, const float* up, uint32_t n, hipStr
 // for rows [row0, row1), any K and N (tessery matmul_f32 / matmul_bias_f32 families,
 // kernels.metal:306-322, 396-487); with gelu the stored value is gelu_f32 of it, bit-identical to
 // the projection followed by the gelu_f32 route.
-// With few output tiles (small batches) and a scratch buffer of scratch_floats floats, K is
-// split over workgroups and the partial sums are added in a fixed order by a second kernel.
-hipError_t launch_matmul_f32(const float* a, const float* bt, const float* bias, float* out,
-                             int row0, int row1, int cols, int k, bool gelu, float* scratch,
-                             size_t scratch_floats, hipStream_t st);
+struct DenseJob {
+  const float *a, *bt, *bias;
+  float* out;
+  int row0, row1, cols, k;
+};
+// sums: partial sums of split-K launches of the fp32 kernel. planes: the operands of the split-bf16
+// one (16-byte aligned).
+struct DenseScratch {
+  float* sums;
+  size_t sums_floats;
+  void* planes;
+  size_t planes_bytes;
+};
+hipError_t launch_matmul_f32(const DenseJob& job, bool gelu, const DenseScratch& scratch,
+                             hipStream_t st);
+// Whether launch_matmul_f32 runs the job on the split-bf16 kernel, whose results depend neither on
+// the rows of the launch nor on the projections beside it.
+bool matmul_on_planes(const DenseJob& job, const DenseScratch& scratch);
+// One to three such projections of the same rows of one a, with the bits of separate launches.
+hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
+                                const DenseScratch& scratch, hipStream_t st);
 // x[i] += bias[i % cols] (kernels.metal:376-379).
 hipError_t launch_add_bias_f32(float* x, const float* bias, uint32_t n, uint32_t cols,
                                hipStream_t st);

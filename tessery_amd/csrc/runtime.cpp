@@ -159,6 +159,7 @@ struct Runtime {
   uint64_t graph_launches = 0, graph_builds = 0;
   uint64_t fused_pairs = 0, fused_gated = 0;  // launch-time fusions (diagnostics)
   float* dense_scratch = nullptr;  // split-K partial sums of small-batch projections
+  void* dense_planes = nullptr;    // split operands of fp32 projections
   void* planes[2] = {};  // planes of the activations uint4 projections read, and of their output
   std::vector<Segment> segments;
   hipStream_t stream = nullptr;
@@ -568,9 +569,17 @@ bool is_linear4(Route r) {
 
 bool is_gated4(Route r) { return r == R_GATED4_16X32 || r == R_GATED4_8X32; }
 
+bool is_dense(Route r) {
+  return r == R_MATMUL || r == R_MATMUL_TILED || r == R_MATMUL_CHUNK32 || r == R_MATMUL_BIAS ||
+         r == R_MATMUL_BIAS_CHUNK32;
+}
+
 // Scratch of the split-K projection paths (dense and uint4), allocated once per runtime on first
 // use (its address never changes, so a captured graph keeps pointing at it).
 constexpr size_t kDenseScratchFloats = size_t{8} << 20;  // 32 MiB
+// Split operands of the dense projections: at most 512 tiles of 64 x 128 outputs (more run on
+// matmul_x3), which is 96 MiB where they are one column of tiles of K = 512.
+constexpr size_t kDensePlanesBytes = size_t{104} << 20;
 // Each of the two planes scratches: 1023 rows (more run on linear4_hilo) of 3072 inputs, Qwen3's
 // widest, in 18.4 MiB. Others go through it in row ranges.
 constexpr size_t kPlanesBytes = size_t{20} << 20;
@@ -597,6 +606,11 @@ bool prepare(Runtime* rt, Route r, const Params& p) {
       if (!rt->dense_scratch &&
           hipMalloc(&rt->dense_scratch, kDenseScratchFloats * sizeof(float)) != hipSuccess) {
         rt->dense_scratch = nullptr;
+        return false;
+      }
+      if (is_dense(r) && !rt->dense_planes &&
+          hipMalloc(&rt->dense_planes, kDensePlanesBytes) != hipSuccess) {
+        rt->dense_planes = nullptr;
         return false;
       }
       for (void*& p : rt->planes)
@@ -702,6 +716,26 @@ bool gated4_jobs(const Op& op, tessery::Linear4Job* jobs) {
   return true;
 }
 
+// The projection of a dense op (buffers a, bt, out [, bias]).
+bool dense_job(const Op& op, tessery::DenseJob* job) {
+  RowRange rr;
+  if (!is_dense(op.route) || !matmul_range(op.route, op.p, op.threads, op.group, &rr)) return false;
+  const bool bias = op.route == R_MATMUL_BIAS || op.route == R_MATMUL_BIAS_CHUNK32;
+  *job = {static_cast<const float*>(op.ptr[0]),
+          static_cast<const float*>(op.ptr[1]),
+          bias ? static_cast<const float*>(op.ptr[3]) : nullptr,
+          static_cast<float*>(op.ptr[2]),
+          static_cast<int>(rr.r0),
+          static_cast<int>(rr.r1),
+          static_cast<int>(op.p.cols),
+          static_cast<int>(op.p.k)};
+  return true;
+}
+
+tessery::DenseScratch dense_scratch(Runtime* rt) {
+  return {rt->dense_scratch, kDenseScratchFloats, rt->dense_planes, kDensePlanesBytes};
+}
+
 // `in` is the planes scratch `slot`, `out` the other one.
 tessery::PlanesScratch planes_scratch(Runtime* rt, int slot) {
   return {rt->planes[slot], rt->planes[1 - slot], kPlanesBytes};
@@ -776,14 +810,9 @@ hipError_t launch(Runtime* rt, const Op& op, void* planes) {
     case R_MATMUL_CHUNK32:
     case R_MATMUL_BIAS:
     case R_MATMUL_BIAS_CHUNK32: {
-      RowRange rr;
-      if (!matmul_range(op.route, p, op.threads, op.group, &rr)) return hipErrorInvalidValue;
-      const bool bias = op.route == R_MATMUL_BIAS || op.route == R_MATMUL_BIAS_CHUNK32;
-      return tessery::launch_matmul_f32(
-          static_cast<const float*>(op.ptr[0]), static_cast<const float*>(op.ptr[1]),
-          bias ? static_cast<const float*>(op.ptr[3]) : nullptr, static_cast<float*>(op.ptr[2]),
-          static_cast<int>(rr.r0), static_cast<int>(rr.r1), static_cast<int>(p.cols),
-          static_cast<int>(p.k), false, rt->dense_scratch, kDenseScratchFloats, st);
+      tessery::DenseJob job;
+      if (!dense_job(op, &job)) return hipErrorInvalidValue;
+      return tessery::launch_matmul_f32(job, false, dense_scratch(rt), st);
     }
     case R_ADD_BIAS:
       return tessery::launch_add_bias_f32(static_cast<float*>(op.ptr[0]),
@@ -894,6 +923,7 @@ void mi_destroy(void* runtime) {
     (void)hipFree(kv.second.sin);
   }
   if (rt->dense_scratch) (void)hipFree(rt->dense_scratch);
+  if (rt->dense_planes) (void)hipFree(rt->dense_planes);
   for (void* p : rt->planes)
     if (p) (void)hipFree(p);
   release_profile_events(rt);
@@ -989,8 +1019,6 @@ hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
 
 // Pairs of queued launches that one kernel runs with the same bits (the second op of a pair is
 // then not launched on its own):
-//   a projection covering every row of its output, then gelu_f32 over exactly that output
-//     -> the projection with the GELU epilogue;
 //   add(a, b -> a), then layer_norm(a -> a) over the same rows
 //     -> one pass that adds and normalizes in place;
 //   add(a, b -> a), then rms_norm(a -> y) -> one pass (add_rms_norm_f32);
@@ -1006,22 +1034,6 @@ hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
 hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes) {
   hipStream_t st = rt->stream;
   if (is_linear4(a.route)) return launch_fused_dual(rt, a, b, false);
-  const bool projection = a.route == R_MATMUL || a.route == R_MATMUL_TILED ||
-                          a.route == R_MATMUL_CHUNK32 || a.route == R_MATMUL_BIAS ||
-                          a.route == R_MATMUL_BIAS_CHUNK32;
-  if (projection && b.route == R_GELU && b.ptr[0] == a.ptr[2]) {
-    RowRange rr;
-    if (!matmul_range(a.route, a.p, a.threads, a.group, &rr)) return hipErrorNotReady;
-    if (rr.r0 != 0 || rr.r1 != a.p.rows ||
-        static_cast<uint64_t>(b.p.n) != static_cast<uint64_t>(a.p.rows) * a.p.cols)
-      return hipErrorNotReady;
-    const bool bias = a.route == R_MATMUL_BIAS || a.route == R_MATMUL_BIAS_CHUNK32;
-    return tessery::launch_matmul_f32(
-        static_cast<const float*>(a.ptr[0]), static_cast<const float*>(a.ptr[1]),
-        bias ? static_cast<const float*>(a.ptr[3]) : nullptr, static_cast<float*>(a.ptr[2]),
-        0, static_cast<int>(rr.r1), static_cast<int>(a.p.cols), static_cast<int>(a.p.k), true,
-        rt->dense_scratch, kDenseScratchFloats, st);
-  }
   if (a.route == R_ADD && b.route == R_LAYER_NORM && a.ptr[2] == a.ptr[0] &&
       b.ptr[0] == a.ptr[0] && b.ptr[3] == a.ptr[0] && a.ptr[1] != a.ptr[0] &&
       static_cast<uint64_t>(a.p.n) == (b.threads / 32) * b.p.cols) {
@@ -1253,6 +1265,78 @@ bool find_projection(Runtime* rt, size_t first, size_t last, Projection* p) {
   return true;
 }
 
+// A dense launch over ops [first, end).
+struct DenseProjection {
+  tessery::DenseJob jobs[3];
+  int count;
+  bool gelu;
+  size_t end;
+};
+
+// One projection's launches over consecutive row ranges (as the planners partition its rows) from op
+// `first`, joined; false when it is no dense projection.
+bool dense_run(Runtime* rt, size_t first, size_t last, tessery::DenseJob* job, size_t* end) {
+  if (!dense_job(rt->ops[first], job)) return false;
+  *end = first + 1;
+  const Op& a = rt->ops[first];
+  for (uint32_t i = 0; i < a.count; ++i)
+    if (i != 2 && a.ptr[i] == a.ptr[2]) return true;
+  for (; *end < last; ++*end) {
+    const Op& b = rt->ops[*end];
+    tessery::DenseJob next;
+    if (!dense_job(b, &next) || b.p.rows != a.p.rows || next.a != job->a || next.bt != job->bt ||
+        next.bias != job->bias || next.out != job->out || next.cols != job->cols ||
+        next.k != job->k || next.row0 != job->row1)
+      break;
+    job->row1 = next.row1;
+  }
+  return true;
+}
+
+// The launch that starts at op `first`: one projection, with the gelu_f32 over its whole output that
+// follows, or up to three of the same rows of one input (q, k and v) on matmul_planes. False: op
+// `first` is no dense projection.
+bool find_dense(Runtime* rt, size_t first, size_t last, DenseProjection* p) {
+  if (!is_dense(rt->ops[first].route) || !dense_run(rt, first, last, &p->jobs[0], &p->end))
+    return false;
+  p->count = 1;
+  p->gelu = false;
+  const tessery::DenseJob& lead = p->jobs[0];
+  if (p->end < last) {
+    const Op& b = rt->ops[p->end];
+    if (b.route == R_GELU && b.ptr[0] == lead.out && lead.row0 == 0 &&
+        static_cast<uint64_t>(lead.row1) == rt->ops[first].p.rows &&
+        static_cast<uint64_t>(b.p.n) ==
+            static_cast<uint64_t>(lead.row1) * static_cast<uint64_t>(lead.cols)) {
+      p->gelu = true;
+      ++p->end;
+      return true;
+    }
+  }
+  const tessery::DenseScratch scratch = dense_scratch(rt);
+  while (p->count < 3 && p->end < last && tessery::matmul_on_planes(lead, scratch)) {
+    tessery::DenseJob j;
+    size_t end;
+    if (!dense_run(rt, p->end, last, &j, &end) || !tessery::matmul_on_planes(j, scratch) ||
+        j.a != lead.a || j.k != lead.k ||
+        j.row0 != lead.row0 || j.row1 != lead.row1 || j.out == j.a)
+      break;
+    // no output is an input or output of another projection of the launch
+    bool apart = true;
+    for (int i = 0; i < p->count; ++i) {
+      const tessery::DenseJob& o = p->jobs[i];
+      apart = apart && o.out != j.a && o.out != j.bt && o.out != j.bias && o.out != j.out &&
+              j.out != o.bt && j.out != o.bias;
+    }
+    // its own gelu_f32 runs with it
+    const bool gelu = end < last && rt->ops[end].route == R_GELU && rt->ops[end].ptr[0] == j.out;
+    if (!apart || gelu) break;
+    p->jobs[p->count++] = j;
+    p->end = end;
+  }
+  return true;
+}
+
 // What the launch before left for the next one: the planes of x [rows, k], in a planes scratch.
 struct Ready {
   const void* x = nullptr;
@@ -1298,6 +1382,16 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
       pass->ready = {j.out, static_cast<uint64_t>(j.row1), static_cast<uint64_t>(j.cols), 1 - slot};
     return tessery::launch_linear4_rows(p.jobs, p.count, p.gated, planes_scratch(rt, slot),
                                         prepared, keep, rt->stream);
+  }
+  DenseProjection d;
+  if (find_dense(rt, first, last, &d)) {
+    *taken = d.end - first;
+    const hipError_t e =
+        d.count > 1
+            ? tessery::launch_matmul_planes(d.jobs, d.count, false, dense_scratch(rt), rt->stream)
+            : tessery::launch_matmul_f32(d.jobs[0], d.gelu, dense_scratch(rt), rt->stream);
+    pass->fused.pairs += d.gelu && e == hipSuccess;
+    return e;
   }
   const hipError_t gated =
       first + 2 < last ? launch_fused_gated(rt, op, rt->ops[first + 1], rt->ops[first + 2])

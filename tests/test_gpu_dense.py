@@ -395,3 +395,66 @@ def test_plan_replay_graphs_match_eager(monkeypatch, graphs):
         np.testing.assert_array_equal(out, outs[0])
     np.testing.assert_allclose(outs[0], ref.layer(x, lengths, w, heads=heads, eps=eps), atol=5e-5,
                                rtol=5e-5)
+
+
+# Rows and columns at the edges of the 64 x 64 tiles, under and over 128 of them (both halves of K at
+# once, or in turn), K of 1, 2, 3, 5, 12 and 16 chunks (empty and uneven halves); then, past K = 512,
+# split K at few tiles (from 8 chunks) and the shapes that stay on the fp32 kernel.
+@pytest.mark.parametrize("rows,cols,k", [(1, 1, 32), (31, 33, 64), (64, 64, 96), (65, 129, 160),
+                                         (33, 384, 384), (543, 1152, 384), (1000, 384, 384),
+                                         (129, 4160, 512), (16, 128, 544), (65, 384, 1536),
+                                         (543, 384, 1536), (1, 256, 1568), (20, 100, 1536)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
+    """Within 2e-6 of sum_k |x| |w| of float64 (fp32 sums of exact products), the rows after the range
+    untouched; row magnitudes spread over 2^-30 .. 2^30."""
+    rng = np.random.default_rng(rows + 7 * cols + k)
+    x = rng.normal(size=(rows, k)).astype(np.float32)
+    x *= np.exp2(rng.integers(-30, 31, rows)).astype(np.float32)[:, None]
+    w = rng.normal(size=(cols, k)).astype(np.float32)
+    b = rng.normal(size=cols).astype(np.float32)
+    bufs = [runtime.upload(a) for a in (x, w, np.full((rows + 1, cols), np.nan, np.float32), b)]
+    try:
+        with runtime.command():
+            name = "matmul_bias_f32" if bias else "matmul_f32"
+            runtime._dispatch(name, bufs if bias else bufs[:3], threads=(rows + 3) // 4 * cols * 32,
+                              group_size=32, rows=rows, cols=cols, k=k)
+        got = runtime.read(bufs[2], (rows + 1, cols))
+    finally:
+        for buf in bufs:
+            buf.close()
+    assert np.isnan(got[rows:]).all()
+    xd, wd = x.astype(np.float64), w.astype(np.float64)
+    err = np.abs(got[:rows] - (xd @ wd.T + (b if bias else 0)))
+    bound = 2e-6 * (np.abs(xd) @ np.abs(wd).T + (np.abs(b) if bias else 0))
+    assert np.all(err <= bound), float((err / bound).max())
+
+
+@pytest.mark.parametrize("rows", [7, 41, 543, 656])
+def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
+    """Three projections of one input queued in one command run as one launch, their row ranges
+    joined; each output holds the bits of a command of its own."""
+    rng = np.random.default_rng(rows)
+    x = rng.normal(size=(rows, 384)).astype(np.float32)
+    sets = [(rng.normal(size=(384, 384)).astype(np.float32), rng.normal(size=384).astype(np.float32))
+            for _ in range(3)]
+    results = []
+    for separate in (False, True):
+        xb = runtime.upload(x)
+        bufs = [(runtime.upload(w), runtime.upload(b), runtime.buffer(x.nbytes)) for w, b in sets]
+        steps = [lambda w=w, b=b, o=o: runtime._matmul_bias_f32([xb, w, o, b], rows=rows, cols=384,
+                                                                k=384) for w, b, o in bufs]
+        if separate:
+            for step in steps:
+                with runtime.command():
+                    step()
+        else:
+            with runtime.command():
+                for step in steps:
+                    step()
+        results.append([runtime.read(o, x.shape) for _, _, o in bufs])
+        for buf in [xb, *(b for group in bufs for b in group)]:
+            buf.close()
+    for (w, b), together, alone in zip(sets, *results):
+        np.testing.assert_array_equal(together, alone)
+        np.testing.assert_allclose(together, ref.linear(x, w, b), atol=2e-4, rtol=5e-5)
