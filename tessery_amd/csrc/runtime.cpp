@@ -191,6 +191,7 @@ struct PlanOp {
 // Launch-time fusions made while queuing a range of ops (see launch_range).
 struct FusionCount {
   uint64_t pairs = 0, gated = 0;
+  size_t launches = 0;  // steps of launch_next (a few are two or three kernels)
 };
 
 // An instantiated HIP graph of a plan's launches for one binding of its slots, with the fusions
@@ -206,9 +207,15 @@ struct Plan {
   std::vector<uint64_t> sizes;
   std::vector<PlanOp> ops;
   std::vector<CachedGraph> graphs;  // most recently used last, at most kPlanGraphs
+  bool direct = false;              // too short for a graph (see kGraphLaunches)
 };
 
 constexpr size_t kPlanGraphs = 4;
+// A plan of fewer launches is replayed launch by launch: starting a graph costs more than its
+// launches save. Measured per replay, as a graph and directly: 5 launches of short attention 55.9 and
+// 50.0 us, of a 32 x 464 batch 242.5 and 234.5, 4 of projection and attention 162 and 155; but 10 of a
+// decoder layer 87.8 and 96.5, 9 (13 kernels) of an encoder layer 122.2 and 125.4.
+constexpr size_t kGraphLaunches = 6;
 
 inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
@@ -1433,6 +1440,7 @@ hipError_t launch_range(Runtime* rt, size_t first, size_t last, FusionCount* fc)
   for (size_t i = first, taken = 0; i < last; i += taken) {
     const hipError_t e = launch_next(rt, i, last, &taken, &pass);
     if (e != hipSuccess) return e;
+    ++fc->launches;
   }
   fc->pairs += pass.fused.pairs;
   fc->gated += pass.fused.gated;
@@ -1447,9 +1455,10 @@ void count_fusions(Runtime* rt, const FusionCount& fc) {
 // A plan replay as one graph launch: the graph of this plan for this binding is instantiated the
 // first time (stream capture of launch_range, which records the same kernels with the same
 // arguments) and reused afterwards. Captured launches do not run, so on any capture error the
-// caller launches the segment directly. hipErrorNotReady: graphs are off for this runtime.
+// caller launches the segment directly. hipErrorNotReady: graphs are off for this runtime, or the
+// plan is a short one.
 hipError_t launch_segment_graph(Runtime* rt, const Segment& seg) {
-  if (!rt->graphs) return hipErrorNotReady;
+  if (!rt->graphs || seg.plan->direct) return hipErrorNotReady;
   auto& cache = seg.plan->graphs;
   for (size_t j = 0; j < cache.size(); ++j)
     if (cache[j].key == seg.key) {
@@ -1470,6 +1479,11 @@ hipError_t launch_segment_graph(Runtime* rt, const Segment& seg) {
   if (recorded != hipSuccess || ended != hipSuccess || !graph) {
     if (graph) (void)hipGraphDestroy(graph);
     (void)hipGetLastError();
+    return hipErrorNotReady;
+  }
+  if (fc.launches < kGraphLaunches) {
+    seg.plan->direct = true;
+    (void)hipGraphDestroy(graph);
     return hipErrorNotReady;
   }
   hipGraphExec_t exec = nullptr;
