@@ -27,6 +27,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "lds_dma.h"
+#include "planes.h"
 
 #include <math.h>
 
@@ -1542,6 +1543,7 @@ struct X3Args {
   float scale_log2, scale_log2_lo;  // scale * log2(e) as the sum of two floats
   int bidi;
   F16Shape shp;
+  Planes planes;  // where the output also goes for the projection after it (terms null: nowhere)
 };
 
 // fp32 attention on bf16 MFMA, the split products summed by size: one accumulator for the leading
@@ -1818,6 +1820,32 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
 #pragma unroll
   for (int i = 0; i < NI; ++i)
     val[i] = *reinterpret_cast<const uint4v*>(ob + (i * RPI + lo) * RS + 16 * (lane % OCH));
+  if (a.planes.terms && g.active) {
+    // Lane = row of the wave block + 16 (chunk % 4): a chunk's rows, mostly one position apart, make
+    // contiguous pieces of up to 128 bytes (written from the output's own lanes, 8 bytes each,
+    // they cost 4 x 77 tokens 3.7 us of 13.2). The sums add as in store_planes4.
+    const int idx = lane & 15, pos = g.p0 + (idx >> g.hsh), head = g.head0 + (idx & hmask);
+    const int row = static_cast<int>(g.b) * S + pos, prow = row % kPlaneRows;
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) {
+      const int chunk = (lane >> 4) + 4 * i, col = head * D + 8 * chunk;
+      const floatx4 u = *reinterpret_cast<const floatx4*>(ob + idx * RS + 32 * chunk);
+      const floatx4 v = *reinterpret_cast<const floatx4*>(ob + idx * RS + 32 * chunk + 16);
+      uint4v t[3];
+      split3x8(u, v, t[0], t[1], t[2]);
+      float sum = ((u[0] + u[1]) + (u[2] + u[3])) + ((v[0] + v[1]) + (v[2] + v[3]));
+      sum += __shfl_xor(sum, 16);
+      sum += __shfl_xor(sum, 32);
+      if (pos >= S) continue;
+      const size_t at = static_cast<size_t>(row / kPlaneRows) * (H * D >> 6) + (col >> 6);
+      const int plane_lane = prow + 32 * ((col >> 5) & 1);
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        *reinterpret_cast<uint4v*>(a.planes.terms + at * kPlaneGroup + k * kPlaneTerm +
+                                   ((col >> 3) & 3) * 512 + plane_lane * 8) = t[k];
+      if (lane < 16) a.planes.sums[at * kPlaneSums + plane_lane] = sum;
+    }
+  }
   if (g.active) {
     const int room = S - g.p0;
     if ((16 >> g.hsh) <= room) {
@@ -1883,6 +1911,15 @@ bool attention_scalar_fits(uint64_t B, uint64_t S, uint64_t H) {
 
 static bool attention_f32x3_fits(int B, int S, int H, int KV, int D);
 
+// Rows of fewer keys than this stay on attn_scalar (see launch_attention_scalar).
+constexpr int kX3MinKeys = 16;
+
+bool attention_leaves_planes(const AttnArgs& a, bool scalar) {
+  return (!scalar || a.S >= kX3MinKeys) && !a.in_f16 && !a.out_f16 && a.H * a.D % 64 == 0 &&
+         attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D) &&
+         attention_f32_fits(a.B, a.S, a.H, a.KV);
+}
+
 hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   if (!attention_scalar_fits(a.B, a.S, a.H)) return hipErrorInvalidValue;
   const unsigned grid = static_cast<unsigned>(a.B * a.S * a.H);
@@ -1891,7 +1928,7 @@ hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   // attn_scalar's keys are a serial chain of wave reductions, about 1.25 us each whatever the
   // batch (24 tokens of 16 heads 30.9 against 8.0 us, 16 x 41 tokens of 12 heads 39.6 against
   // 9.1 us per launch). Under 16 keys the chain is as short as the tile's latency.
-  if (a.S >= 16 && !a.in_f16 && !a.out_f16 &&
+  if (a.S >= kX3MinKeys && !a.in_f16 && !a.out_f16 &&
       attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D) &&
       attention_f32_fits(a.B, a.S, a.H, a.KV))
     return launch_attention_f32(a, st);
@@ -1981,6 +2018,7 @@ hipError_t launch_attention_f32(const AttnArgs& a, hipStream_t st) {
     x.scale_log2_lo = static_cast<float>(c - static_cast<double>(x.scale_log2));
     x.bidi = a.bidi;
     x.shp = f16_shape(a.B, a.S, a.H, a.KV);
+    if (a.planes) x.planes = planes_at(a.planes, a.B * a.S, a.H * a.D);
     const dim3 grid = sched_grid(a.B, a.KV, (x.shp.nwb + 3) / 4);
     switch (a.D) {
       case 32:

@@ -36,6 +36,9 @@ struct AttnArgs {
   const float* pro_cos;       // [S, D/2]
   const float* pro_sin;
   float pro_eps;
+  // fp32 attention that attention_leaves_planes takes: where the output also goes as planes.h's
+  // terms of rows [B S, H D]; null when unused.
+  void* planes;
 };
 
 // Shape limits of the attention launchers (grid sizes, 32-bit offsets, exact reciprocal
@@ -45,6 +48,10 @@ bool attention_f32_fits(int B, int S, int H, int KV);
 bool attention_f16_fits(int B, int S, int H, int KV, int D);
 // Whether a fused-route launch of this shape can carry another layer's k prologue (AttnArgs pro_*).
 bool attention_f16_carries_prologue(int B, int S, int H, int KV, int D);
+
+// Whether launch_attention_f32, or launch_attention_scalar (`scalar`), can leave its output as planes
+// too: attn_f32x3 runs it, and rows of whole 64-input groups.
+bool attention_leaves_planes(const AttnArgs& a, bool scalar);
 
 hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st);
 hipError_t launch_attention_f32(const AttnArgs& a, hipStream_t st);
@@ -67,11 +74,17 @@ hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, 
                                    int rows, int cols, float eps, void* planes,
                                    hipStream_t st);
 // launch_rms_norm_f32 in place (x == out) followed by launch_rope_f32 on the same rows, as one
-// kernel with the same bits; hipErrorNotReady when the shape is not covered (8 | dim <= 256, x
-// 16-byte aligned) and the two launches must run instead.
-hipError_t launch_rms_norm_rope_f32(float* x, const uint16_t* w, const float* cos_tab,
-                                   const float* sin_tab, int rows, int dim, float eps, int heads,
-                                   int seq, hipStream_t st);
+// kernel with the same bits, over one or two sets of rows (q, then k) of one dim and seq;
+// hipErrorNotReady when the shape is not covered (8 | dim <= 256, x 16-byte aligned) and the
+// separate launches must run instead.
+struct NormRopeRows {
+  float* x;
+  const uint16_t* w;
+  int rows, heads;
+  float eps;
+};
+hipError_t launch_rms_norm_rope_f32(const NormRopeRows* sets, int count, const float* cos_tab,
+                                   const float* sin_tab, int dim, int seq, hipStream_t st);
 // Fused per-head RMSNorm + RoPE on fp16 rows [B,S,heads,D] -> fp16 rows, rows with
 // position >= lengths[b] skipped (they are padding that attention never reads). With split the
 // output holds two planes: y[0 : rows*D] = fp16(r), y[rows*D : 2*rows*D] = fp16(r - fp16(r)).

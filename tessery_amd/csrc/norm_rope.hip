@@ -92,13 +92,19 @@ __global__ __launch_bounds__(256) void rope_f32(float* x, const float* __restric
 // pieces for the rotation. PAIR (dim <= 128): two rows per wavefront, one per 32-lane half; the
 // half-wave butterfly gives the bits of wave_sum with the other half zero (its first step adds
 // exact zeros).
+// Workgroups from blocks0 on take the second set (the k rows after the q rows, one launch for both).
 template <bool PAIR>
-__global__ __launch_bounds__(256) void rms_norm_rope_f32(float* x, const uint16_t* __restrict__ w,
+__global__ __launch_bounds__(256) void rms_norm_rope_f32(NormRopeRows set0, NormRopeRows set1,
+                                                         unsigned blocks0,
                                                          const float* __restrict__ cos_tab,
-                                                         const float* __restrict__ sin_tab,
-                                                         int rows, int dim, float eps, int heads,
+                                                         const float* __restrict__ sin_tab, int dim,
                                                          int seq) {
-  const int slot = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const bool second = blockIdx.x >= blocks0;
+  float* const x = second ? set1.x : set0.x;
+  const uint16_t* const w = second ? set1.w : set0.w;
+  const int rows = second ? set1.rows : set0.rows, heads = second ? set1.heads : set0.heads;
+  const float eps = second ? set1.eps : set0.eps;
+  const int slot = static_cast<int>(blockIdx.x - (second ? blocks0 : 0)) * 4 + (threadIdx.x >> 6);
   const int lane = PAIR ? (threadIdx.x & 31) : (threadIdx.x & 63);
   const int row = PAIR ? 2 * slot + ((threadIdx.x >> 5) & 1) : slot;
   const bool live = row < rows;
@@ -268,21 +274,24 @@ hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, 
   return hipGetLastError();
 }
 
-hipError_t launch_rms_norm_rope_f32(float* x, const uint16_t* w, const float* cos_tab,
-                                   const float* sin_tab, int rows, int dim, float eps, int heads,
-                                   int seq, hipStream_t st) {
-  if (rows <= 0) return hipSuccess;
-  if (dim <= 0 || dim % 8 || dim > 256 || heads <= 0 || seq <= 0 ||
-      (reinterpret_cast<uintptr_t>(x) & 15))
+hipError_t launch_rms_norm_rope_f32(const NormRopeRows* sets, int count, const float* cos_tab,
+                                   const float* sin_tab, int dim, int seq, hipStream_t st) {
+  if (count < 1 || count > 2 || dim <= 0 || dim % 8 || dim > 256 || seq <= 0)
     return hipErrorNotReady;  // the separate kernels run instead
-  if (dim <= 128) {
-    const int pairs = (rows + 1) / 2;
-    rms_norm_rope_f32<true><<<(pairs + 3) / 4, 256, 0, st>>>(x, w, cos_tab, sin_tab, rows, dim,
-                                                             eps, heads, seq);
-  } else {
-    rms_norm_rope_f32<false><<<(rows + 3) / 4, 256, 0, st>>>(x, w, cos_tab, sin_tab, rows, dim,
-                                                             eps, heads, seq);
+  unsigned blocks[2] = {};
+  for (int i = 0; i < count; ++i) {
+    if (sets[i].rows <= 0 || sets[i].heads <= 0 || (reinterpret_cast<uintptr_t>(sets[i].x) & 15))
+      return hipErrorNotReady;
+    const int slots = dim <= 128 ? (sets[i].rows + 1) / 2 : sets[i].rows;
+    blocks[i] = static_cast<unsigned>((slots + 3) / 4);
   }
+  const NormRopeRows& last = sets[count - 1];
+  if (dim <= 128)
+    rms_norm_rope_f32<true><<<blocks[0] + blocks[1], 256, 0, st>>>(sets[0], last, blocks[0], cos_tab,
+                                                                   sin_tab, dim, seq);
+  else
+    rms_norm_rope_f32<false><<<blocks[0] + blocks[1], 256, 0, st>>>(sets[0], last, blocks[0],
+                                                                    cos_tab, sin_tab, dim, seq);
   return hipGetLastError();
 }
 

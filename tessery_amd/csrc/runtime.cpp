@@ -748,7 +748,7 @@ tessery::PlanesScratch planes_scratch(Runtime* rt, int slot) {
   return {rt->planes[slot], rt->planes[1 - slot], kPlanesBytes};
 }
 
-// planes: where a rms_norm also leaves its output as planes (null: nowhere).
+// planes: where a rms_norm or an attention also leaves its output as planes (null: nowhere).
 hipError_t launch(Runtime* rt, const Op& op, void* planes) {
   hipStream_t st = rt->stream;
   const Params& p = op.p;
@@ -762,6 +762,7 @@ hipError_t launch(Runtime* rt, const Op& op, void* planes) {
     case R_ATTENTION_F16_NORM_ROPE: {
       tessery::AttnArgs a{};
       if (!attention_args(rt, op, &a)) return hipErrorInvalidValue;
+      a.planes = planes;
       if (op.route == R_ATTENTION || op.route == R_ATTENTION_F16_SCALAR)
         return tessery::launch_attention_scalar(a, st);
       if (op.route == R_ATTENTION_F16 || op.route == R_ATTENTION_F16_NORM_ROPE)
@@ -1024,6 +1025,33 @@ int mi_dispatch(void* runtime, const char* name, void** buffers, uint32_t count,
 
 hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
 
+// The rows of an in-place rms_norm whose rope follows.
+bool norm_rope_rows(const Op& a, const Op& b, tessery::NormRopeRows* rows) {
+  if (a.route != R_RMS_NORM || b.route != R_ROPE || a.ptr[2] != a.ptr[0] || b.ptr[0] != a.ptr[0] ||
+      b.p.dim != a.p.cols || static_cast<uint64_t>(b.p.n) != (a.threads / 32) * (a.p.cols / 2))
+    return false;
+  *rows = {static_cast<float*>(a.ptr[0]), static_cast<const uint16_t*>(a.ptr[1]),
+           static_cast<int>(a.threads / 32), static_cast<int>(b.p.heads), a.p.eps};
+  return true;
+}
+
+// Two such pairs over different buffers of one dim, seq and theta (a layer's q, then k) as one
+// launch of ops first .. first + 3; hipErrorNotReady when they are not that.
+hipError_t launch_norm_rope_pairs(Runtime* rt, size_t first, size_t last) {
+  tessery::NormRopeRows rows[2];
+  if (first + 3 >= last) return hipErrorNotReady;
+  const Op *a = &rt->ops[first], *b = a + 1, *c = a + 2, *d = a + 3;
+  if (!norm_rope_rows(*a, *b, &rows[0]) || !norm_rope_rows(*c, *d, &rows[1]) ||
+      a->p.cols != c->p.cols || b->p.seq != d->p.seq ||
+      float_bits(b->p.theta) != float_bits(d->p.theta) || a->ptr[0] == c->ptr[0] ||
+      a->ptr[1] == c->ptr[0] || c->ptr[1] == a->ptr[0])
+    return hipErrorNotReady;
+  const RopeTable* t = rope_of(rt, b->p);
+  if (!t) return hipErrorNotReady;
+  return tessery::launch_rms_norm_rope_f32(rows, 2, t->cos, t->sin, static_cast<int>(a->p.cols),
+                                           static_cast<int>(b->p.seq), rt->stream);
+}
+
 // Pairs of queued launches that one kernel runs with the same bits (the second op of a pair is
 // then not launched on its own):
 //   add(a, b -> a), then layer_norm(a -> a) over the same rows
@@ -1104,15 +1132,12 @@ hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes
     args.pro_eps = b.p.eps;
     return tessery::launch_attention_f16(args, st);
   }
-  if (a.route == R_RMS_NORM && b.route == R_ROPE && a.ptr[2] == a.ptr[0] &&
-      b.ptr[0] == a.ptr[0] && b.p.dim == a.p.cols &&
-      static_cast<uint64_t>(b.p.n) == (a.threads / 32) * (a.p.cols / 2)) {
+  tessery::NormRopeRows rows;
+  if (norm_rope_rows(a, b, &rows)) {
     const RopeTable* t = rope_of(rt, b.p);
     if (!t) return hipErrorNotReady;
-    return tessery::launch_rms_norm_rope_f32(
-        static_cast<float*>(a.ptr[0]), static_cast<const uint16_t*>(a.ptr[1]), t->cos, t->sin,
-        static_cast<int>(a.threads / 32), static_cast<int>(a.p.cols), a.p.eps,
-        static_cast<int>(b.p.heads), static_cast<int>(b.p.seq), st);
+    return tessery::launch_rms_norm_rope_f32(&rows, 1, t->cos, t->sin, static_cast<int>(a.p.cols),
+                                             static_cast<int>(b.p.seq), st);
   }
   return hipErrorNotReady;
 }
@@ -1408,6 +1433,12 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
     *taken = 3;
     return gated;
   }
+  const hipError_t pairs = launch_norm_rope_pairs(rt, first, last);
+  if (pairs != hipErrorNotReady) {
+    if (pairs == hipSuccess) pass->fused.pairs += 2;
+    *taken = 4;
+    return pairs;
+  }
   // the planes of a rms_norm (alone, or after the add it runs with) that projections read
   auto norm_ready = [&](size_t at) {
     const Op& n = rt->ops[at];
@@ -1429,6 +1460,13 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
   }
   *taken = 1;
   pass->ready = norm_ready(first);
+  tessery::AttnArgs at{};
+  if (attention_args(rt, op, &at) && tessery::attention_leaves_planes(at, op.route == R_ATTENTION)) {
+    const uint64_t rows = static_cast<uint64_t>(at.B) * static_cast<uint64_t>(at.S);
+    const uint64_t width = static_cast<uint64_t>(at.H) * static_cast<uint64_t>(at.D);
+    if (reads_planes(rt, first + 1, last, at.out, rows, width))
+      pass->ready = Ready{at.out, rows, width, 0};
+  }
   return launch(rt, op, pass->ready.x ? rt->planes[pass->ready.slot] : nullptr);
 }
 

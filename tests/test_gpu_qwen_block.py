@@ -71,3 +71,53 @@ def test_qkv4_norm_rope_attention_16x256(runtime):
     assert err <= FUSED_F32_MAX, err
     end_to_end = float(np.max(np.abs(got.astype(np.float64) - chain(*exact))))
     print(f"attention stage max-abs {err:.3e}; against the all-float64 chain {end_to_end:.3e}")
+
+
+@pytest.mark.parametrize("batch,seq,heads,kv,dim", [(1, 24, 16, 8, 128), (4, 77, 16, 8, 128),
+                                                    (2, 17, 4, 4, 64), (3, 33, 6, 2, 32),
+                                                    (2, 15, 4, 2, 128), (1, 64, 3, 1, 128)])
+def test_norms_attention_and_projection_in_one_command_keep_their_bits(runtime, batch, seq, heads,
+                                                                       kv, dim):
+    """q and k RMSNorm + RoPE (one launch for both), attention and the projection of its output (on
+    activations the attention kernel split) queued in one command hold the bits of a command each;
+    rows of fewer than 16 keys and head counts that do not fill a wavefront's 16 rows included."""
+    rng = np.random.default_rng(seq * 7 + dim)
+    tokens, width, cols = batch * seq, heads * dim, 96
+    q, k, v = [rng.normal(size=(tokens, h * dim)).astype(np.float32) for h in (heads, kv, kv)]
+    lengths = rng.integers(1, seq + 1, size=batch).astype(np.uint32)
+    gammas = [workloads.bf16_words(rng.uniform(0.5, 1.5, dim)) for _ in range(2)]
+    projection = [ref_quant4.pack(rng.integers(0, 16, size=(cols, width), dtype=np.uint32)),
+                  workloads.bf16_words(rng.uniform(0.01, 0.2, size=(cols, width // 64))),
+                  workloads.bf16_words(rng.uniform(-1, 0.1, size=(cols, width // 64)))] if width % 64 == 0 else None
+    results = []
+    for separate in (False, True):
+        bufs = [runtime.upload(a) for a in (q, k, v, lengths, *gammas, *(projection or []))]
+        att, out = runtime.buffer(tokens * width * 4), runtime.buffer(tokens * cols * 4)
+        steps = []
+        for buf, gamma, h in ((bufs[0], bufs[4], heads), (bufs[1], bufs[5], kv)):
+            steps.append(lambda buf=buf, gamma=gamma, h=h: runtime._dispatch(
+                "rms_norm", [buf, gamma, buf], threads=tokens * h * 32, group_size=32, cols=dim,
+                eps=1e-6))
+            steps.append(lambda buf=buf, h=h: runtime._dispatch(
+                "rope", [buf], threads=tokens * h * dim // 2, n=tokens * h * dim // 2, heads=h,
+                seq=seq, dim=dim, theta=1e6))
+        steps.append(lambda: runtime._attention([*bufs[:4], att], tokens=tokens, seq=seq,
+                                                heads=heads, kv_heads=kv, dim=dim))
+        if projection:
+            steps.append(lambda: runtime._linear4([att, *bufs[6:9], out], rows=tokens, cols=cols,
+                                                  k=width))
+        if separate:
+            for step in steps:
+                with runtime.command():
+                    step()
+        else:
+            with runtime.command():
+                for step in steps:
+                    step()
+        results.append([runtime.read(b, a.shape) for b, a in zip(bufs[:2], (q, k))]
+                       + [runtime.read(att, (tokens, width)), runtime.read(out, (tokens, cols))])
+        for b in [*bufs, att, out]:
+            b.close()
+    for together, alone in zip(*results):
+        np.testing.assert_array_equal(together, alone)
+        assert np.isfinite(together).all()
