@@ -118,6 +118,24 @@ __device__ __forceinline__ void split2(float x0, float x1, float one, half2v& hi
               static_cast<_Float16>(fmaf(-static_cast<float>(hi.y), one, x1))};
 }
 
+// The power of two that brings a row's largest magnitude mx into [2^13, 2^14) (1 for all-zero and
+// non-finite rows), by which linear4_hilo scales the row.
+__device__ __forceinline__ float row_scale_of(float mx) {
+  float scale = 1.0f;
+  if (mx > 0.0f && mx <= 3.402823466e38f) {
+    int ex;
+    frexpf(mx, &ex);  // mx = f * 2^ex, f in [0.5, 1): mx * 2^(14 - ex) in [2^13, 2^14)
+    scale = ldexpf(1.0f, min(max(14 - ex, -126), 126));
+  }
+  return scale;
+}
+
+__device__ __forceinline__ float wave_max(float x) {
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
+  return x;
+}
+
 __device__ __forceinline__ float wave_sum(float x) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) x += __shfl_xor(x, off);

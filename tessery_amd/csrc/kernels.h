@@ -59,7 +59,7 @@ hipError_t launch_attention_f16(const AttnArgs& a, hipStream_t st);
 
 // tessery rms_norm (kernels.metal:53-63): rows x cols fp32, bf16 weight, out may alias x.
 hipError_t launch_rms_norm_f32(const float* x, const uint16_t* w, float* out, int rows, int cols,
-                               float eps, void* planes, hipStream_t st);
+                               float eps, void* planes, float* scales, hipStream_t st);
 // RoPE tables [S, D/2] of cos / sin(pos * theta^(-2j/D)), evaluated in float64 on the device
 // and rounded once to float32.
 bool rope_tables_fit(int S, int D);
@@ -72,7 +72,7 @@ hipError_t launch_rope_f32(float* x, const float* cos_tab, const float* sin_tab,
 // hipErrorNotReady unless cols % 4 == 0 and x, r, y are 16-byte aligned.
 hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, float* y,
                                    int rows, int cols, float eps, void* planes,
-                                   hipStream_t st);
+                                   float* scales, hipStream_t st);
 // launch_rms_norm_f32 in place (x == out) followed by launch_rope_f32 on the same rows, as one
 // kernel with the same bits, over one or two sets of rows (q, then k) of one dim and seq;
 // hipErrorNotReady when the shape is not covered (8 | dim <= 256, x 16-byte aligned) and the
@@ -111,8 +111,9 @@ struct PlanesScratch {
   void *in, *out;
   size_t bytes;
 };
+// scaled: the row scales that linear4_hilo reads are in scratch already.
 hipError_t launch_linear4_f32(const Linear4Job& job, float* scratch, size_t scratch_floats,
-                              const PlanesScratch& planes, hipStream_t st);
+                              bool scaled, const PlanesScratch& planes, hipStream_t st);
 // Whether launch_linear4_f32 runs the job on linear4_rows, whose results depend neither on the rows
 // of the launch nor on the projections beside it.
 bool linear4_on_rows(const Linear4Job& job, const float* scratch, size_t scratch_floats);
@@ -127,11 +128,12 @@ hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated,
                                hipStream_t st);
 // The same projection for M >= kLinear4HiloRows rows on fp16 MFMA: rows scaled by powers of two
 // and split into hi + lo fp16 halves (about 22 bits), exact codes, fp32 sums. scratch holds the M
-// row scales. x and y start at row 0 of the range; N % 128 == 0, K % 64 == 0.
+// row scales (scaled: it does already). x and y start at row 0 of the range; N % 128 == 0, K % 64 == 0.
 constexpr int kLinear4HiloRows = 1024;
 hipError_t launch_linear4_hilo_f32(const float* x, const uint32_t* w, const uint16_t* scales,
                                    const uint16_t* biases, float* y, int M, int N, int K,
-                                   float* scratch, size_t scratch_floats, hipStream_t st);
+                                   float* scratch, size_t scratch_floats, bool scaled,
+                                   hipStream_t st);
 // Two projections of one x with the same shape in one launch on the same path: u = x Wu^T and
 // y = x Wg^T, or with `gated` (the gated MLP) y = silu(x Wg^T) * u: the values linear4 (-> y) +
 // linear4 (-> u) (+ silu_gate(y, u)) leave, bit for bit. M >= kLinear4HiloRows, both sets' scale
@@ -141,7 +143,7 @@ hipError_t launch_linear4_hilo_dual_f32(const float* x, const uint32_t* w, const
                                         const uint16_t* biases, float* y, const uint32_t* uw,
                                         const uint16_t* uscales, const uint16_t* ubiases, float* u,
                                         bool gated, int M, int N, int K, float* scratch,
-                                        size_t scratch_floats, hipStream_t st);
+                                        size_t scratch_floats, bool scaled, hipStream_t st);
 // gate[i] = silu(gate[i]) * up[i] for i < n (tessery silu_gate, kernels.metal:334-337).
 hipError_t launch_silu_gate_f32(float* gate, const float* up, uint32_t n, hipStream_t st);
 

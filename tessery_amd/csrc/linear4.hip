@@ -560,12 +560,12 @@ hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated,
 }
 
 hipError_t launch_linear4_f32(const Linear4Job& j, float* scratch, size_t scratch_floats,
-                              const PlanesScratch& planes, hipStream_t st) {
+                              bool scaled, const PlanesScratch& planes, hipStream_t st) {
   if (j.row1 <= j.row0 || j.cols <= 0) return hipSuccess;
   if (runs_hilo(j, scratch, scratch_floats))
     return launch_linear4_hilo_f32(j.x + static_cast<size_t>(j.row0) * j.k, j.w, j.scales, j.biases,
                                    j.out + static_cast<size_t>(j.row0) * j.cols, j.row1 - j.row0,
-                                   j.cols, j.k, scratch, scratch_floats, st);
+                                   j.cols, j.k, scratch, scratch_floats, scaled, st);
   return launch_linear4_rows(&j, 1, false, planes, false, false, st);
 }
 

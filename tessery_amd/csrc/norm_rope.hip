@@ -33,11 +33,12 @@ __device__ __forceinline__ float rope_second(float a, float b, float cv, float s
 
 // One wavefront per row, 4 rows per 256-thread workgroup. out may alias x. With VEC (cols a
 // multiple of 4, x and out 16-byte aligned) rows are read and written as float4. With PLANES (VEC,
-// cols a multiple of 64) the result also goes out as planes.h's terms, for the projections after it.
+// cols a multiple of 64) the result also goes out as planes.h's terms, for the projections after it;
+// with `scales` (VEC), the row scales that linear4_hilo reads.
 template <bool VEC, bool PLANES>
 __global__ __launch_bounds__(256) void rms_norm_f32(const float* x, const uint16_t* __restrict__ w,
                                                     float* out, int rows, int cols, float eps,
-                                                    Planes planes) {
+                                                    Planes planes, float* scales) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;  // row-uniform: the whole wavefront leaves together
@@ -53,6 +54,7 @@ __global__ __launch_bounds__(256) void rms_norm_f32(const float* x, const uint16
     }
     const float inv = inv_rms(squares, cols, eps);
     floatx4* y4 = reinterpret_cast<floatx4*>(yr);
+    float largest = 0.0f;
 #pragma unroll 4
     for (int c = lane; c < c4n; c += 64) {
       const floatx4 v = x4[c];
@@ -61,6 +63,11 @@ __global__ __launch_bounds__(256) void rms_norm_f32(const float* x, const uint16
       for (int j = 0; j < 4; ++j) r[j] = v[j] * inv * bf16_to_float(w[4 * c + j]);
       y4[c] = r;
       if constexpr (PLANES) store_planes4(planes, row, 4 * c, cols >> 6, r);
+      largest = fmaxf(fmaxf(largest, fmaxf(fabsf(r[0]), fabsf(r[1]))), fmaxf(fabsf(r[2]), fabsf(r[3])));
+    }
+    if (scales) {
+      largest = wave_max(largest);
+      if (lane == 0) scales[row] = row_scale_of(largest);
     }
     return;
   }
@@ -203,19 +210,19 @@ __global__ __launch_bounds__(256) void norm_rope_f16(const _Float16* __restrict_
 }
 
 hipError_t launch_rms_norm_f32(const float* x, const uint16_t* w, float* out, int rows, int cols,
-                               float eps, void* planes, hipStream_t st) {
+                               float eps, void* planes, float* scales, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
   const bool vec = (cols & 3) == 0 &&
                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-  if (planes && (!vec || cols % 64)) return hipErrorInvalidValue;
+  if ((planes || scales) && (!vec || cols % 64)) return hipErrorInvalidValue;
   const dim3 grid((rows + 3) / 4);
   if (planes)
     rms_norm_f32<true, true><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps,
-                                                   planes_at(planes, rows, cols));
+                                                   planes_at(planes, rows, cols), scales);
   else if (vec)
-    rms_norm_f32<true, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{});
+    rms_norm_f32<true, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{}, scales);
   else
-    rms_norm_f32<false, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{});
+    rms_norm_f32<false, false><<<grid, 256, 0, st>>>(x, w, out, rows, cols, eps, Planes{}, nullptr);
   return hipGetLastError();
 }
 
@@ -226,7 +233,7 @@ template <bool PLANES>
 __global__ __launch_bounds__(256) void add_rms_norm_f32(float* x, const float* __restrict__ r,
                                                         const uint16_t* __restrict__ w, float* y,
                                                         int rows, int cols, float eps,
-                                                        Planes planes) {
+                                                        Planes planes, float* scales) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
@@ -245,6 +252,7 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32(float* x, const float* _
   }
   const float inv = inv_rms(squares, cols, eps);
   floatx4* y4 = reinterpret_cast<floatx4*>(y + static_cast<size_t>(row) * cols);
+  float largest = 0.0f;
 #pragma unroll 4
   for (int c = lane; c < c4n; c += 64) {
     const floatx4 v = x4[c];  // this lane's own store above
@@ -253,14 +261,19 @@ __global__ __launch_bounds__(256) void add_rms_norm_f32(float* x, const float* _
     for (int j = 0; j < 4; ++j) o[j] = v[j] * inv * bf16_to_float(w[4 * c + j]);
     y4[c] = o;
     if constexpr (PLANES) store_planes4(planes, row, 4 * c, cols >> 6, o);
+    largest = fmaxf(fmaxf(largest, fmaxf(fabsf(o[0]), fabsf(o[1]))), fmaxf(fabsf(o[2]), fabsf(o[3])));
+  }
+  if (scales) {
+    largest = wave_max(largest);
+    if (lane == 0) scales[row] = row_scale_of(largest);
   }
 }
 
 hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, float* y,
                                    int rows, int cols, float eps, void* planes,
-                                   hipStream_t st) {
+                                   float* scales, hipStream_t st) {
   if (rows <= 0) return hipSuccess;
-  if (planes && cols % 64) return hipErrorInvalidValue;
+  if ((planes || scales) && cols % 64) return hipErrorInvalidValue;
   if (cols <= 0 || cols % 4 ||
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(r) |
         reinterpret_cast<uintptr_t>(y)) & 15))
@@ -268,9 +281,9 @@ hipError_t launch_add_rms_norm_f32(float* x, const float* r, const uint16_t* w, 
   const dim3 grid((rows + 3) / 4);
   if (planes)
     add_rms_norm_f32<true><<<grid, 256, 0, st>>>(x, r, w, y, rows, cols, eps,
-                                                 planes_at(planes, rows, cols));
+                                                 planes_at(planes, rows, cols), scales);
   else
-    add_rms_norm_f32<false><<<grid, 256, 0, st>>>(x, r, w, y, rows, cols, eps, Planes{});
+    add_rms_norm_f32<false><<<grid, 256, 0, st>>>(x, r, w, y, rows, cols, eps, Planes{}, scales);
   return hipGetLastError();
 }
 

@@ -421,13 +421,7 @@ __global__ __launch_bounds__(256) void row_scales_f32(const float* __restrict__ 
     const floatx4 v = xr[c];
     mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
   }
-  for (int off = 32; off >= 1; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-  float scale = 1.0f;
-  if (mx > 0.0f && mx <= 3.402823466e38f) {
-    int ex;
-    frexpf(mx, &ex);  // mx = f * 2^ex, f in [0.5, 1): mx * 2^(14 - ex) in [2^13, 2^14)
-    scale = ldexpf(1.0f, min(max(14 - ex, -126), 126));
-  }
+  const float scale = row_scale_of(wave_max(mx));
   if (lane == 0) rs[row] = scale;
 }
 
@@ -753,11 +747,12 @@ static bool hilo_fits(int M, int N, int K, const float* x, const float* y, const
 
 hipError_t launch_linear4_hilo_f32(const float* x, const uint32_t* w, const uint16_t* scales,
                                    const uint16_t* biases, float* y, int M, int N, int K,
-                                   float* scratch, size_t scratch_floats, hipStream_t st) {
+                                   float* scratch, size_t scratch_floats, bool scaled,
+                                   hipStream_t st) {
   if (M <= 0) return hipSuccess;
   if (!hilo_fits(M, N, K, x, y, scratch, scratch_floats) || hilo_sb_bytes(K) > 64 * 1024)
     return hipErrorInvalidValue;
-  row_scales_f32<<<(M + 3) / 4, 256, 0, st>>>(x, M, K, scratch);
+  if (!scaled) row_scales_f32<<<(M + 3) / 4, 256, 0, st>>>(x, M, K, scratch);
   dim3 grid((M + 63) / 64, N / 128);
   linear4_hilo<false><<<grid, 256, hilo_sb_bytes(K), st>>>(x, scratch, w, scales, biases, y,
                                                           nullptr, nullptr, nullptr, nullptr, 0,
@@ -776,12 +771,12 @@ hipError_t launch_linear4_hilo_dual_f32(const float* x, const uint32_t* w, const
                                         const uint16_t* biases, float* y, const uint32_t* uw,
                                         const uint16_t* uscales, const uint16_t* ubiases, float* u,
                                         bool gated, int M, int N, int K, float* scratch,
-                                        size_t scratch_floats, hipStream_t st) {
+                                        size_t scratch_floats, bool scaled, hipStream_t st) {
   if (M <= 0) return hipSuccess;
   if (!linear4_hilo_dual_fits(M, N, K) || !hilo_fits(M, N, K, x, y, scratch, scratch_floats) ||
       (reinterpret_cast<uintptr_t>(u) & 15))
     return hipErrorInvalidValue;
-  row_scales_f32<<<(M + 3) / 4, 256, 0, st>>>(x, M, K, scratch);
+  if (!scaled) row_scales_f32<<<(M + 3) / 4, 256, 0, st>>>(x, M, K, scratch);
   dim3 grid((M + 63) / 64, N / 128);
   linear4_hilo<true><<<grid, 256, 2 * hilo_sb_bytes(K), st>>>(x, scratch, w, scales, biases, y,
                                                              uw, uscales, ubiases, u,

@@ -748,8 +748,16 @@ tessery::PlanesScratch planes_scratch(Runtime* rt, int slot) {
   return {rt->planes[slot], rt->planes[1 - slot], kPlanesBytes};
 }
 
-// planes: where a rms_norm or an attention also leaves its output as planes (null: nowhere).
-hipError_t launch(Runtime* rt, const Op& op, void* planes) {
+// What a launch leaves and finds beside its op's buffers: where a rms_norm or an attention also puts
+// its output as planes, where a rms_norm puts the row scales of its output (null: nowhere), and
+// whether a projection finds the row scales of its input in the dense scratch.
+struct Beside {
+  void* planes = nullptr;
+  float* scales = nullptr;
+  bool scaled = false;
+};
+
+hipError_t launch(Runtime* rt, const Op& op, const Beside& beside) {
   hipStream_t st = rt->stream;
   const Params& p = op.p;
   switch (op.route) {
@@ -762,7 +770,7 @@ hipError_t launch(Runtime* rt, const Op& op, void* planes) {
     case R_ATTENTION_F16_NORM_ROPE: {
       tessery::AttnArgs a{};
       if (!attention_args(rt, op, &a)) return hipErrorInvalidValue;
-      a.planes = planes;
+      a.planes = beside.planes;
       if (op.route == R_ATTENTION || op.route == R_ATTENTION_F16_SCALAR)
         return tessery::launch_attention_scalar(a, st);
       if (op.route == R_ATTENTION_F16 || op.route == R_ATTENTION_F16_NORM_ROPE)
@@ -783,7 +791,7 @@ hipError_t launch(Runtime* rt, const Op& op, void* planes) {
       return tessery::launch_rms_norm_f32(
           static_cast<const float*>(op.ptr[0]), static_cast<const uint16_t*>(op.ptr[1]),
           static_cast<float*>(op.ptr[2]), static_cast<int>(op.threads / 32),
-          static_cast<int>(p.cols), p.eps, planes, st);
+          static_cast<int>(p.cols), p.eps, beside.planes, beside.scales, st);
     case R_ROPE: {
       const RopeTable* t = rope_of(rt, p);
       if (!t) return hipErrorInvalidValue;
@@ -799,7 +807,7 @@ hipError_t launch(Runtime* rt, const Op& op, void* planes) {
     case R_LINEAR4_SMALL3: {
       tessery::Linear4Job job;
       if (!linear4_job(op, &job)) return hipErrorInvalidValue;
-      return tessery::launch_linear4_f32(job, rt->dense_scratch, kDenseScratchFloats,
+      return tessery::launch_linear4_f32(job, rt->dense_scratch, kDenseScratchFloats, beside.scaled,
                                          planes_scratch(rt, 0), st);
     }
     case R_QKV4_F16:
@@ -1023,7 +1031,7 @@ int mi_dispatch(void* runtime, const char* name, void** buffers, uint32_t count,
   return queue_op(rt, op) ? 0 : 1;
 }
 
-hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated);
+hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated, bool scaled);
 
 // The rows of an in-place rms_norm whose rope follows.
 bool norm_rope_rows(const Op& a, const Op& b, tessery::NormRopeRows* rows) {
@@ -1066,9 +1074,9 @@ hipError_t launch_norm_rope_pairs(Runtime* rt, size_t first, size_t last) {
 //     same shape and lengths, neither writing a buffer of the other -> the attention launch with
 //     the prologue in extra workgroups.
 // Returns the launch status, or hipErrorNotReady when ops[i], ops[i + 1] are not such a pair.
-hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes) {
+hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, const Beside& beside) {
   hipStream_t st = rt->stream;
-  if (is_linear4(a.route)) return launch_fused_dual(rt, a, b, false);
+  if (is_linear4(a.route)) return launch_fused_dual(rt, a, b, false, beside.scaled);
   if (a.route == R_ADD && b.route == R_LAYER_NORM && a.ptr[2] == a.ptr[0] &&
       b.ptr[0] == a.ptr[0] && b.ptr[3] == a.ptr[0] && a.ptr[1] != a.ptr[0] &&
       static_cast<uint64_t>(a.p.n) == (b.threads / 32) * b.p.cols) {
@@ -1083,7 +1091,7 @@ hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes
     return tessery::launch_add_rms_norm_f32(
         static_cast<float*>(a.ptr[0]), static_cast<const float*>(a.ptr[1]),
         static_cast<const uint16_t*>(b.ptr[1]), static_cast<float*>(b.ptr[2]),
-        static_cast<int>(b.threads / 32), static_cast<int>(b.p.cols), b.p.eps, planes, st);
+        static_cast<int>(b.threads / 32), static_cast<int>(b.p.cols), b.p.eps, beside.planes, beside.scales, st);
   }
   if (a.route == R_QKV4_F16 && b.route == R_NORM_ROPE_F16 && b.ptr[0] == a.ptr[5] &&
       b.p.dim == 128 && static_cast<uint64_t>(b.p.heads) * 128 == a.p.n &&
@@ -1147,18 +1155,18 @@ hipError_t launch_fused_pair(Runtime* rt, const Op& a, const Op& b, void* planes
 // of their outputs and would run the fp16-MFMA kernel, one launch computes both from one staging
 // of x and leaves the same bits in g and u. Returns the launch status, or hipErrorNotReady when
 // ops[i .. i + 2] are not such a triple.
-hipError_t launch_fused_gated(Runtime* rt, const Op& a, const Op& b, const Op& c) {
+hipError_t launch_fused_gated(Runtime* rt, const Op& a, const Op& b, const Op& c, bool scaled) {
   if (c.route != R_SILU_GATE || c.ptr[0] != a.ptr[4] || c.ptr[1] != b.ptr[4] ||
       static_cast<uint64_t>(c.p.n) != static_cast<uint64_t>(a.p.rows) * a.p.cols)
     return hipErrorNotReady;
-  return launch_fused_dual(rt, a, b, true);
+  return launch_fused_dual(rt, a, b, true, scaled);
 }
 
 // Two uint4 projections of the same x with the same shape (the k and v projections of a Qwen3
 // layer, or the gated MLP's gate and up) as one launch of the fp16-MFMA kernel, with the bits of
 // the two launches; with `gated` the first output receives silu(first) * second. Returns the
 // launch status, or hipErrorNotReady when the pair does not qualify.
-hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated) {
+hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated, bool scaled) {
   if (!is_linear4(a.route) || b.route != a.route) return hipErrorNotReady;
   const Params &pa = a.p, &pb = b.p;
   if (pa.rows != pb.rows || pa.cols != pb.cols || pa.k != pb.k || a.ptr[0] != b.ptr[0])
@@ -1184,7 +1192,7 @@ hipError_t launch_fused_dual(Runtime* rt, const Op& a, const Op& b, bool gated) 
       static_cast<float*>(a.ptr[4]), static_cast<const uint32_t*>(b.ptr[1]),
       static_cast<const uint16_t*>(b.ptr[2]), static_cast<const uint16_t*>(b.ptr[3]),
       static_cast<float*>(b.ptr[4]), gated, M, N, K, rt->dense_scratch, kDenseScratchFloats,
-      rt->stream);
+      scaled, rt->stream);
   // hipErrorInvalidValue: nothing was launched (alignment or sizes); the ops run as queued
   return e == hipErrorInvalidValue ? hipErrorNotReady : e;
 }
@@ -1380,7 +1388,14 @@ struct Ready {
 struct Pass {
   FusionCount fused;
   Ready ready;
+  Ready scaled;  // the row scales of x [rows, k], in the dense scratch
 };
+
+// The projection of op `at` when it starts at row 0 and runs on linear4_hilo, which reads row scales.
+bool reads_scales(Runtime* rt, size_t at, size_t last, tessery::Linear4Job* job) {
+  return at < last && linear4_job(rt->ops[at], job) && job->row0 == 0 &&
+         !tessery::linear4_on_rows(*job, rt->dense_scratch, kDenseScratchFloats);
+}
 
 // Whether op `at` starts a projection that reads all of x [rows, k] as planes the scratch holds.
 bool reads_planes(Runtime* rt, size_t at, size_t last, const void* x, uint64_t rows, uint64_t k) {
@@ -1396,8 +1411,8 @@ bool reads_planes(Runtime* rt, size_t at, size_t last, const void* x, uint64_t r
 // launch_fused_pair (the last two counted). A kernel whose output the next launch projects leaves
 // its planes too. *taken: the ops launched.
 hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pass* pass) {
-  const Ready ready = pass->ready;
-  pass->ready = {};
+  const Ready ready = pass->ready, scaled = pass->scaled;
+  pass->ready = pass->scaled = {};
   const Op& op = rt->ops[first];
   Projection p;
   if (find_projection(rt, first, last, &p)) {
@@ -1410,6 +1425,10 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
     const bool keep = p.gated && j.row0 == 0 && j.out != j.x &&
                       tessery::planes_bytes(j.row1, j.k) <= kPlanesBytes &&
                       reads_planes(rt, p.end, last, j.out, j.row1, j.cols);
+    // its scratch is another one: the row scales of its input stay
+    bool untouched = true;
+    for (int i = 0; i < p.count; ++i) untouched = untouched && p.jobs[i].out != scaled.x;
+    if (untouched) pass->scaled = scaled;
     if (keep)
       pass->ready = {j.out, static_cast<uint64_t>(j.row1), static_cast<uint64_t>(j.cols), 1 - slot};
     return tessery::launch_linear4_rows(p.jobs, p.count, p.gated, planes_scratch(rt, slot),
@@ -1425,10 +1444,24 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
     pass->fused.pairs += d.gelu && e == hipSuccess;
     return e;
   }
+  Beside beside;
+  tessery::Linear4Job hilo;
+  const bool on_hilo = reads_scales(rt, first, last, &hilo);
+  if (on_hilo) {
+    beside.scaled = scaled.x == hilo.x && scaled.rows >= static_cast<uint64_t>(hilo.row1) &&
+                    scaled.k == static_cast<uint64_t>(hilo.k);
+    // for the next projection of the same input
+    if (hilo.out != hilo.x)
+      pass->scaled = beside.scaled ? scaled
+                                   : Ready{hilo.x, static_cast<uint64_t>(hilo.row1),
+                                           static_cast<uint64_t>(hilo.k), 0};
+  }
   const hipError_t gated =
-      first + 2 < last ? launch_fused_gated(rt, op, rt->ops[first + 1], rt->ops[first + 2])
-                       : hipErrorNotReady;
+      first + 2 < last
+          ? launch_fused_gated(rt, op, rt->ops[first + 1], rt->ops[first + 2], beside.scaled)
+          : hipErrorNotReady;
   if (gated != hipErrorNotReady) {
+    pass->scaled = {};  // of no use to what follows the gated projections
     pass->fused.gated += gated == hipSuccess;
     *taken = 3;
     return gated;
@@ -1447,19 +1480,42 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
       return Ready{n.ptr[2], rows, n.p.cols, 0};
     return Ready{};
   };
+  // the row scales of a rms_norm's output that a projection reads
+  auto norm_scales = [&](size_t at) {
+    const Op& n = rt->ops[at];
+    const uint64_t rows = n.threads / 32;
+    tessery::Linear4Job job;
+    if (n.route == R_RMS_NORM && reads_scales(rt, at + 1, last, &job) && job.x == n.ptr[2] &&
+        static_cast<uint64_t>(job.row1) <= rows && rows <= kDenseScratchFloats &&
+        job.k == static_cast<int>(n.p.cols))
+      return Ready{n.ptr[2], rows, n.p.cols, 0};
+    return Ready{};
+  };
   if (first + 1 < last) {
-    const Ready after = op.route == R_ADD ? norm_ready(first + 1) : Ready{};
-    const hipError_t pair = launch_fused_pair(rt, op, rt->ops[first + 1],
-                                              after.x ? rt->planes[after.slot] : nullptr);
+    Ready after, scales;
+    if (op.route == R_ADD) {
+      after = norm_ready(first + 1);
+      scales = norm_scales(first + 1);
+      beside.planes = after.x ? rt->planes[after.slot] : nullptr;
+      beside.scales = scales.x ? rt->dense_scratch : nullptr;
+    }
+    const hipError_t pair = launch_fused_pair(rt, op, rt->ops[first + 1], beside);
     if (pair != hipErrorNotReady) {
       pass->fused.pairs += pair == hipSuccess;
       pass->ready = after;
+      if (scales.x) pass->scaled = scales;
+      // a second projection of the input: its output may be that input only in the pair itself
+      if (on_hilo && rt->ops[first + 1].ptr[4] == hilo.x) pass->scaled = {};
       *taken = 2;
       return pair;
     }
   }
   *taken = 1;
   pass->ready = norm_ready(first);
+  if (const Ready scales = norm_scales(first); scales.x) {
+    pass->scaled = scales;
+    beside.scales = rt->dense_scratch;
+  }
   tessery::AttnArgs at{};
   if (attention_args(rt, op, &at) && tessery::attention_leaves_planes(at, op.route == R_ATTENTION)) {
     const uint64_t rows = static_cast<uint64_t>(at.B) * static_cast<uint64_t>(at.S);
@@ -1467,7 +1523,8 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
     if (reads_planes(rt, first + 1, last, at.out, rows, width))
       pass->ready = Ready{at.out, rows, width, 0};
   }
-  return launch(rt, op, pass->ready.x ? rt->planes[pass->ready.slot] : nullptr);
+  beside.planes = pass->ready.x ? rt->planes[pass->ready.slot] : nullptr;
+  return launch(rt, op, beside);
 }
 
 // Launches ops [first, last) in order; the fusions made are added to *fc. Under stream capture
