@@ -4,8 +4,9 @@
 // K and N: the matmul_f32 / matmul_f32_tiled / matmul_f32_chunk32 / matmul_bias_f32 /
 // matmul_bias_f32_chunk32 routes (kernels.metal:306-322, 396-487). Weights stay [N, K] as in the
 // reference ("transposed weight"). Products accumulate in K32 partial sums added to the total
-// (the chunk32 order, kernels.metal:416-436), every route runs this one kernel, and the bias is
-// added once after the last partial sum.
+// (the chunk32 order, kernels.metal:416-436), and the bias is added once after the last one. Every
+// route runs the same kernels: matmul_planes and matmul_x3 on bf16 MFMA where K % 32 == 0 (below),
+// matmul_f32 for the rest.
 // add_bias, gelu_f32 and layer_norm follow kernels.metal:362-394.
 #include <algorithm>
 
@@ -151,14 +152,14 @@ __global__ __launch_bounds__(256) void matmul_f32(const float* __restrict__ a,
     }
 }
 
-// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are split exactly into three bf16 planes each (split3x8)
-// and every fp32 product is taken as the six terms b_i c_j with i + j <= 4 on
-// v_mfma_f32_32x32x16_bf16 in fp32 (the bf16 rate is 16x the fp32 one, so six products cost well
-// under half the fp32 instructions). Tile 64 rows x 128 columns; wavefront w
-// owns rows 32 (w >> 1) .. +31 and columns 64 (w & 1) .. +63 (two 32x32 tiles). Per 32-wide K
-// chunk every thread loads 8 floats of one x row and 16 of one weight row into registers (one
-// chunk ahead), splits them after the barrier that retires the previous chunk's reads, and
-// stores the three planes to LDS as rows of 64 bytes (four 16-byte chunks, chunk c of row r at
+// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are split
+// exactly into three bf16 planes each (split3x8) and every fp32 product is taken as the six terms
+// b_i c_j with i + j <= 4 on v_mfma_f32_32x32x16_bf16 in fp32 (the bf16 rate is 16x the fp32 one, so
+// six products cost well under half the fp32 instructions). Tile 64 rows x 128 columns; wavefront w
+// owns rows 32 (w >> 1) .. +31 and columns 64 (w & 1) .. +63 (two 32x32 tiles). Per 32-wide K chunk
+// every thread loads 8 floats of one x row and 16 of one weight row into registers (one chunk
+// ahead), splits them after the barrier that retires the previous chunk's reads, and stores the
+// three planes to LDS as rows of 64 bytes (four 16-byte chunks, chunk c of row r at
 // c ^ ((r >> 1) & 3): conflict-free for the 16-lane reads and the 8-lane writes on gfx950). As in
 // matmul_f32, each 32-wide chunk's products form a partial sum added to the total (the chunk32
 // order), and the bias and GELU are applied the same way. Rows past row1 read row0 and are never
@@ -702,8 +703,8 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
   const int row0 = j.row0, row1 = j.row1, cols = j.cols, k = j.k;
   const size_t scratch_floats = dense.sums_floats;
   const int rows = row1 - row0, chunks = (k + 63) / 64;
-  // large shapes on bf16 MFMA (split x3), with 16-byte rows: at least two tiles per CU, or K
-  // split over workgroups into partial sums (about 768 workgroups) from 64 tiles
+  // bf16 MFMA (split x3), with 16-byte rows: at least two tiles per CU, or K split over workgroups
+  // into partial sums
   const int x3_tiles = ((rows + kX3Rows - 1) / kX3Rows) * (cols / 128);
   const int x3_splits = k % 32 == 0 && cols % 128 == 0 &&
                                 ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(bt)) &

@@ -158,7 +158,7 @@ struct Runtime {
   bool graphs = true;  // replay plans through cached HIP graphs (TESSERY_HIP_GRAPHS=0 disables)
   uint64_t graph_launches = 0, graph_builds = 0;
   uint64_t fused_pairs = 0, fused_gated = 0;  // launch-time fusions (diagnostics)
-  float* dense_scratch = nullptr;  // split-K partial sums of small-batch projections
+  float* dense_scratch = nullptr;  // split-K partial sums of dense projections, row scales of uint4
   void* dense_planes = nullptr;    // split operands of fp32 projections
   void* planes[2] = {};  // planes of the activations uint4 projections read, and of their output
   std::vector<Segment> segments;
@@ -581,8 +581,8 @@ bool is_dense(Route r) {
          r == R_MATMUL_BIAS_CHUNK32;
 }
 
-// Scratch of the split-K projection paths (dense and uint4), allocated once per runtime on first
-// use (its address never changes, so a captured graph keeps pointing at it).
+// Scratch of the split-K dense projections and of the fp16-MFMA uint4 ones' row scales, allocated
+// once per runtime on first use (its address never changes, so a captured graph keeps pointing at it).
 constexpr size_t kDenseScratchFloats = size_t{8} << 20;  // 32 MiB
 // Split operands of the dense projections: at most 512 tiles of 64 x 128 outputs (more run on
 // matmul_x3), which is 96 MiB where they are one column of tiles of K = 512.
