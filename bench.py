@@ -674,7 +674,7 @@ def bench_qwen_tail(args, tokens: int = 16 * 256) -> dict:
             "algorithmic_flop": flop,
             "algorithmic_bytes": gemm_bytes,
             "kernel": kernel + (" (fp16 MFMA, hi + lo halves: 2x the algorithmic MFMA work)"
-                                if hilo else " (fp32 MFMA)"),
+                                if hilo else " (bf16 MFMA, exact three-term split)"),
         },
     }
     if not args.no_cpu_baseline:
