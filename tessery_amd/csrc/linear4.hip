@@ -26,14 +26,19 @@ namespace tessery {
 
 namespace {
 
-// Per group of 64 inputs, with c' = c - 8 and b' = 8 scale + bias (w = scale c' + b'):
-//     y[m][n] += 16 scale[n] * sum_k x[m][k] (c'[n][k] / 16) + b'[n] * sum_k x[m][k]
-// x is split exactly into three bf16 terms (split3x8) and c' / 16 is exact in bf16, so every
-// product on v_mfma_f32_32x32x16_bf16 is exact and the sums are fp32: nothing is rounded that the
-// fp32 product would keep, at three bf16 MFMAs of 32 cycles per 16 inputs where fp32 MFMA takes
-// eight of 64. The second term is one more MFMA per group, its two factors split into three bf16
-// terms each. Centred codes keep the sums as small as the result (uncentred ones cancel against
-// the bias term).
+// Per group of 64 inputs, with c' = c - z and b' = z scale + bias (w = scale c' + b'), z being the whole
+// number of 0 .. 15 nearest to -bias / scale, for each column and group:
+//     y[m][n] += scale[n] * sum_k x[m][k] c'[n][k] + b'[n] * sum_k x[m][k]
+// x is split exactly into three bf16 terms (split3x8) and c' is exact in bf16, so every product on
+// v_mfma_f32_32x32x16_bf16 is exact and the sums are fp32, at three bf16 MFMAs of 32 cycles per 16
+// inputs where fp32 MFMA takes eight of 64. The second term is one more MFMA per group, its two
+// factors split into three bf16 terms each.
+//
+// z keeps both terms as small as w: where it is not cut off, |b'| <= |scale| / 2, so that
+// |scale c'| <= 2 |w| and |b'| <= |w| for every code; where it is, both terms have one sign. With one
+// z for all groups (8), a group whose codes sit at one end against a bias that cancels them lost
+// the result in the difference of two large sums: codes 0 with bias 2^-12 scale, 5.8e-4 of
+// sum |x| |w| instead of 1e-7.
 //
 // K order: eight partitions of consecutive groups (partition p: groups [p G / 8, (p + 1) G / 8)),
 // each summed on its own, then added as a balanced tree.
@@ -67,18 +72,39 @@ struct L4Args {
   Planes next;  // GATED: the planes of the output (terms null: none), row0 = 0
 };
 
-// (c - 8) / 16 of the eight codes of a weight word as bf16, in natural order
-__device__ __forceinline__ bf16x8 decode_centred(uint32_t word) {
-  const uint32_t even = word ^ 0x88888888u;
-  uint32_t odd = even >> 4;
-  asm("" : "+v"(odd));  // its bytes are then operand selects of the conversions, not shifts
+// z of a column's group, and -(2^(23 - 4 i) + z) for the codes at bits 4 i of a word.
+struct Centre {
+  float z, base[5];
+};
+__device__ __forceinline__ Centre centre_of(float scale, float bias) {
+  Centre c;
+  // any z is exact; the nearest one (within the reciprocal's rounding) is well conditioned. scale 0
+  // gives 0 or 15
+  c.z = __builtin_rintf(
+      __builtin_amdgcn_fmed3f(-bias * __builtin_amdgcn_rcpf(scale), 0.0f, 15.0f));
+#pragma unroll
+  for (int i = 0; i < 5; ++i) c.base[i] = -static_cast<float>(1 << (23 - 4 * i)) - c.z;
+  return c;
+}
+
+// c - z of the eight codes of a weight word as bf16, in natural order. A code at bits 4 i .. 4 i + 3 of
+// the significand of 2.0 makes 2 + c 2^(4 i - 22), and one fma c - z: two full-rate instructions a code
+// (masks and factors in scalar registers, 2.0 inline), where v_cvt_off_f32_i4 alone takes 16 cycles.
+__device__ __forceinline__ bf16x8 decode_centred(uint32_t word, const Centre& c) {
+  const uint32_t late = word >> 12;  // codes 5, 6 and 7 where 2, 3 and 4 were
+  uint32_t f[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int i = j < 5 ? j : j - 3;
+    uint32_t mask = 15u << (4 * i);
+    asm("" : "+s"(mask));  // a register, so that the mask and 2.0 fit one instruction
+    const uint32_t bits = ((j < 5 ? word : late) & mask) | 0x40000000u;
+    f[j] = __float_as_uint(
+        fmaf(__uint_as_float(bits), static_cast<float>(1 << (22 - 4 * i)), c.base[i]));
+  }
   uint4v r;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint32_t e = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((even >> (8 * j)) & 0xffu));
-    const uint32_t o = __float_as_uint(__builtin_amdgcn_cvt_off_f32_i4((odd >> (8 * j)) & 0xffu));
-    r[j] = __builtin_amdgcn_perm(o, e, 0x07060302u);
-  }
+  for (int j = 0; j < 4; ++j) r[j] = __builtin_amdgcn_perm(f[2 * j + 1], f[2 * j], 0x07060302u);
   return __builtin_bit_cast(bf16x8, r);
 }
 
@@ -179,20 +205,21 @@ __device__ __forceinline__ void column_tile(const L4Args& a, int width, int& til
 // k-slots, against the terms of its half-group sum) and the scale.
 struct Prepared {
   bf16x8 codes[4], bias;
-  float s16;
+  float scale;
 };
 // of group j (a constant after unrolling) of aligned words
 template <int N>
 __device__ __forceinline__ Prepared prepare_group(const Words<N>& words, int j) {
   auto upper = [&](uint32_t v) { return __uint_as_float(j & 1 ? v & 0xffff0000u : v << 16); };
   const float scale = upper(words.s[j / 2]), bias = upper(words.b[j / 2]);
+  const Centre centre = centre_of(scale, bias);
   Prepared r;
 #pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) r.codes[s4] = decode_centred(words.w[j][s4]);
-  const Split3 bs = split3(fmaf(8.0f, scale, bias));
+  for (int s4 = 0; s4 < 4; ++s4) r.codes[s4] = decode_centred(words.w[j][s4], centre);
+  const Split3 bs = split3(fmaf(centre.z, scale, bias));
   const uint32_t b12 = upper_pair(bs.t[0], bs.t[1]);
   r.bias = __builtin_bit_cast(bf16x8, uint4v{b12, b12, upper_pair(bs.t[2], bs.t[0]), 0u});
-  r.s16 = 16.0f * scale;
+  r.scale = scale;
   return r;
 }
 
@@ -214,7 +241,7 @@ __device__ __forceinline__ void multiply_group(const Prepared& w, X x, float xsu
     for (int s4 = 0; s4 < 4; ++s4)
       p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x(t, s4), w.codes[s4], p, 0, 0, 0);
 #pragma unroll
-  for (int e = 0; e < 16; ++e) acc[e] = fmaf(w.s16, p[e], acc[e]);
+  for (int e = 0; e < 16; ++e) acc[e] = fmaf(w.scale, p[e], acc[e]);
 }
 
 // The end of a tile of BLOCKS column blocks (GATED: the gate's, then the up projection's), one a
@@ -352,7 +379,7 @@ __global__ __launch_bounds__(512, 2) void linear4_rows(L4Args a) {
 // (GATED: half of the blocks are the gate's columns, half the up projection's). One group of x a
 // slot at a time is copied to LDS (two stages, the copy of the next group under way while this one
 // is multiplied) and read by the slot's WC wavefronts. Bound: the issue of VALU instructions
-// (decoding and folding, about 110 beside 13 MFMAs) and a step's barrier and waits. Measured: q, k
+// (decoding and folding, about 150 beside 13 MFMAs) and a step's barrier and waits. Measured: q, k
 // and v of 308 rows 18.1 us, gate and up 20.9; with x split in every workgroup 22 and 26.
 template <int WC, bool GATED>
 __global__ __launch_bounds__(512, WC == 4 ? 4 : 2) void linear4_rows_shared(L4Args a) {

@@ -234,3 +234,28 @@ def test_projections_beside_each_other_keep_their_bits(runtime, m, seq_of_ops):
     xs = x.astype(np.float64) + (r if seq_of_ops == "add" else 0)
     want = xs / np.sqrt((xs * xs).mean(-1, keepdims=True) + 1e-6) * bf16_values(gamma)
     np.testing.assert_allclose(results[0][0], want, atol=1e-5, rtol=1e-5)
+
+
+# Codes at one end of their range, or near it, against a bias that all but cancels them: w is far
+# smaller than scale * code and bias. One to four column blocks a workgroup.
+@pytest.mark.parametrize("m", [24, 300, 700])
+@pytest.mark.parametrize("code,bias,odd", [(0, 2.0**-12, None), (15, -15 + 2.0**-4, None),
+                                           (3, -3 + 2.0**-6, None), (12, -12 - 2.0**-4, None), (5, -5.0, None),
+                                           (0, 2.0**-12, 15), (15, -15 + 2.0**-4, 0)])
+def test_groups_whose_bias_cancels_their_codes(runtime, m, code, bias, odd):
+    """Within 1e-6 of sum_k |x| |w| of float64, as for any other weights; `odd`: one code of another
+    value per group, where x is zero. Scales of both signs and several magnitudes."""
+    n, k = 1056, 448
+    rng = np.random.default_rng(m + code)
+    x = rng.normal(size=(m, k)).astype(np.float32)
+    codes = np.full((n, k), code, np.uint32)
+    if odd is not None:
+        codes[:, 7::64] = odd
+        x[:, 7::64] = 0.0
+    scale = np.exp2(rng.integers(-12, 5, size=(n, k // 64))) * rng.choice((-1.0, 1.0), (n, k // 64))
+    packed, scales, biases = ref.pack(codes), bf16_words(scale), bf16_words(scale * bias)
+    got = project(runtime, [x, packed, scales, biases], m, n, k)
+    w = ref.dequantize(packed, scales, biases, k)
+    err = np.abs(got - x.astype(np.float64) @ w.T)
+    bound = 1e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    assert np.all(err <= bound), float((err / bound).max())
