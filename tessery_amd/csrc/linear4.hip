@@ -32,7 +32,8 @@ namespace {
 // x is split exactly into three bf16 terms (split3x8) and c' is exact in bf16, so every product on
 // v_mfma_f32_32x32x16_bf16 is exact and the sums are fp32, at three bf16 MFMAs of 32 cycles per 16
 // inputs where fp32 MFMA takes eight of 64. The second term is one more MFMA per group, its two
-// factors split into three bf16 terms each.
+// factors split into three bf16 terms each: eight of their nine products fill the lane's eight
+// k-slots, and the ninth (the two smallest terms) is below 2^-30 of the whole.
 //
 // z keeps both terms as small as w: where it is not cut off, |b'| <= |scale| / 2, so that
 // |scale c'| <= 2 |w| and |b'| <= |w| for every code; where it is, both terms have one sign. With one
@@ -218,7 +219,8 @@ __device__ __forceinline__ Prepared prepare_group(const Words<N>& words, int j) 
   for (int s4 = 0; s4 < 4; ++s4) r.codes[s4] = decode_centred(words.w[j][s4], centre);
   const Split3 bs = split3(fmaf(centre.z, scale, bias));
   const uint32_t b12 = upper_pair(bs.t[0], bs.t[1]);
-  r.bias = __builtin_bit_cast(bf16x8, uint4v{b12, b12, upper_pair(bs.t[2], bs.t[0]), 0u});
+  r.bias = __builtin_bit_cast(bf16x8, uint4v{b12, b12, upper_pair(bs.t[2], bs.t[0]),
+                                             upper_pair(bs.t[2], bs.t[1])});
   r.scale = scale;
   return r;
 }
@@ -226,11 +228,11 @@ __device__ __forceinline__ Prepared prepare_group(const Words<N>& words, int j) 
 // acc += the group's products for one 32 x 32 tile; x(t, s4): the operand of term t, k-step s4.
 template <typename X>
 __device__ __forceinline__ void multiply_group(const Prepared& w, X x, float xsum, floatx16& acc) {
-  // bias term: six products of the terms of the lane's half-group sum and b'
+  // bias term: the products of the terms of the lane's half-group sum and b' but the smallest one
   const Split3 xs = split3(xsum);
   const bf16x8 xa = __builtin_bit_cast(
       bf16x8, uint4v{upper_pair(xs.t[0], xs.t[0]), upper_pair(xs.t[1], xs.t[1]),
-                     upper_pair(xs.t[0], xs.t[2]), 0u});
+                     upper_pair(xs.t[0], xs.t[2]), upper_pair(xs.t[1], xs.t[2])});
   acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xa, w.bias, acc, 0, 0, 0);
   floatx16 p;
 #pragma unroll

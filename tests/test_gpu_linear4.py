@@ -259,3 +259,17 @@ def test_groups_whose_bias_cancels_their_codes(runtime, m, code, bias, odd):
     err = np.abs(got - x.astype(np.float64) @ w.T)
     bound = 1e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
     assert np.all(err <= bound), float((err / bound).max())
+
+
+def test_bias_term_keeps_every_product_of_its_terms(runtime):
+    """x and w whose second and third bf16 terms are as large as they get, all of one sign: the
+    products of those terms are 2^-21 of the result. The sums here are exact up to a few roundings
+    of the result (2^-24 each)."""
+    m, n, k = 24, 64, 512
+    x = np.full((m, k), 0x3f80ffff, np.uint32).view(np.float32)
+    scales = bf16_words(np.full((n, k // 64), 2.0**-26))
+    biases = bf16_words(np.full((n, k // 64), -1.0078125))
+    packed = ref.pack(np.full((n, k), 15, np.uint32))
+    got = project(runtime, [x, packed, scales, biases], m, n, k)
+    want = x.astype(np.float64) @ ref.dequantize(packed, scales, biases, k).T
+    assert np.all(np.abs(got - want) <= 2.5e-7 * np.abs(want)), float(np.abs(got / want - 1).max())
