@@ -154,8 +154,10 @@ __global__ __launch_bounds__(256) void matmul_f32(const float* __restrict__ a,
 
 // matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are split
 // exactly into three bf16 planes each (split3x8) and every fp32 product is taken as the six terms
-// b_i c_j with i + j <= 4 on v_mfma_f32_32x32x16_bf16 in fp32 (the bf16 rate is 16x the fp32 one, so
-// six products cost well under half the fp32 instructions). Tile 64 rows x 128 columns; wavefront w
+// b_i c_j with i + j <= 4, or (EXACT) the eight with i + j <= 5, on v_mfma_f32_32x32x16_bf16 in fp32
+// (the bf16 rate is 16x the fp32 one, so six products cost well under half the fp32 instructions;
+// what they leave out is at most 2^-21 of the product, eight 2^-30, and EXACT sums the leading products
+// apart from the others, so that only they round at the magnitude of the result). Tile 64 rows x 128 columns; wavefront w
 // owns rows 32 (w >> 1) .. +31 and columns 64 (w & 1) .. +63 (two 32x32 tiles). Per 32-wide K chunk
 // every thread loads 8 floats of one x row and 16 of one weight row into registers (one chunk
 // ahead), splits them after the barrier that retires the previous chunk's reads, and stores the
@@ -170,7 +172,7 @@ __device__ __forceinline__ int x3sw(int row) { return (row >> 1) & 3; }
 
 // PARTIAL: as in matmul_f32, workgroup z sums K chunks [z * per, (z + 1) * per) (of 32 here) and
 // stores its raw sums for dense_reduce.
-template <bool BIAS, bool GELU, bool PARTIAL>
+template <bool BIAS, bool GELU, bool PARTIAL, bool EXACT>
 __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
                                                    const float* __restrict__ bt,
                                                    const float* __restrict__ bias,
@@ -231,9 +233,9 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       const int wrow = 64 * wc + 32 * j + l32;
-      floatx16 c;
+      floatx16 c, lo;  // lo: with EXACT, all but the leading products
 #pragma unroll
-      for (int e = 0; e < 16; ++e) c[e] = 0.0f;
+      for (int e = 0; e < 16; ++e) c[e] = lo[e] = 0.0f;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
         const int chunk = 2 * ks + hh;
@@ -245,15 +247,20 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
         const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(&bs[0][bo]);
         const bf16x8 b2 = *reinterpret_cast<const bf16x8*>(&bs[1][bo]);
         const bf16x8 b3 = *reinterpret_cast<const bf16x8*>(&bs[2][bo]);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, b1, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b2, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b3, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b1, c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b2, c, 0, 0, 0);
+        floatx16& l = EXACT ? lo : c;
+        if constexpr (EXACT) {
+          l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, b2, l, 0, 0, 0);
+          l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b3, l, 0, 0, 0);
+        }
+        l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a3, b1, l, 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b2, l, 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b3, l, 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a2, b1, l, 0, 0, 0);
+        l = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b2, l, 0, 0, 0);
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a1, b1, c, 0, 0, 0);
       }
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[j][e] += c[e];
+      for (int e = 0; e < 16; ++e) acc[j][e] += EXACT ? c[e] + lo[e] : c[e];
     }
     __syncthreads();  // every wavefront has read this chunk's planes
   }
@@ -290,8 +297,10 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
 // no partial sums, and q, k and v in one launch. Measured, q, k and v of 656 rows: 3.4 + 12.3 us, 42
 // as three split-K launches of matmul_f32 with their reductions; of 4096: 5 + 28 us, 76 on matmul_x3.
 //
-// K order: two halves, each with its leading products in one sum and the five smaller ones in
-// another (only the leading ones round at the magnitude of the result), added at the end. It is
+// Eight products, all but that of the two smallest terms (below 2^-30 of the whole): nothing is lost
+// against fp32 products. K order: two halves, each with its leading products in one sum and the seven
+// smaller ones in another (only the leading ones round at the magnitude of the result), added at
+// the end. It is
 // the same for every tile shape, so a row's bits depend on no other row and on no projection
 // beside it.
 constexpr int kDenseStep = 3 * 64 * 8;  // bf16 words of a row tile's k-step
@@ -416,15 +425,15 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(Plane
     stage_barrier();
     if (begin + step >= end) return;
     const bool more = begin + step + 2 < end;
-    constexpr int term[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+    constexpr int term[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2}, {1, 2}, {1, 0}, {0, 1}, {0, 0}};
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
+    for (int i = 0; i < 16; ++i) {
       const int ks = i & 1, t = i >> 1;
-      floatx16& c = t < 5 ? lo : hi;
+      floatx16& c = t < 7 ? lo : hi;
       c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][term[t][0]], now.y[ks][term[t][1]], c,
                                                   0, 0, 0);
-      read(next, i, buf ^ 1);  // stale data after the last chunk, unused
-      if (more && (i & 1)) copy(i >> 1, buf, begin + step + 2);
+      if (i < READS) read(next, i, buf ^ 1);  // stale data after the last chunk, unused
+      if (more && i < 2 * COPIES && (i & 1)) copy(i >> 1, buf, begin + step + 2);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (KS == 1 && step + 1 == half) {
@@ -599,11 +608,12 @@ int dense_splits(int rows, int cols, int k, size_t scratch_floats) {
 // least four chunks (656 x 384 outputs of K = 1536: 17.3 us with 7 to 12 splits, 20.8 with 4, 21.8
 // with 24, and 24.9 on matmul_f32); 0 (the fp32 kernel) where the partial sums do not fit the
 // scratch or K is short. Every split holds at least one chunk.
+constexpr int kX3WideTiles = 64;  // fewer take eight products, as precise as matmul_f32 in their place
 static int x3_split_count(int rows, int cols, int k, int tiles, size_t scratch_floats) {
   if (tiles >= 512) return 1;
   const int chunks32 = k / 32;
-  if (tiles < 1 || chunks32 < (tiles < 64 ? 8 : 4)) return 0;
-  int splits = tiles < 64 ? std::min(chunks32 / 4, 256 / tiles)
+  if (tiles < 1 || chunks32 < (tiles < kX3WideTiles ? 8 : 4)) return 0;
+  int splits = tiles < kX3WideTiles ? std::min(chunks32 / 4, 256 / tiles)
                           : std::min(chunks32 / 2, (768 + tiles - 1) / tiles);
   const int per = (chunks32 + splits - 1) / splits;
   splits = (chunks32 + per - 1) / per;
@@ -714,22 +724,26 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
   if (x3_splits == 1) {
     dim3 grid((rows + kX3Rows - 1) / kX3Rows, cols / 128);
     if (bias && gelu)
-      matmul_x3<true, true, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
+      matmul_x3<true, true, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
     else if (bias)
-      matmul_x3<true, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
+      matmul_x3<true, false, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
     else if (gelu)
-      matmul_x3<false, true, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols, k,
+      matmul_x3<false, true, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols, k,
                                                           0);
     else
-      matmul_x3<false, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols,
+      matmul_x3<false, false, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols,
                                                            k, 0);
     return hipGetLastError();
   }
   if (x3_splits > 1) {
     const int chunks32 = k / 32, per = (chunks32 + x3_splits - 1) / x3_splits;
     dim3 grid((rows + kX3Rows - 1) / kX3Rows, cols / 128, x3_splits);
-    matmul_x3<false, false, true><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0, row1, cols,
-                                                        k, per);
+    if (x3_tiles < kX3WideTiles)
+      matmul_x3<false, false, true, true><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0, row1,
+                                                                cols, k, per);
+    else
+      matmul_x3<false, false, true, false><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0,
+                                                                 row1, cols, k, per);
     const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * cols + 255) / 256);
     if (bias && gelu)
       dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols,

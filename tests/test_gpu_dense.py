@@ -458,3 +458,22 @@ def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
     for (w, b), together, alone in zip(sets, *results):
         np.testing.assert_array_equal(together, alone)
         np.testing.assert_allclose(together, ref.linear(x, w, b), atol=2e-4, rtol=5e-5)
+
+
+# the split-operand kernel with both halves of K at once and in turn, and split K at few tiles
+@pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (656, 1152, 512),
+                                         (65, 384, 1536), (1, 256, 1568)])
+def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
+    """Operands whose second and third bf16 terms are near their largest (2^-7 and 2^-15 of the
+    first), all of one sign: the products of those terms add up to 2^-21 of the result, and only the
+    roundings of fp32 sums (2^-24 each, of either sign) may show (3.0e-7 on fp32 MFMA)."""
+    rng = np.random.default_rng(rows)
+
+    def near_largest(*shape):  # 1 + 2^-7 less a little
+        return (0x3f80ffff - rng.integers(0, 64, shape, dtype=np.uint32)).view(np.float32)
+
+    x, w = near_largest(rows, k), near_largest(cols, k)
+    got = run(runtime, "matmul_f32", [x, w], (rows, cols), threads=(rows + 3) // 4 * cols * 32,
+              group_size=32, rows=rows, cols=cols, k=k)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    assert np.all(np.abs(got - want) <= 3.5e-7 * want), float(np.abs(got / want - 1).max())
