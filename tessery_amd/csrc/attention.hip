@@ -1480,16 +1480,19 @@ __global__ __launch_bounds__(256, 2) void attn_f16_mfma(F16Args a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// fp32 attention on bf16 MFMA (routes attention_tiled / attention_tail_32 / attention_tail_128
-// at D = 32, 64, 128).
+// fp32 attention on bf16 MFMA (routes attention_tiled / attention_tail_32 / attention_tail_128, and
+// attention from 16 keys, at D = 32, 64, 128).
 //
 // An fp32 value x splits exactly into three bf16 terms by truncation: b1 = the upper half of x's
 // bits (sign, exponent, 7 mantissa bits), r1 = x - b1 (exact: the lower 16 significand bits),
 // b2 = the upper half of r1, b3 = r1 - b2 (at most 8 significant bits, so exactly a bf16). bf16
 // keeps fp32's exponent range, so no scaling is needed. A product x * y is taken as the six
-// terms b_i c_j with i + j <= 4; the three dropped ones are below 2^-24 |x y| (fp32 rounding),
-// every bf16 product is exact in fp32 and the MFMAs accumulate in fp32. The bf16 rate is 16x the
-// fp32 MFMA rate, so the six products still cost well under half of the fp32 instructions.
+// terms b_i c_j with i + j <= 4, or (EXACT) the eight with i + j <= 5: |b2| < 2^-7 |x| and
+// |b3| < 2^-15 |x|, each with x's sign, so the two that six leave out add up to at most 2^-21 |x y|
+// (for operands like 1.0078124, mostly far less), the one that eight leave out to 2^-30. Every bf16
+// product is exact in fp32 and the MFMAs accumulate in fp32. The bf16 rate is 16x the fp32 MFMA
+// rate, so six products cost well under half of the fp32 instructions. Route "attention" takes
+// eight: what it ran on before, attn_scalar, multiplies in fp32.
 //
 // Geometry, schedule and output layout are those of attn_f16_mfma (16 query rows per wavefront,
 // four wave blocks of one (batch row, kv head) plane per workgroup); tiles hold 2048 / D keys
@@ -1498,10 +1501,10 @@ __global__ __launch_bounds__(256, 2) void attn_f16_mfma(F16Args a) {
 // buffers (48 KiB: three workgroups per CU at <= 168 VGPRs): step t splits tile t + 1 and loads
 // tile t + 2 while its MFMAs run on tile t, one barrier per step.
 //   split [buffer][K, V][plane][2048 / D rows][D] bf16, chunks swizzled by ksw_x3 / vsw_x3
-// Score terms per k-step: (k1,q1) (k1,q2) (k2,q1) (k1,q3) (k2,q2) (k3,q1); output terms per
-// 16-channel block and 16-key block, each MFMA stacking two (probability, value) pairs over the
-// same four keys:
-// [p1,p1]x[v1,v2], [p2,p2]x[v1,v2], [p1,p3]x[v3,v1].
+// Score terms per k-step: (k1,q1), and in a sum of their own (EXACT: (k3,q2) (k2,q3)) (k3,q1) (k2,q2)
+// (k1,q3) (k2,q1) (k1,q2); output terms per 16-channel block and 16-key block, each MFMA stacking
+// two (probability, value) pairs over the same four keys:
+// [p1,p1]x[v1,v2], (EXACT: [p3,p2]x[v2,v3]), [p1,p3]x[v3,v1], [p2,p2]x[v1,v2].
 // ---------------------------------------------------------------------------------------------
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
@@ -1552,7 +1555,7 @@ struct X3Args {
 // D > 32. Error against float64 (normal inputs, S 24 / 41 / 63 at D 128 / 32 / 64): 0.96, 1.5 and
 // 1.6e-7 with SEP, 1.5, 2.6 and 2.6e-7 with every product in one chain; attn_scalar 0.95, 1.8 and
 // 2.1e-7.
-template <int D, bool SEP>
+template <int D, bool SEP, bool EXACT>
 __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   static_assert(D == 32 || D == 64 || D == 128, "the split-bf16 fp32 kernel serves D = 32, 64, 128");
   // KT keys per tile: every tile is 8 KiB of fp32 per tensor, 8 channels of one row per thread
@@ -1678,6 +1681,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
         const bf16x8 k3 = *reinterpret_cast<const bf16x8*>(k1p + 2 * TILE + off);
         floatx4& h = hi[NH > 1 && 2 * s >= NS ? 1 : 0];
         h = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q1[s], h, 0, 0, 0);
+        if constexpr (EXACT) {
+          lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k3, q2[s], lo, 0, 0, 0);
+          lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q3[s], lo, 0, 0, 0);
+        }
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k3, q1[s], lo, 0, 0, 0);
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k2, q2[s], lo, 0, 0, 0);
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q3[s], lo, 0, 0, 0);
@@ -1707,9 +1714,10 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
     // every row sees key 0 in its first tile (L >= 1), so m_new is finite from tile 0 on
     const float m_new = grow ? mloc : m_run;
     // the probabilities as three bf16 terms (exact); per key block, in the order
-    // [p2 p2 p1 p1 p3], of which the B operands [p2,p2], [p1,p1], [p1,p3] are 4-register windows
-    typedef uint32_t u32x10 __attribute__((ext_vector_type(10)));
-    u32x10 pq[NKB];
+    // [p2 p2 p1 p1 p3 p2], of which the B operands [p2,p2], [p1,p1], [p1,p3], [p3,p2] are
+    // 4-register windows
+    typedef uint32_t u32x12 __attribute__((ext_vector_type(12)));
+    u32x12 pq[NKB];
     float psum = 0.0f;
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb) {
@@ -1731,8 +1739,8 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
         pw[1][w] = __builtin_amdgcn_perm(u1[2 * w + 1], u1[2 * w], 0x07060302u);
         pw[2][w] = __builtin_amdgcn_perm(u2[2 * w + 1], u2[2 * w], 0x07060302u);
       }
-      pq[kb] = u32x10{pw[1][0], pw[1][1], pw[1][0], pw[1][1], pw[0][0],
-                      pw[0][1], pw[0][0], pw[0][1], pw[2][0], pw[2][1]};
+      pq[kb] = u32x12{pw[1][0], pw[1][1], pw[1][0], pw[1][1], pw[0][0], pw[0][1],
+                      pw[0][0], pw[0][1], pw[2][0], pw[2][1], pw[1][0], pw[1][1]};
     }
     if (__any(grow)) rescale(m_run - m_new);
     l_run += psum;
@@ -1763,6 +1771,13 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
             __builtin_bit_cast(bf16x8, __builtin_shufflevector(vt, vt, 0, 1, 2, 3, 4, 5, 6, 7));
         o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a12, bp11, o[dt], 0, 0, 0);
         floatx4& lo = SEP ? ol[dt] : o[dt];
+        if constexpr (EXACT) {
+          const bf16x8 a23 =
+              __builtin_bit_cast(bf16x8, __builtin_shufflevector(v2, v3, 0, 1, 2, 3, 4, 5, 6, 7));
+          const bf16x8 bp32 =
+              __builtin_bit_cast(bf16x8, __builtin_shufflevector(pq[kb], pq[kb], 8, 9, 10, 11));
+          lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a23, bp32, lo, 0, 0, 0);
+        }
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a31, bp13, lo, 0, 0, 0);
         lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a12, bp22, lo, 0, 0, 0);
       }
@@ -1920,6 +1935,8 @@ bool attention_leaves_planes(const AttnArgs& a, bool scalar) {
          attention_f32_fits(a.B, a.S, a.H, a.KV);
 }
 
+static hipError_t launch_attention_f32x3(const AttnArgs& a, bool exact, hipStream_t st);
+
 hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   if (!attention_scalar_fits(a.B, a.S, a.H)) return hipErrorInvalidValue;
   const unsigned grid = static_cast<unsigned>(a.B * a.S * a.H);
@@ -1931,7 +1948,7 @@ hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   if (a.S >= kX3MinKeys && !a.in_f16 && !a.out_f16 &&
       attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D) &&
       attention_f32_fits(a.B, a.S, a.H, a.KV))
-    return launch_attention_f32(a, st);
+    return launch_attention_f32x3(a, true, st);
   const float scale = a.scale;
   if (!a.in_f16 && !a.out_f16)
     attn_scalar<float, float><<<grid, 64, 0, st>>>(
@@ -1986,9 +2003,55 @@ bool attention_f32_fits(int B, int S, int H, int KV) {
   return geometry_fits(B, KV, G * ((S + 31) / 32), G);
 }
 
+// A shape that attention_f32x3_fits. exact: EXACT arithmetic.
+static hipError_t launch_attention_f32x3(const AttnArgs& a, bool exact, hipStream_t st) {
+  X3Args x{};
+  x.q = static_cast<const float*>(a.q);
+  x.k = static_cast<const float*>(a.k);
+  x.v = static_cast<const float*>(a.v);
+  x.lengths = a.lengths;
+  x.out = static_cast<float*>(a.out);
+  x.B = a.B;
+  x.S = a.S;
+  x.H = a.H;
+  x.KV = a.KV;
+  const double c = static_cast<double>(a.scale) * 1.4426950408889634073599;
+  x.scale_log2 = static_cast<float>(c);
+  x.scale_log2_lo = static_cast<float>(c - static_cast<double>(x.scale_log2));
+  x.bidi = a.bidi;
+  x.shp = f16_shape(a.B, a.S, a.H, a.KV);
+  if (a.planes) x.planes = planes_at(a.planes, a.B * a.S, a.H * a.D);
+  const dim3 grid = sched_grid(a.B, a.KV, (x.shp.nwb + 3) / 4);
+  switch (a.D) {
+    case 32:
+      if (exact)
+        attn_f32x3<32, true, true><<<grid, 256, 0, st>>>(x);
+      else
+        attn_f32x3<32, true, false><<<grid, 256, 0, st>>>(x);
+      break;
+    case 64:
+      if (exact)
+        attn_f32x3<64, true, true><<<grid, 256, 0, st>>>(x);
+      else
+        attn_f32x3<64, true, false><<<grid, 256, 0, st>>>(x);
+      break;
+    default:
+      // the sums of P V apart (SEP) take two workgroups per CU where long rows need the three that
+      // one sum leaves room for: 67 against 83 us at 8 x 512
+      if (exact || a.S < 64)
+        attn_f32x3<128, true, true><<<grid, 256, 0, st>>>(x);
+      else
+        attn_f32x3<128, false, false><<<grid, 256, 0, st>>>(x);
+      break;
+  }
+  return hipGetLastError();
+}
+
 hipError_t launch_attention_f32(const AttnArgs& a, hipStream_t st) {
   if (!a.B || !a.S || !a.H) return hipSuccess;
   if (!attention_f32_fits(a.B, a.S, a.H, a.KV)) return hipErrorInvalidValue;
+  if (attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D)) return launch_attention_f32x3(a, false, st);
+  // shapes beyond attn_f32x3's 32-bit offsets: the fp32-MFMA kernels
   const dim3 grid = mfma_grid(a.B, a.S, a.H, a.KV);
   F32Shape shp;
   shp.G = a.H / a.KV;
@@ -2002,44 +2065,6 @@ hipError_t launch_attention_f32(const AttnArgs& a, hipStream_t st) {
   auto q = static_cast<const float*>(a.q), k = static_cast<const float*>(a.k),
        v = static_cast<const float*>(a.v);
   auto o = static_cast<float*>(a.out);
-  if (attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D)) {
-    X3Args x{};
-    x.q = q;
-    x.k = k;
-    x.v = v;
-    x.lengths = a.lengths;
-    x.out = o;
-    x.B = a.B;
-    x.S = a.S;
-    x.H = a.H;
-    x.KV = a.KV;
-    const double c = static_cast<double>(a.scale) * 1.4426950408889634073599;
-    x.scale_log2 = static_cast<float>(c);
-    x.scale_log2_lo = static_cast<float>(c - static_cast<double>(x.scale_log2));
-    x.bidi = a.bidi;
-    x.shp = f16_shape(a.B, a.S, a.H, a.KV);
-    if (a.planes) x.planes = planes_at(a.planes, a.B * a.S, a.H * a.D);
-    const dim3 grid = sched_grid(a.B, a.KV, (x.shp.nwb + 3) / 4);
-    switch (a.D) {
-      case 32:
-        attn_f32x3<32, true><<<grid, 256, 0, st>>>(x);
-        break;
-      case 64:
-        attn_f32x3<64, true><<<grid, 256, 0, st>>>(x);
-        break;
-      default:
-        // short rows (the calls that ran on attn_scalar) keep the smaller products of P and V
-        // in accumulators of their own, at 184 registers (two workgroups per CU) against 152
-        // (three), which long rows need: 67 against 83 us at 8 x 512
-        if (a.S < 64)
-          attn_f32x3<128, true><<<grid, 256, 0, st>>>(x);
-        else
-          attn_f32x3<128, false><<<grid, 256, 0, st>>>(x);
-        break;
-    }
-    return hipGetLastError();
-  }
-  // shapes beyond attn_f32x3's 32-bit offsets: the fp32-MFMA kernels
   switch (a.D) {
     case 32:
       attn_f32_ring<32><<<grid, 256, 0, st>>>(q, k, v, a.lengths, o, a.B, a.S, a.H, a.KV, sl2, a.bidi, shp);

@@ -147,9 +147,11 @@ constexpr float kLog2e = 1.4426950408889634f;
 
 // An fp32 value splits exactly into three bf16 terms by truncation: b1 = the upper half of x's
 // bits, r1 = x - b1 (exact), b2 = the upper half of r1, b3 = r1 - b2 (at most 8 significant bits,
-// so exactly a bf16). bf16 keeps fp32's exponent range, so no scaling is needed; a product x * y
-// is taken as the six terms b_i c_j with i + j <= 4 (the three dropped ones are below 2^-24 |x y|)
-// and every bf16 product is exact in fp32.
+// so exactly a bf16). bf16 keeps fp32's exponent range, so no scaling is needed, and every bf16
+// product is exact in fp32. |b2| < 2^-7 |x| and |b3| < 2^-15 |x|, both with x's sign: of the nine
+// products b_i c_j of x * y, the six with i + j <= 4 leave out up to 2^-21 |x y|, always with its
+// sign, and the eight with i + j <= 5 up to 2^-30. Where eight are taken, the result keeps what
+// fp32 products keep.
 // x[0..7] -> three packed bf16x8 words (channel pairs (2m, 2m + 1) in word m)
 __device__ __forceinline__ void split3x8(const floatx4& x0, const floatx4& x1, uint4v& p1,
                                          uint4v& p2, uint4v& p3) {

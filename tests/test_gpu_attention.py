@@ -466,3 +466,37 @@ def test_f16_routes_are_deterministic(runtime, route):
         first = attend(runtime, q, k, v, lengths, bidirectional=False, precision="f16")
         second = attend(runtime, q, k, v, lengths, bidirectional=False, precision="f16")
     np.testing.assert_array_equal(first, second)
+
+
+@pytest.mark.parametrize("dim,heads,kv", [(32, 12, 12), (64, 4, 2), (128, 16, 8)])
+@pytest.mark.parametrize("seq", [16, 24, 63, 130])
+def test_scalar_route_keeps_what_fp32_products_keep(runtime, dim, heads, kv, seq):
+    """Operands whose second and third bf16 terms are near their largest, all of one sign: the products
+    of those terms are 2^-21 of a score, and 2^-22 of P V. Two keys, scores 16 and 8 in powers of two
+    (the scale keeps q's bits): the second one's share of the output errs by the scores' rounding,
+    2.6e-6 at most and 6e-8 in the mean in fp32 (without those products 3.4e-6, and 2.3e-6 in the
+    mean). Values of 1.0078124 under random probabilities: 2e-9 in the mean (without, 5e-8)."""
+    rng = np.random.default_rng(dim + seq)
+
+    def near_largest(*shape):  # 1 + 2^-7 less a little
+        return (0x3f80ffff - rng.integers(0, 64, shape, dtype=np.uint32)).view(np.float32)
+
+    scale = np.float32(16 / dim * np.log(2))
+    lengths = np.array([2, 2], np.uint32)
+
+    def errors(q, k, v):
+        got = run(runtime, "attention", [q, k, v, lengths], q.shape, threads=2 * seq * heads * 32,
+                  group_size=32, seq=seq, heads=heads, kv_heads=kv, dim=dim, scale=scale,
+                  bidirectional=True)
+        return got / ref.attention(q, k, v, lengths, scale=float(scale), bidirectional=True) - 1
+
+    q, k = near_largest(2, seq, heads, dim), near_largest(2, seq, kv, dim)
+    k[:, 1] *= 0.5
+    v = np.zeros((2, seq, kv, dim), np.float32)
+    v[:, 1] = 1.0
+    share = errors(q, k, v)
+    assert np.abs(share).max() <= 2.6e-6 and abs(share.mean()) <= 5e-7, (share.max(), share.mean())
+    q = rng.normal(size=q.shape).astype(np.float32)
+    k = (rng.normal(size=k.shape) * 0.1).astype(np.float32)
+    value = errors(q, k, near_largest(2, seq, kv, dim))
+    assert np.abs(value).max() <= 2.6e-7 and abs(value.mean()) <= 1.5e-8, (value.max(), value.mean())
