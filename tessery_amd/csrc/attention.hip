@@ -37,6 +37,43 @@ namespace tessery {
 // Scalar fallback: one wavefront per (token, head), lanes across channels, online softmax over
 // keys. Same arithmetic order per key as kernels.metal:76-103 (dot, scale, running max, rescale).
 // ---------------------------------------------------------------------------------------------
+
+// One row: channels lane + 64 i of its output (C of them cover D) over keys 0 .. end - 1 of one batch
+// row and key/value head. q at the row, k and v at key 0, stride floats from key to key.
+template <int C, typename TIn>
+__device__ __forceinline__ void attend_row(const TIn* q, const TIn* k, const TIn* v, size_t stride,
+                                           int D, int end, float scale, int lane, float (&out)[C]) {
+  float qv[C], acc[C];
+#pragma unroll
+  for (int i = 0; i < C; ++i) {
+    const int c = lane + 64 * i;
+    qv[i] = c < D ? static_cast<float>(q[c]) : 0.0f;
+    acc[i] = 0.0f;
+  }
+  float maximum = -INFINITY, denominator = 0.0f;
+  for (int key = 0; key < end; ++key) {
+    const size_t at = key * stride;
+    float dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int c = lane + 64 * i;
+      if (c < D) dot += qv[i] * static_cast<float>(k[at + c]);
+    }
+    const float score = wave_sum(dot) * scale;
+    const float next = fmaxf(maximum, score);
+    const float correction = expf(maximum - next), prob = expf(score - next);
+    denominator = denominator * correction + prob;
+#pragma unroll
+    for (int i = 0; i < C; ++i) {
+      const int c = lane + 64 * i;
+      if (c < D) acc[i] = acc[i] * correction + prob * static_cast<float>(v[at + c]);
+    }
+    maximum = next;
+  }
+#pragma unroll
+  for (int i = 0; i < C; ++i) out[i] = acc[i] / denominator;
+}
+
 template <typename TIn, typename TOut>
 __global__ __launch_bounds__(64) void attn_scalar(const TIn* __restrict__ q,
                                                   const TIn* __restrict__ k,
@@ -47,41 +84,16 @@ __global__ __launch_bounds__(64) void attn_scalar(const TIn* __restrict__ q,
   const int row = blockIdx.x;  // token * H + head
   const int head = row % H, token = row / H;
   const int b = token / S, pos = token % S;
-  const int kvh = head / (H / KV);
   const int lane = threadIdx.x;
   const int L = static_cast<int>(min(lengths[b], static_cast<uint32_t>(S)));
-  const int end = bidi ? L : min(pos + 1, L);
-  float qv[4], acc[4];
+  const size_t plane = (static_cast<size_t>(b) * S * KV + head / (H / KV)) * D;
+  float y[4];
+  attend_row<4>(q + static_cast<size_t>(row) * D, k + plane, v + plane,
+                static_cast<size_t>(KV) * D, D, bidi ? L : min(pos + 1, L), scale, lane, y);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = lane + 64 * i;
-    qv[i] = c < D ? static_cast<float>(q[static_cast<size_t>(row) * D + c]) : 0.0f;
-    acc[i] = 0.0f;
-  }
-  float maximum = -INFINITY, denominator = 0.0f;
-  for (int key = 0; key < end; ++key) {
-    const size_t kvrow = (static_cast<size_t>(b) * S + key) * KV + kvh;
-    float dot = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = lane + 64 * i;
-      if (c < D) dot += qv[i] * static_cast<float>(k[kvrow * D + c]);
-    }
-    const float score = wave_sum(dot) * scale;
-    const float next = fmaxf(maximum, score);
-    const float correction = expf(maximum - next), prob = expf(score - next);
-    denominator = denominator * correction + prob;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = lane + 64 * i;
-      if (c < D) acc[i] = acc[i] * correction + prob * static_cast<float>(v[kvrow * D + c]);
-    }
-    maximum = next;
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int c = lane + 64 * i;
-    if (c < D) out[static_cast<size_t>(row) * D + c] = static_cast<TOut>(acc[i] / denominator);
+    if (c < D) out[static_cast<size_t>(row) * D + c] = static_cast<TOut>(y[i]);
   }
 }
 
@@ -1543,6 +1555,7 @@ struct X3Args {
   const uint32_t* lengths;
   float* out;
   int B, S, H, KV;
+  float scale;
   float scale_log2, scale_log2_lo;  // scale * log2(e) as the sum of two floats
   int bidi;
   F16Shape shp;
@@ -1813,6 +1826,7 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
   char* const ob = lds + wave * 16 * RS;
   char* const obase = reinterpret_cast<char*>(a.out) +
                       ((static_cast<size_t>(g.b) * S + g.p0) * H + g.head0) * RB;
+  [[maybe_unused]] bool finite = true;
   {
     char* const orow = ob + r * RS;
 #pragma unroll
@@ -1824,11 +1838,38 @@ __global__ __launch_bounds__(256, 2) void attn_f32x3(X3Args a) {
       for (int j = 0; j < 4; ++j) {
         q[j] = o[dt][j] * inv;
         if constexpr (SEP) q[j] = fmaf(fmaf(-q[j], l_row, o[dt][j]), inv, q[j]);
+        if constexpr (EXACT) {
+          uint32_t bits = __float_as_uint(q[j]);
+          asm("" : "+v"(bits));  // this file is compiled for finite values: no float comparison
+          finite = finite && (bits & 0x7f800000u) != 0x7f800000u;
+        }
       }
       *reinterpret_cast<floatx4*>(orow + 4 * (16 * dt + 4 * gq)) = q;
     }
   }
   const int lo = lane / OCH, hmask = (1 << g.hsh) - 1;
+  if constexpr (EXACT) {
+    // A row with a result that isn't finite is made again as attn_scalar makes it: an infinite operand
+    // splits into NaN terms, and a key past the row's last one counts with probability 0, which
+    // its infinite or NaN value turns into NaN. Rows of finite operands hardly ever come here.
+    unsigned long long again = __ballot(!finite);
+    again |= again >> 32;
+    again = (again | again >> 16) & 0xffffu;
+    while (again && g.active) {
+      const int idx = __builtin_ctzll(again);
+      again &= again - 1;
+      const int pos = g.p0 + (idx >> g.hsh);
+      if (pos >= S) continue;
+      constexpr int C = (D + 63) / 64;
+      float y[C];
+      attend_row<C>(qrow + static_cast<size_t>(pos * H + g.head0 + (idx & hmask)) * D, kbase, vbase,
+                    static_cast<size_t>(KV) * D, D, a.bidi ? g.L : min(pos + 1, g.L), a.scale, lane,
+                    y);
+#pragma unroll
+      for (int i = 0; i < C; ++i)
+        if (lane + 64 * i < D) *reinterpret_cast<float*>(ob + idx * RS + 4 * (lane + 64 * i)) = y[i];
+    }
+  }
   const uint32_t voff =
       static_cast<uint32_t>(((lo >> g.hsh) * H + (lo & hmask)) * RB + 16 * (lane % OCH));
   uint4v val[NI];
@@ -2015,6 +2056,7 @@ static hipError_t launch_attention_f32x3(const AttnArgs& a, bool exact, hipStrea
   x.S = a.S;
   x.H = a.H;
   x.KV = a.KV;
+  x.scale = a.scale;
   const double c = static_cast<double>(a.scale) * 1.4426950408889634073599;
   x.scale_log2 = static_cast<float>(c);
   x.scale_log2_lo = static_cast<float>(c - static_cast<double>(x.scale_log2));

@@ -500,3 +500,27 @@ def test_scalar_route_keeps_what_fp32_products_keep(runtime, dim, heads, kv, seq
     k = (rng.normal(size=k.shape) * 0.1).astype(np.float32)
     value = errors(q, k, near_largest(2, seq, kv, dim))
     assert np.abs(value).max() <= 2.6e-7 and abs(value.mean()) <= 1.5e-8, (value.max(), value.mean())
+
+
+@pytest.mark.parametrize("dim,heads,kv", [(32, 12, 12), (64, 4, 2), (128, 16, 8), (128, 3, 1)])
+@pytest.mark.parametrize("seq", [16, 41, 63, 130])
+def test_later_non_finite_tokens_leave_earlier_rows_alone(runtime, dim, heads, kv, seq):
+    """Route "attention", causal: an infinite value or a NaN key of a later token, which no earlier
+    row attends, changes no earlier row; rows that attend it hold what the products give."""
+    rng = np.random.default_rng(seq + dim)
+    q = rng.normal(size=(2, seq, heads, dim)).astype(np.float32)
+    k, v = [rng.normal(size=(2, seq, kv, dim)).astype(np.float32) for _ in range(2)]
+    lengths = np.array([seq, seq - 3], np.uint32)
+
+    want, at = ref.attention(q, k, v, lengths, bidirectional=False), seq - 6
+    k2, v2 = k.copy(), v.copy()
+    v2[0, at, 0, 3], k2[1, at, 0, 1] = np.inf, np.nan
+    v2[:, seq - 3:] = np.nan  # batch row 1's padding, row 0's last tokens
+    got = run(runtime, "attention", [q, k2, v2, lengths], q.shape, threads=2 * seq * heads * 32,
+              group_size=32, seq=seq, heads=heads, kv_heads=kv, dim=dim, scale=dim**-0.5)
+    group = heads // kv
+    check_f32(got[:, :at], want[:, :at])
+    assert np.all(np.isposinf(got[0, at:seq - 3, :group, 3]))
+    assert np.isnan(got[1, at:, :group]).all() and np.isnan(got[0, seq - 3:]).all()
+    others = [c for c in range(dim) if c != 3]
+    check_f32(got[0, at:seq - 3][..., others], want[0, at:seq - 3][..., others])
