@@ -36,6 +36,19 @@ __device__ __forceinline__ float gelu_value(float value) {
   return 0.5f * value * (value < 0.0f ? tail : 2.0f - tail);
 }
 
+// x . w over k inputs as fp32 products: for a result of the split-operand kernels that isn't finite. An
+// infinite operand splits into NaN terms there, and a finite sum may overflow on its way.
+__device__ __forceinline__ float fp32_dot(const float* x, const float* w, int k) {
+  float y = 0.0f;
+  for (int i = 0; i < k; i += 32) {
+    float part = 0.0f;
+    for (int j = i; j < min(i + 32, k); ++j) part = fmaf(x[j], w[j], part);
+    y += part;
+  }
+  return y;
+}
+__device__ __forceinline__ bool is_finite(float y) { return fabsf(y) <= 3.402823466e38f; }
+
 // PARTIAL: workgroup z sums chunks [z * per, (z + 1) * per) only and stores its raw sums to
 // out + z * (row1 - row0) * cols (rows relative to row0), for dense_reduce to add in z order.
 template <bool BIAS, bool GELU, bool PARTIAL>
@@ -337,6 +350,7 @@ __global__ __launch_bounds__(256) void split_dense(SplitArgs a) {
 }
 
 struct PlanesSet {
+  const float* bt;    // the weights as they came
   const float* bias;  // null: none
   float* out;
   int cols;
@@ -345,6 +359,7 @@ struct PlanesSet {
 struct PlanesArgs {
   const uint16_t* x;
   const uint16_t* w;
+  const float* a;  // the inputs as they came
   PlanesSet set[3];
   int count, row0, row1, k;
 };
@@ -478,26 +493,42 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(Plane
   const int col = ct * 64 + 32 * wc + l32;
   if (col >= set.cols) return;
   const float bias = set.bias ? set.bias[col] : 0.0f;
-#pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int r = a.row0 + rt * 64 + 32 * wr + 8 * (e >> 2) + 4 * hh + (e & 3);
-    if (r >= a.row1) continue;
-    float y = first[e] + acc[e];
+  auto row_of = [&](int e) {
+    return a.row0 + rt * 64 + 32 * wr + 8 * (e >> 2) + 4 * hh + (e & 3);
+  };
+  auto store = [&](int r, float y) {
     if (set.bias) y += bias;
     set.out[static_cast<size_t>(r) * set.cols + col] = GELU ? gelu_value(y) : y;
+  };
+  uint32_t again = 0;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const float y = first[e] + acc[e];
+    if (row_of(e) >= a.row1) continue;
+    store(row_of(e), y);
+    again |= is_finite(y) ? 0u : 1u << e;
+  }
+  for (; again; again &= again - 1) {
+    const int r = row_of(__builtin_ctz(again));
+    store(r, fp32_dot(a.a + static_cast<size_t>(r) * a.k, set.bt + static_cast<size_t>(col) * a.k,
+                      a.k));
   }
 }
 
-// Split-K epilogue: out[r][n] = sum over z in order of part[z][r - row0][n] (+ bias, GELU).
+// Split-K epilogue: out[r][n] = sum over z in order of part[z][r - row0][n] (+ bias, GELU). With a (split
+// operands): a result that isn't finite is made again from rows of a and bt.
 template <bool BIAS, bool GELU>
 __global__ __launch_bounds__(256) void dense_reduce(const float* __restrict__ part,
                                                     const float* __restrict__ bias,
                                                     float* __restrict__ out, int row0, int rows,
-                                                    int cols, int splits) {
+                                                    int cols, int splits, const float* a,
+                                                    const float* bt, int k) {
   const size_t i = blockIdx.x * 256ull + threadIdx.x, total = static_cast<size_t>(rows) * cols;
   if (i >= total) return;
   float y = part[i];
   for (int z = 1; z < splits; ++z) y += part[static_cast<size_t>(z) * total + i];
+  if (a && !is_finite(y))
+    y = fp32_dot(a + (static_cast<size_t>(row0) + i / cols) * k, bt + (i % cols) * k, k);
   if (BIAS) y += bias[i % cols];
   out[static_cast<size_t>(row0) * cols + i] = GELU ? gelu_value(y) : y;
 }
@@ -675,6 +706,7 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
   s.k = p.k = j.k;
   s.planes = static_cast<uint16_t*>(scratch.planes);
   p.x = s.planes;
+  p.a = j.a;
   p.row0 = j.row0;
   p.row1 = j.row1;
   p.count = count;
@@ -690,7 +722,7 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
     s.src[i + 1] = jobs[i].bt;
     s.rows[i + 1] = jobs[i].cols;
     s.tiles[i + 1] = (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles
-    p.set[i] = PlanesSet{jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
+    p.set[i] = PlanesSet{jobs[i].bt, jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
     wtiles += s.tiles[i + 1];
   }
   split_dense<<<dim3(static_cast<unsigned>(xtiles + wtiles), (j.k + 63) / 64), 256, 0, st>>>(s);
@@ -744,19 +776,20 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
     else
       matmul_x3<false, false, true, false><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0,
                                                                  row1, cols, k, per);
+    const float* const again = x3_tiles < kX3WideTiles ? a : nullptr;
     const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * cols + 255) / 256);
     if (bias && gelu)
       dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols,
-                                                       x3_splits);
+                                                       x3_splits, again, bt, k);
     else if (bias)
       dense_reduce<true, false><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols,
-                                                        x3_splits);
+                                                       x3_splits, again, bt, k);
     else if (gelu)
       dense_reduce<false, true><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols,
-                                                        x3_splits);
+                                                       x3_splits, again, bt, k);
     else
       dense_reduce<false, false><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols,
-                                                         x3_splits);
+                                                       x3_splits, again, bt, k);
     return hipGetLastError();
   }
   const int splits = scratch ? dense_splits(rows, cols, k, scratch_floats) : 1;
@@ -768,13 +801,17 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
                                                          cols, k, per);
     const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * cols + 255) / 256);
     if (bias && gelu)
-      dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits);
+      dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits, nullptr, nullptr,
+                                                       0);
     else if (bias)
-      dense_reduce<true, false><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits);
+      dense_reduce<true, false><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits, nullptr, nullptr,
+                                                       0);
     else if (gelu)
-      dense_reduce<false, true><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits);
+      dense_reduce<false, true><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits, nullptr, nullptr,
+                                                       0);
     else
-      dense_reduce<false, false><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits);
+      dense_reduce<false, false><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits, nullptr, nullptr,
+                                                       0);
     return hipGetLastError();
   }
   dim3 grid((rows + kDenseRows - 1) / kDenseRows, (cols + 127) / 128);

@@ -477,3 +477,43 @@ def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
               group_size=32, rows=rows, cols=cols, k=k)
     want = x.astype(np.float64) @ w.astype(np.float64).T
     assert np.all(np.abs(got - want) <= 3.5e-7 * want), float(np.abs(got / want - 1).max())
+
+
+@pytest.mark.parametrize("rows,cols,k", [(33, 70, 64), (656, 1152, 384), (65, 384, 1536)])
+@pytest.mark.parametrize("gelu", [False, True])
+def test_non_finite_operands_give_what_fp32_gives(runtime, rows, cols, k, gelu):
+    """Infinities and NaN in x, W and the bias: what sums of fp32 products give (infinities where no
+    NaN and no opposite infinity takes part), and the other rows and columns as ever. So too for
+    values that overflow a bf16 term's neighbour: the largest finite ones."""
+    rng = np.random.default_rng(rows + cols)
+    x = rng.normal(size=(rows, k)).astype(np.float32)
+    w = rng.normal(size=(cols, k)).astype(np.float32)
+    b = rng.normal(size=cols).astype(np.float32)
+    x[1, 5], x[4, 60], x[rows - 1, k - 1] = np.inf, np.nan, -np.inf
+    x[6, 3] = np.finfo(np.float32).max
+    w[:, 3] = np.clip(w[:, 3], -0.5, 0.5)
+    w[7, 2], w[33, 0], b[9] = np.inf, np.nan, -np.inf
+    bufs = [runtime.upload(a) for a in (x, w, np.zeros((rows, cols), np.float32), b)]
+    try:
+        with runtime.command():
+            runtime._dispatch("matmul_bias_f32", bufs, threads=(rows + 3) // 4 * cols * 32,
+                              group_size=32, rows=rows, cols=cols, k=k)
+            if gelu:
+                runtime._dispatch("gelu_f32", [bufs[2]], threads=rows * cols, n=rows * cols)
+        got = runtime.read(bufs[2], (rows, cols))
+    finally:
+        for buf in bufs:
+            buf.close()
+    special = np.zeros((rows, cols), bool)
+    special[[1, 4, 6, rows - 1]] = True
+    special[:, [7, 9, 33]] = True
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = np.array([[np.sum(x[r].astype(np.float64) * w[c]) + b[c] for c in range(cols)]
+                         if special[r].any() else np.zeros(cols) for r in range(rows)])
+        want = np.where(special, want, x.astype(np.float64) @ w.astype(np.float64).T + b)
+        if gelu:
+            want = ref.gelu(want)
+    for r, c in zip(*np.nonzero(special)):
+        v, g = want[r, c], got[r, c]
+        assert (np.isnan(v) and np.isnan(g)) or v == g or abs(g / v - 1) < 1e-5, (r, c, g, v)
+    np.testing.assert_allclose(got[~special], want[~special], atol=2e-4, rtol=5e-5)
