@@ -67,6 +67,7 @@ struct L4Set {
 // silu(gate) * up, out of set 1 (may be null) the up projection.
 struct L4Args {
   Planes x;  // of rows row0 .. row1 - 1
+  const float* rows;  // the whole x as it came
   L4Set set[3];
   int row0, row1, k;
   int vec;      // every out 16-byte aligned and every width a multiple of 4
@@ -246,6 +247,26 @@ __device__ __forceinline__ void multiply_group(const Prepared& w, X x, float xsu
   for (int e = 0; e < 16; ++e) acc[e] = fmaf(w.scale, p[e], acc[e]);
 }
 
+// x . w of one row and column as fp32 products: for a result that isn't finite. An infinite x splits
+// into NaN terms, and so does an infinite scale or bias.
+__device__ __forceinline__ float fp32_dot(const L4Args& a, const L4Set& set, int row, int col) {
+  const int groups = a.k >> 6;
+  const float* x = a.rows + static_cast<size_t>(row) * a.k;
+  const uint32_t* w = set.w + static_cast<size_t>(col) * (a.k >> 3);
+  float y = 0.0f;
+  for (int g = 0; g < groups; ++g) {
+    const size_t at = static_cast<size_t>(col) * groups + g;
+    const float scale = bf16_to_float(set.s[at]), bias = bf16_to_float(set.b[at]);
+    float part = 0.0f;
+    for (int i = 0; i < 64; ++i) {
+      const uint32_t code = w[8 * g + (i >> 3)] >> (4 * (i & 7)) & 15u;
+      part = fmaf(x[64 * g + i], fmaf(static_cast<float>(code), scale, bias), part);
+    }
+    y += part;
+  }
+  return y;
+}
+
 // The end of a tile of BLOCKS column blocks (GATED: the gate's, then the up projection's), one a
 // wavefront: the sums of the SLOTS slots meet in LDS (`red`, free by now), then whole-row stores.
 template <int BLOCKS, int SLOTS, bool GATED>
@@ -275,6 +296,18 @@ __device__ __forceinline__ void store_tile(const L4Args& a, float* red,
     else
       return add(at(0), at(1));
   };
+  auto made_again = [&](const L4Set& set, int row, int c0, floatx4& y) {
+    uint32_t again = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      again |= fabsf(y[j]) <= 3.402823466e38f || c0 + j >= set.cols ? 0u : 1u << j;
+    for (; again; again &= again - 1) {
+      const int at = __builtin_ctz(again);
+      const float dot = fp32_dot(a, set, row, c0 + at);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) y[j] = j == at ? dot : y[j];
+    }
+  };
   auto store = [&](const L4Set& set, int row, int c0, const floatx4& y) {
     float* const dst = set.out + static_cast<size_t>(row) * set.cols + c0;
     if (a.vec && c0 + 4 <= set.cols) {
@@ -289,8 +322,10 @@ __device__ __forceinline__ void store_tile(const L4Args& a, float* red,
     const int row = i / (TC / 4), c = 4 * (i % (TC / 4)), block = c >> 5;
     if (rbase + row >= a.row1) break;  // rows ascend with i
     floatx4 y = sum4(block, row, c & 31);
+    made_again(a.set[GATED ? 0 : first], rbase + row, tile * TC + c, y);
     if constexpr (GATED) {
-      const floatx4 up = sum4(block + BLOCKS / 2, row, c & 31);
+      floatx4 up = sum4(block + BLOCKS / 2, row, c & 31);
+      made_again(a.set[1], rbase + row, tile * TC + c, up);
       if (a.set[1].out) store(a.set[1], rbase + row, tile * TC + c, up);
 #pragma unroll
       for (int j = 0; j < 4; ++j) y[j] = silu_times(y[j], up[j]);
@@ -499,6 +534,7 @@ hipError_t launch_rows(const Linear4Job* jobs, int count, bool gated, const Plan
                        int row1, const Planes& next, hipStream_t st) {
   L4Args a{};
   a.x = x;
+  a.rows = jobs[0].x;
   a.row0 = row0;
   a.row1 = row1;
   a.k = jobs[0].k;

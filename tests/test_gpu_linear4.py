@@ -273,3 +273,27 @@ def test_bias_term_keeps_every_product_of_its_terms(runtime):
     got = project(runtime, [x, packed, scales, biases], m, n, k)
     want = x.astype(np.float64) @ ref.dequantize(packed, scales, biases, k).T
     assert np.all(np.abs(got - want) <= 2.5e-7 * np.abs(want)), float(np.abs(got / want - 1).max())
+
+
+@pytest.mark.parametrize("m", [24, 300, 700])
+def test_non_finite_activations_and_scales_give_what_fp32_gives(runtime, m):
+    """An infinite or NaN activation makes its row, and a non-finite scale or bias its column, what
+    sums of fp32 products give: infinities where no NaN and no opposite infinity takes part."""
+    n, k = 1056, 448
+    x, packed, scales, biases = make(m, m, n, k)
+    x[1, 5], x[4, 100], x[m - 1, k - 1] = np.inf, np.nan, -np.inf
+    scales[7, 2], biases[33, 0], biases[n - 1, 1] = 0x7f80, 0xff80, 0x7fc0
+    got = project(runtime, [x, packed, scales, biases], m, n, k)
+    with np.errstate(invalid="ignore"):
+        codes = ((packed[:, :, None] >> np.arange(0, 32, 4, dtype=np.uint32)) & 15).reshape(n, k)
+        w = (codes * np.repeat(bf16_values(scales), 64, 1)
+             + np.repeat(bf16_values(biases), 64, 1)).astype(np.float64)
+        special = np.zeros((m, n), bool)
+        special[[1, 4, m - 1]] = True
+        special[:, [7, 33, n - 1]] = True
+        for r, c in zip(*np.nonzero(special)):
+            want = np.float32(np.sum(x[r].astype(np.float64) * w[c]))
+            assert (np.isnan(want) and np.isnan(got[r, c])) or got[r, c] == want, (r, c, got[r, c])
+    rows, cols = ~special.all(1), ~special.all(0)
+    np.testing.assert_allclose(got[rows][:, cols], x[rows].astype(np.float64) @ w[cols].T,
+                               atol=2e-4, rtol=5e-5)
