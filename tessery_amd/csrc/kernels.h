@@ -128,8 +128,12 @@ hipError_t launch_linear4_rows(const Linear4Job* jobs, int count, bool gated,
                                hipStream_t st);
 // The same projection for M >= kLinear4HiloRows rows on fp16 MFMA: rows scaled by powers of two
 // and split into hi + lo fp16 halves (about 22 bits), exact codes, fp32 sums. scratch holds the M
-// row scales (scaled: it does already). x and y start at row 0 of the range; N % 128 == 0, K % 64 == 0.
+// row scales (scaled: it does already). x and y start at row 0 of the range.
 constexpr int kLinear4HiloRows = 1024;
+// Whether launch_linear4_hilo_f32 takes the shape (up to K = 8192, M K < 2^30);
+// linear4_rows runs the others.
+bool linear4_hilo_fits(int M, int N, int K, const float* x, const float* y, const float* scratch,
+                       size_t scratch_floats);
 hipError_t launch_linear4_hilo_f32(const float* x, const uint32_t* w, const uint16_t* scales,
                                    const uint16_t* biases, float* y, int M, int N, int K,
                                    float* scratch, size_t scratch_floats, bool scaled,

@@ -561,15 +561,11 @@ hipError_t launch_rows(const Linear4Job* jobs, int count, bool gated, const Plan
   return hipGetLastError();
 }
 
+// large batches: fp16 MFMA on row-scaled hi + lo activations (fp32-grade, several times the fp32 MFMA
+// rate)
 bool runs_hilo(const Linear4Job& j, const float* scratch, size_t scratch_floats) {
-  // large batches: fp16 MFMA on row-scaled hi + lo activations (fp32-grade, several times the
-  // fp32 MFMA rate)
-  const int rows = j.row1 - j.row0;
-  const float* xr = j.x + static_cast<size_t>(j.row0) * j.k;
-  const float* yr = j.out + static_cast<size_t>(j.row0) * j.cols;
-  return rows >= kLinear4HiloRows && j.cols % 128 == 0 && scratch &&
-         static_cast<size_t>(rows) <= scratch_floats &&
-         ((reinterpret_cast<uintptr_t>(xr) | reinterpret_cast<uintptr_t>(yr)) & 15) == 0;
+  return linear4_hilo_fits(j.row1 - j.row0, j.cols, j.k, j.x + static_cast<size_t>(j.row0) * j.k,
+                           j.out + static_cast<size_t>(j.row0) * j.cols, scratch, scratch_floats);
 }
 
 __global__ __launch_bounds__(256) void silu_gate_f32(float* __restrict__ gate,

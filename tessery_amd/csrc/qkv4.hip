@@ -736,7 +736,7 @@ __global__ __launch_bounds__(256, 2) void linear4_hilo(const float* __restrict__
 // 48 KiB of x / weight stages and row sums two workgroups fit a CU up to K = 4096)
 static size_t hilo_sb_bytes(int K) { return static_cast<size_t>(2 * 128 * 2) * (K / 64); }
 
-// x is read and y written in 16-byte pieces
+// x is read and y written in 16-byte pieces; x within 32-bit DMA offsets
 static bool hilo_fits(int M, int N, int K, const float* x, const float* y, const float* scratch,
                       size_t scratch_floats) {
   return K > 0 && K % 64 == 0 && N > 0 && N % 128 == 0 && scratch &&
@@ -745,13 +745,18 @@ static bool hilo_fits(int M, int N, int K, const float* x, const float* y, const
          ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
 }
 
+bool linear4_hilo_fits(int M, int N, int K, const float* x, const float* y, const float* scratch,
+                       size_t scratch_floats) {
+  return M >= kLinear4HiloRows && hilo_fits(M, N, K, x, y, scratch, scratch_floats) &&
+         hilo_sb_bytes(K) <= 64 * 1024;
+}
+
 hipError_t launch_linear4_hilo_f32(const float* x, const uint32_t* w, const uint16_t* scales,
                                    const uint16_t* biases, float* y, int M, int N, int K,
                                    float* scratch, size_t scratch_floats, bool scaled,
                                    hipStream_t st) {
   if (M <= 0) return hipSuccess;
-  if (!hilo_fits(M, N, K, x, y, scratch, scratch_floats) || hilo_sb_bytes(K) > 64 * 1024)
-    return hipErrorInvalidValue;
+  if (!linear4_hilo_fits(M, N, K, x, y, scratch, scratch_floats)) return hipErrorInvalidValue;
   if (!scaled) row_scales_f32<<<(M + 3) / 4, 256, 0, st>>>(x, M, K, scratch);
   dim3 grid((M + 63) / 64, N / 128);
   linear4_hilo<false><<<grid, 256, hilo_sb_bytes(K), st>>>(x, scratch, w, scales, biases, y,

@@ -297,3 +297,16 @@ def test_non_finite_activations_and_scales_give_what_fp32_gives(runtime, m):
     rows, cols = ~special.all(1), ~special.all(0)
     np.testing.assert_allclose(got[rows][:, cols], x[rows].astype(np.float64) @ w[cols].T,
                                atol=2e-4, rtol=5e-5)
+
+
+@pytest.mark.parametrize("k", [8192, 8256])
+def test_large_batch_beyond_the_fp16_kernels_k(runtime, k):
+    """From 1024 rows on, the longest K the fp16-MFMA kernel's scale words leave room for, and the next
+    one, which the split-bf16 kernel takes (in row ranges that fit the planes scratch)."""
+    m, n = 1024, 128
+    x, packed, scales, biases = make(k, m, n, k)
+    got = project(runtime, [x, packed, scales, biases], m, n, k)
+    w = ref.dequantize(packed, scales, biases, k)
+    err = np.abs(got - x.astype(np.float64) @ w.T)
+    bound = 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    assert np.all(err <= bound), float((err / bound).max())
