@@ -673,12 +673,16 @@ static size_t dense_planes_bytes(int64_t rows, int k) {
 // split-K launches and their reduction (656 x 384 outputs of K = 1536: 4.6 + 22 us against 17). Up
 // to 512 tiles of 64 x 128, where matmul_x3 fills the chip without split K and splits nothing
 // beforehand (16384 x 384 outputs of K = 384: 16 + 35 us against 40, 4096 x 1536: 8 + 38 against 42).
-bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
+bool matmul_shape_on_planes(const DenseJob& j, size_t planes_bytes) {
   const int64_t tiles = static_cast<int64_t>((j.row1 - j.row0 + 63) / 64) * ((j.cols + 127) / 128);
-  return scratch.planes && j.k > 0 && j.k % 32 == 0 && j.k <= 512 && j.cols > 0 && tiles < 512 &&
-         dense_planes_bytes(64, j.k) * static_cast<size_t>((j.row1 - j.row0 + 63) / 64 + 3 * ((j.cols + 63) / 64)) <=
-             scratch.planes_bytes &&
+  return j.k > 0 && j.k % 32 == 0 && j.k <= 512 && j.cols > 0 && tiles < 512 &&
+         dense_planes_bytes(64, j.k) * static_cast<size_t>((j.row1 - j.row0 + 63) / 64 +
+                                                           3 * ((j.cols + 63) / 64)) <= planes_bytes &&
          ((reinterpret_cast<uintptr_t>(j.a) | reinterpret_cast<uintptr_t>(j.bt)) & 15) == 0;
+}
+
+bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
+  return scratch.planes && matmul_shape_on_planes(j, scratch.planes_bytes);
 }
 
 hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,

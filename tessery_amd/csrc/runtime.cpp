@@ -581,8 +581,9 @@ bool is_dense(Route r) {
          r == R_MATMUL_BIAS_CHUNK32;
 }
 
-// Scratch of the split-K dense projections and of the fp16-MFMA uint4 ones' row scales, allocated
-// once per runtime on first use (its address never changes, so a captured graph keeps pointing at it).
+// Scratch is allocated by the first op that runs on it and kept for the runtime's life (a captured graph
+// keeps pointing at it). Split-K partial sums of dense projections, and the row scales that the
+// fp16-MFMA uint4 projections read:
 constexpr size_t kDenseScratchFloats = size_t{8} << 20;  // 32 MiB
 // Split operands of the dense projections: at most 512 tiles of 64 x 128 outputs (more run on
 // matmul_x3), which is 96 MiB where they are one column of tiles of K = 512.
@@ -590,46 +591,6 @@ constexpr size_t kDensePlanesBytes = size_t{104} << 20;
 // Each of the two planes scratches: 1023 rows (more run on linear4_hilo) of 3072 inputs, Qwen3's
 // widest, in 18.4 MiB. Others go through it in row ranges.
 constexpr size_t kPlanesBytes = size_t{20} << 20;
-
-bool prepare(Runtime* rt, Route r, const Params& p) {
-  switch (r) {
-    case R_ATTENTION_F16_NORM_ROPE:
-    case R_NORM_ROPE_F16:
-    case R_ROPE:
-      return ensure_rope(rt, p.seq, p.dim, p.theta);
-    case R_MATMUL:
-    case R_MATMUL_TILED:
-    case R_MATMUL_CHUNK32:
-    case R_MATMUL_BIAS:
-    case R_MATMUL_BIAS_CHUNK32:
-    case R_LINEAR4:
-    case R_LINEAR4_TILED:
-    case R_LINEAR4_TAIL:
-    case R_LINEAR4_16X32:
-    case R_LINEAR4_32X32:
-    case R_LINEAR4_SMALL3:
-    case R_GATED4_16X32:
-    case R_GATED4_8X32:
-      if (!rt->dense_scratch &&
-          hipMalloc(&rt->dense_scratch, kDenseScratchFloats * sizeof(float)) != hipSuccess) {
-        rt->dense_scratch = nullptr;
-        return false;
-      }
-      if (is_dense(r) && !rt->dense_planes &&
-          hipMalloc(&rt->dense_planes, kDensePlanesBytes) != hipSuccess) {
-        rt->dense_planes = nullptr;
-        return false;
-      }
-      for (void*& p : rt->planes)
-        if ((is_linear4(r) || is_gated4(r)) && !p && hipMalloc(&p, kPlanesBytes) != hipSuccess) {
-          p = nullptr;
-          return false;
-        }
-      return true;
-    default:
-      return true;
-  }
-}
 
 const RopeTable* rope_of(Runtime* rt, const Params& p) {
   auto it = rt->rope.find(std::make_tuple(p.seq, p.dim, float_bits(p.theta)));
@@ -746,6 +707,42 @@ tessery::DenseScratch dense_scratch(Runtime* rt) {
 // `in` is the planes scratch `slot`, `out` the other one.
 tessery::PlanesScratch planes_scratch(Runtime* rt, int slot) {
   return {rt->planes[slot], rt->planes[1 - slot], kPlanesBytes};
+}
+
+// Allocates *block once; false (and no error left for the launches to find) when it cannot be had.
+template <typename T>
+bool have_scratch(T** block, size_t bytes) {
+  if (!*block && hipMalloc(reinterpret_cast<void**>(block), bytes) != hipSuccess) {
+    *block = nullptr;
+    (void)hipGetLastError();
+  }
+  return *block;
+}
+
+// What op needs beside its buffers. A scratch that another kernel does without is left out when it
+// cannot be had.
+bool prepare(Runtime* rt, const Op& op) {
+  const Params& p = op.p;
+  const size_t sums_bytes = kDenseScratchFloats * sizeof(float);
+  if (op.route == R_ATTENTION_F16_NORM_ROPE || op.route == R_NORM_ROPE_F16 || op.route == R_ROPE)
+    return ensure_rope(rt, p.seq, p.dim, p.theta);
+  tessery::DenseJob dense;
+  if (dense_job(op, &dense)) {
+    if (tessery::matmul_shape_on_planes(dense, kDensePlanesBytes))
+      (void)have_scratch(&rt->dense_planes, kDensePlanesBytes);
+    return have_scratch(&rt->dense_scratch, sums_bytes);
+  }
+  tessery::Linear4Job job, gated[2];
+  if (linear4_job(op, &job)) {
+    if (job.row1 - job.row0 >= tessery::kLinear4HiloRows &&
+        have_scratch(&rt->dense_scratch, sums_bytes) &&
+        !tessery::linear4_on_rows(job, rt->dense_scratch, kDenseScratchFloats))
+      return true;
+  } else if (!gated4_jobs(op, gated)) {
+    return true;
+  }
+  (void)have_scratch(&rt->planes[1], kPlanesBytes);
+  return have_scratch(&rt->planes[0], kPlanesBytes);
 }
 
 // What a launch leaves and finds beside its op's buffers: where a rms_norm or an attention also puts
@@ -1025,9 +1022,9 @@ int mi_dispatch(void* runtime, const char* name, void** buffers, uint32_t count,
     sizes[i] = b->size;
   }
   if (!validate(r, p, threads, group, sizes, count, nbuf)) return 1;
-  if (hipSetDevice(rt->device) != hipSuccess || !prepare(rt, r, p)) return 1;
   Op op;
   make_op(r, p, threads, group, ptrs, sizes, count, &op);
+  if (hipSetDevice(rt->device) != hipSuccess || !prepare(rt, op)) return 1;
   return queue_op(rt, op) ? 0 : 1;
 }
 
@@ -1422,7 +1419,7 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
                           ready.k == static_cast<uint64_t>(j.k);
     const int slot = prepared ? ready.slot : 0;
     *taken = p.end - first;
-    const bool keep = p.gated && j.row0 == 0 && j.out != j.x &&
+    const bool keep = p.gated && j.row0 == 0 && j.out != j.x && rt->planes[1 - slot] &&
                       tessery::planes_bytes(j.row1, j.k) <= kPlanesBytes &&
                       reads_planes(rt, p.end, last, j.out, j.row1, j.cols);
     // its scratch is another one: the row scales of its input stay
@@ -1815,8 +1812,8 @@ int mi_plan_run(void* runtime, void* plan, void** buffers, uint32_t count) {
     if (!b || b->owner != rt || b->size != pl->sizes[i]) return 1;
   }
   if (hipSetDevice(rt->device) != hipSuccess) return 1;
-  for (const auto& po : pl->ops)
-    if (!prepare(rt, po.route, po.p)) return 1;
+  std::vector<Op> ops;
+  ops.reserve(pl->ops.size());
   for (const auto& po : pl->ops) {
     void* ptrs[kMaxBuffers] = {};
     uint64_t sizes[kMaxBuffers] = {};
@@ -1827,8 +1824,10 @@ int mi_plan_run(void* runtime, void* plan, void** buffers, uint32_t count) {
     }
     Op op;
     make_op(po.route, po.p, po.threads, po.group, ptrs, sizes, po.count, &op);
-    rt->ops.push_back(op);
+    if (!prepare(rt, op)) return 1;
+    ops.push_back(op);
   }
+  rt->ops.insert(rt->ops.end(), ops.begin(), ops.end());
   Segment seg{rt->ops.size() - pl->ops.size(), pl->ops.size(), pl, {}};
   for (uint32_t i = 0; i < count; ++i) seg.key.push_back(static_cast<Buffer*>(buffers[i])->ptr);
   rt->segments.push_back(std::move(seg));

@@ -316,3 +316,43 @@ def test_launcher_limits_are_rejected_at_dispatch(runtime, case):
     finally:
         for b in bufs:
             b.close()
+
+
+@pytest.mark.parametrize("route,rows,k,mib", [("matmul_f32", 5, 1536, 32), ("matmul_f32", 5, 384, 136),
+                                              ("linear4", 5, 128, 40), ("linear4", 1024, 128, 32)])
+def test_projections_take_the_scratch_they_run_on(runtime, route, rows, k, mib):
+    """A runtime's first projection takes the device memory its own kernel works in: 32 MiB of partial
+    sums or row scales, 104 MiB of split operands only for the dense shapes that use them, 40 MiB of
+    split activations only for uint4 ones of under 1024 rows."""
+    import ctypes
+
+    from tessery_amd import HipRuntime
+    from tessery_amd.runtime import library_path
+
+    library, cols = ctypes.CDLL(str(library_path())), 128
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert library.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    def project(rt):
+        if route == "matmul_f32":
+            bufs = [rt.buffer(rows * k * 4), rt.buffer(cols * k * 4), rt.buffer(rows * cols * 4)]
+        else:
+            scales = cols * (k // 64) * 2
+            bufs = [rt.buffer(rows * k * 4), rt.buffer(cols * k // 2), rt.buffer(scales),
+                    rt.buffer(scales), rt.buffer(rows * cols * 4)]
+        before = free_bytes()
+        with rt.command():
+            rt._dispatch(route, bufs, threads=(rows + 3) // 4 * cols * 32, group_size=32, rows=rows,
+                         cols=cols, k=k)
+        taken = before - free_bytes()
+        for b in bufs:
+            b.close()
+        return taken
+
+    project(runtime)  # the kernels are loaded by now
+    with HipRuntime() as fresh:
+        # small buffers share allocator blocks of up to 2 MiB with the scratch
+        assert abs(project(fresh) - (mib << 20)) <= 4 << 20
