@@ -307,15 +307,14 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
 // [row tile of 32][k-step of 16][term][lane][8], lane = row % 32 + 32 h holding inputs
 // 16 step + 8 h .. + 7. matmul_planes then only copies operands to LDS (global_load_lds_dwordx4:
 // whole KiB pieces, read back by lane, no bank conflicts) and multiplies, all of K in one workgroup:
-// no partial sums, and q, k and v in one launch. Measured, q, k and v of 656 rows: 3.4 + 12.3 us, 42
-// as three split-K launches of matmul_f32 with their reductions; of 4096: 5 + 28 us, 76 on matmul_x3.
+// no partial sums, and q, k and v in one launch. Measured, q, k and v of 1024 rows of 384: 19.3 us, 47.5
+// as three split-K launches with their reductions; of 4096: 36.8 us, 72.0 on matmul_x3.
 //
 // Eight products, all but that of the two smallest terms (below 2^-30 of the whole): nothing is lost
 // against fp32 products. K order: two halves, each with its leading products in one sum and the seven
 // smaller ones in another (only the leading ones round at the magnitude of the result), added at
-// the end. It is
-// the same for every tile shape, so a row's bits depend on no other row and on no projection
-// beside it.
+// the end. It is the same for every tile shape, so a row's bits depend on no other row and on no
+// projection beside it.
 constexpr int kDenseStep = 3 * 64 * 8;  // bf16 words of a row tile's k-step
 
 struct SplitArgs {
@@ -364,21 +363,53 @@ struct PlanesArgs {
   int count, row0, row1, k;
 };
 
-// Tile 64 x 64, KS slots (one a half of K; KS = 1 takes them in turn) of 4 wavefronts of 32 x 32 each.
-// Two LDS stages of a 32-input chunk. While a chunk's products run, its wavefront reads the
-// operands of the next one from LDS and copies those of the one after, one instruction between two
-// products (issued together they cost as much as the products). Bound: few tiles, the issue and
-// latency of a chunk's copies; many, L2 (13 TB/s at 16384 rows). Tiles of 64 x 128 and 128 x 128,
+// The outputs of a 32 x 32 tile at `row`, `col` of set `which`, from the sums over the halves of K.
+template <bool GELU>
+__device__ __forceinline__ void store_halves(const PlanesArgs& a, int which, int row, int col,
+                                             const floatx16& first, const floatx16& second) {
+  const PlanesSet set = a.set[which];
+  const int lane = threadIdx.x & 63, hh = lane >> 5;
+  col += lane & 31;
+  if (col >= set.cols) return;
+  const float bias = set.bias ? set.bias[col] : 0.0f;
+  auto row_of = [&](int e) { return row + 8 * (e >> 2) + 4 * hh + (e & 3); };
+  auto store = [&](int r, float y) {
+    if (set.bias) y += bias;
+    set.out[static_cast<size_t>(r) * set.cols + col] = GELU ? gelu_value(y) : y;
+  };
+  uint32_t again = 0;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const float y = first[e] + second[e];
+    if (row_of(e) >= a.row1) continue;
+    store(row_of(e), y);
+    again |= is_finite(y) ? 0u : 1u << e;
+  }
+  for (; again; again &= again - 1) {
+    const int r = row_of(__builtin_ctz(again));
+    store(r, fp32_dot(a.a + static_cast<size_t>(r) * a.k, set.bt + static_cast<size_t>(col) * a.k,
+                      a.k));
+  }
+}
+
+// The products of two operands' terms that are taken, the smallest first; the last one leads.
+__device__ constexpr int kTerms[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2},
+                                         {1, 2}, {1, 0}, {0, 1}, {0, 0}};
+
+// Tile 64 x 64, 4 wavefronts of 32 x 32 each. Two LDS stages of a 32-input chunk. While a chunk's
+// products run, its wavefront reads the operands of the next one from LDS and copies those of the
+// one after, one instruction between two products (issued together they cost as much as the
+// products). Bound: few tiles, the issue and latency of a chunk's copies; many, L2 (13 TB/s at 16384
+// rows). Tiles of 64 x 128 and 128 x 128,
 // which ask L2 for less, or more stages leave too few wavefronts on a CU to hide either: 16384 x
 // 1152 outputs 97 and 194 us, 130 with three stages, against 94. Workgroups are numbered so that
 // an XCD takes all columns of a row tile in turn, from its own L2.
-template <int KS, bool GELU>
-__global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(PlanesArgs a,
-                                                                          int row_tiles,
-                                                                          int col_tiles) {
+template <bool GELU>
+__global__ __launch_bounds__(256, 3) void matmul_planes(PlanesArgs a, int row_tiles,
+                                                        int col_tiles) {
   constexpr int STAGE = 24 * 512;  // bf16 words: 12 KiB of x, then 12 KiB of weights
   constexpr int COPIES = 6, READS = 12;
-  __shared__ __attribute__((aligned(1024))) uint16_t mem[2 * KS * STAGE];
+  __shared__ __attribute__((aligned(1024))) uint16_t mem[2 * STAGE];
   const int block = blockIdx.x, turn = block >> 3;
   const int rt = (block & 7) + 8 * (turn / col_tiles);
   if (rt >= row_tiles) return;
@@ -389,24 +420,24 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(Plane
   }
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5;
-  const int slot = wave >> 2, w4 = wave & 3, wr = w4 >> 1, wc = w4 & 1;
+  const int wr = wave >> 1, wc = wave & 1;
   const int ksteps = a.k >> 4, chunks = a.k >> 5, half = chunks >> 1;
   // A wavefront copies the 6 KiB of one operand tile: row tiles 0 and 1, column tiles 0 and 1.
   // Row tiles past the last one read it again (their rows aren't stored).
   const int last = (a.row1 - a.row0 - 1) >> 5;
-  const int from = w4 < 2 ? min(2 * rt + w4, last) : a.set[which].tile0 + 2 * ct + w4 - 2;
+  const int from = wave < 2 ? min(2 * rt + wave, last) : a.set[which].tile0 + 2 * ct + wave - 2;
   const uint16_t* const src =
-      (w4 < 2 ? a.x : a.w) + static_cast<size_t>(from) * ksteps * kDenseStep;
+      (wave < 2 ? a.x : a.w) + static_cast<size_t>(from) * ksteps * kDenseStep;
   auto copy = [&](int i, int buf, int chunk) {
     dma16_at(src + static_cast<size_t>(chunk) * (2 * kDenseStep) + i * 512, 16u * lane,
-             reinterpret_cast<_Float16*>(mem + (buf * KS + slot) * STAGE + (6 * w4 + i) * 512));
+             reinterpret_cast<_Float16*>(mem + buf * STAGE + (6 * wave + i) * 512));
   };
   struct Operands {
     bf16x8 x[2][3], y[2][3];
   };
   // read i of a chunk's operands, in the order the products need them: terms (2, 0), (1, 1), (0, 2)
   auto read = [&](Operands& f, int i, int buf) {
-    const uint16_t* const at = mem + (buf * KS + slot) * STAGE + lane * 8;
+    const uint16_t* const at = mem + buf * STAGE + lane * 8;
     const int t = i / 4, ks = (i >> 1) & 1;
     if (i & 1)
       f.y[ks][t] = *reinterpret_cast<const bf16x8*>(at + ((2 + wc) * 6 + ks * 3 + t) * 512);
@@ -417,41 +448,35 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(Plane
   floatx16 hi, lo, first;
 #pragma unroll
   for (int e = 0; e < 16; ++e) hi[e] = lo[e] = first[e] = 0.0f;
-  const int begin = slot ? half : 0, end = KS == 2 && !slot ? half : chunks;
-  const int steps = KS == 2 ? chunks - half : chunks;  // of the longer slot
   Operands even, odd;
-  if (begin < end) {
 #pragma unroll
-    for (int i = 0; i < COPIES; ++i) copy(i, 0, begin);
-  }
+  for (int i = 0; i < COPIES; ++i) copy(i, 0, 0);
   wait_vmcnt<0>();
   stage_barrier();
-  if (begin + 1 < end) {
+  if (chunks > 1) {
 #pragma unroll
-    for (int i = 0; i < COPIES; ++i) copy(i, 1, begin + 1);
+    for (int i = 0; i < COPIES; ++i) copy(i, 1, 1);
   }
 #pragma unroll
   for (int i = 0; i < READS; ++i) read(even, i, 0);
-  // chunk begin + step from `now`; `next` takes the one after
+  // chunk `step` from `now`; `next` takes the one after
   auto chunk = [&](int step, int buf, const Operands& now, Operands& next) {
     // the next chunk's copy has landed, and every wavefront has read this one's stage
     wait_vmcnt<0>();
     wait_lgkmcnt<0>();
     stage_barrier();
-    if (begin + step >= end) return;
-    const bool more = begin + step + 2 < end;
-    constexpr int term[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2}, {1, 2}, {1, 0}, {0, 1}, {0, 0}};
+    const bool more = step + 2 < chunks;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int ks = i & 1, t = i >> 1;
       floatx16& c = t < 7 ? lo : hi;
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][term[t][0]], now.y[ks][term[t][1]], c,
-                                                  0, 0, 0);
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][kTerms[t][0]], now.y[ks][kTerms[t][1]],
+                                                  c, 0, 0, 0);
       if (i < READS) read(next, i, buf ^ 1);  // stale data after the last chunk, unused
-      if (more && i < 2 * COPIES && (i & 1)) copy(i >> 1, buf, begin + step + 2);
+      if (more && i < 2 * COPIES && (i & 1)) copy(i >> 1, buf, step + 2);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (KS == 1 && step + 1 == half) {
+    if (step + 1 == half) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) {
         first[e] = hi[e] + lo[e];
@@ -459,60 +484,122 @@ __global__ __launch_bounds__(256 * KS, KS == 1 ? 3 : 2) void matmul_planes(Plane
       }
     }
   };
-  for (int step = 0; step < steps; step += 2) {
+  for (int step = 0; step < chunks; step += 2) {
     chunk(step, 0, even, odd);
-    if (step + 1 < steps) chunk(step + 1, 1, odd, even);
+    if (step + 1 < chunks) chunk(step + 1, 1, odd, even);
   }
   floatx16 acc;
 #pragma unroll
   for (int e = 0; e < 16; ++e) acc[e] = hi[e] + lo[e];
-  // the last chunk's reads ahead have landed before the kernel ends or reuses their stage
-  wait_lgkmcnt<0>();
+  wait_lgkmcnt<0>();  // the last chunk's reads ahead have landed before the kernel ends
+  store_halves<GELU>(a, which, a.row0 + rt * 64 + 32 * wr, ct * 64 + 32 * wc, first, acc);
+}
 
-  if constexpr (KS == 2) {
-    // the second half's sums through LDS to the first slot
-    stage_barrier();  // the stages are free
-    floatx4* const sums = reinterpret_cast<floatx4*>(mem) + w4 * 256 + lane;
+// The same for few tiles, with the same bits, straight from the operands as they came. A workgroup makes
+// a tile of 32 x 32, a wavefront one half of K; each splits the operands of the next chunk in
+// registers beside the products of this one, loaded a chunk before. Bound: the latency of that chain
+// (deeper loads ahead only lengthen its start: 9.1 us for 24 to 656 rows of 384 x 384 with four chunks
+// ahead, 8.3 with two, 9.4 with splits and products in turn). Per launch, against the pass that splits
+// and matmul_planes, and matmul_f32 with its reduction: 24 x 384 outputs of K = 384 7.7, 11.6 and 8.8
+// us, 128 x 1536 8.3, 16.3 and 11.3, 64 x 512 of K = 512 9.1, 14.5 and 10.3; q, k and v of 128 rows
+// 8.5, 15.2 and 29.4.
+template <bool GELU>
+__global__ __launch_bounds__(128) void matmul_direct(PlanesArgs a) {
+  constexpr int DEPTH = 2;  // chunks loaded ahead
+  __shared__ __attribute__((aligned(16))) float sums[4 * 64 * 4];
+  int ct = blockIdx.y, which = 0;
+  while (which + 1 < a.count && ct >= (a.set[which].cols + 31) / 32) {
+    ct -= (a.set[which].cols + 31) / 32;
+    ++which;
+  }
+  const int tid = threadIdx.x, half = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, l32 = lane & 31, hh = lane >> 5, k = a.k;
+  const int row = a.row0 + 32 * static_cast<int>(blockIdx.x), chunks = k >> 5;
+  const int begin = half ? chunks >> 1 : 0, end = half ? chunks : chunks >> 1;
+  // rows and columns past the last one repeat it (they aren't stored)
+  const float* const x = a.a + static_cast<size_t>(min(row + l32, a.row1 - 1)) * k + 8 * hh;
+  const float* const w =
+      a.set[which].bt + static_cast<size_t>(min(32 * ct + l32, a.set[which].cols - 1)) * k + 8 * hh;
+
+  struct Chunk {
+    floatx4 x[2][2], w[2][2];
+  };
+  auto load = [&](Chunk& c, int at) {
+    const int from = 32 * min(at, end - 1);  // past the last one it again, unused
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (slot) sums[q * 64] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-    wait_lgkmcnt<0>();
-    stage_barrier();
-    if (slot) return;
+    for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const floatx4 second = sums[q * 64];
+      for (int i = 0; i < 2; ++i) {
+        c.x[ks][i] = *reinterpret_cast<const floatx4*>(x + from + 16 * ks + 4 * i);
+        c.w[ks][i] = *reinterpret_cast<const floatx4*>(w + from + 16 * ks + 4 * i);
+      }
+  };
+  floatx16 hi, lo;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        first[4 * q + j] = acc[4 * q + j];
-        acc[4 * q + j] = second[j];
+  for (int e = 0; e < 16; ++e) hi[e] = lo[e] = 0.0f;
+  struct Operands {
+    bf16x8 x[2][3], w[2][3];
+  };
+  auto split = [&](Operands& o, const Chunk& c) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      uint4v t[3];
+      split3x8(c.x[ks][0], c.x[ks][1], t[0], t[1], t[2]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) o.x[ks][i] = __builtin_bit_cast(bf16x8, t[i]);
+      split3x8(c.w[ks][0], c.w[ks][1], t[0], t[1], t[2]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) o.w[ks][i] = __builtin_bit_cast(bf16x8, t[i]);
+    }
+  };
+  auto multiply = [&](const Operands& o) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int ks = i & 1, t = i >> 1;
+      floatx16& sum = t < 7 ? lo : hi;
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.x[ks][kTerms[t][0]], o.w[ks][kTerms[t][1]],
+                                                    sum, 0, 0, 0);
+    }
+  };
+  if (begin < end) {
+    Chunk ring[DEPTH];
+    Operands now[2];
+#pragma unroll
+    for (int i = 0; i < DEPTH; ++i) load(ring[i], begin + i);
+    split(now[0], ring[0]);
+    for (int at = begin; at < end; at += DEPTH) {
+#pragma unroll
+      for (int i = 0; i < DEPTH; ++i) {
+        if (at + i >= end) break;
+        load(ring[i], at + i + DEPTH);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(now[i & 1]);
+        split(now[(i + 1) & 1], ring[(i + 1) % DEPTH]);
+#pragma unroll
+        for (int m = 0; m < 16; ++m) {  // an MFMA, then the splitting that fits beside it
+          __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 11, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
     }
   }
-  const PlanesSet set = a.set[which];
-  const int col = ct * 64 + 32 * wc + l32;
-  if (col >= set.cols) return;
-  const float bias = set.bias ? set.bias[col] : 0.0f;
-  auto row_of = [&](int e) {
-    return a.row0 + rt * 64 + 32 * wr + 8 * (e >> 2) + 4 * hh + (e & 3);
-  };
-  auto store = [&](int r, float y) {
-    if (set.bias) y += bias;
-    set.out[static_cast<size_t>(r) * set.cols + col] = GELU ? gelu_value(y) : y;
-  };
-  uint32_t again = 0;
+  floatx16 acc, second;
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const float y = first[e] + acc[e];
-    if (row_of(e) >= a.row1) continue;
-    store(row_of(e), y);
-    again |= is_finite(y) ? 0u : 1u << e;
+  for (int e = 0; e < 16; ++e) acc[e] = hi[e] + lo[e];
+  floatx4* const at = reinterpret_cast<floatx4*>(sums) + lane;
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (half) at[q * 64] = floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+  __syncthreads();
+  if (half) return;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const floatx4 s = at[q * 64];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) second[4 * q + j] = s[j];
   }
-  for (; again; again &= again - 1) {
-    const int r = row_of(__builtin_ctz(again));
-    store(r, fp32_dot(a.a + static_cast<size_t>(r) * a.k, set.bt + static_cast<size_t>(col) * a.k,
-                      a.k));
-  }
+  store_halves<GELU>(a, which, row, 32 * ct, acc, second);
 }
 
 // Split-K epilogue: out[r][n] = sum over z in order of part[z][r - row0][n] (+ bias, GELU). With a (split
@@ -652,7 +739,6 @@ static int x3_split_count(int rows, int cols, int k, int tiles, size_t scratch_f
   return splits;
 }
 
-template <int KS>
 static void run_planes(const PlanesArgs& a, bool gelu, hipStream_t st) {
   const int row_tiles = (a.row1 - a.row0 + 63) / 64;
   int col_tiles = 0;
@@ -660,9 +746,9 @@ static void run_planes(const PlanesArgs& a, bool gelu, hipStream_t st) {
   const unsigned grid = 8u * static_cast<unsigned>((row_tiles + 7) / 8) *
                         static_cast<unsigned>(col_tiles);
   if (gelu)
-    matmul_planes<KS, true><<<grid, 256 * KS, 0, st>>>(a, row_tiles, col_tiles);
+    matmul_planes<true><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
   else
-    matmul_planes<KS, false><<<grid, 256 * KS, 0, st>>>(a, row_tiles, col_tiles);
+    matmul_planes<false><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
 }
 
 static size_t dense_planes_bytes(int64_t rows, int k) {
@@ -673,7 +759,7 @@ static size_t dense_planes_bytes(int64_t rows, int k) {
 // split-K launches and their reduction (656 x 384 outputs of K = 1536: 4.6 + 22 us against 17). Up
 // to 512 tiles of 64 x 128, where matmul_x3 fills the chip without split K and splits nothing
 // beforehand (16384 x 384 outputs of K = 384: 16 + 35 us against 40, 4096 x 1536: 8 + 38 against 42).
-bool matmul_shape_on_planes(const DenseJob& j, size_t planes_bytes) {
+static bool split_shape(const DenseJob& j, size_t planes_bytes) {
   const int64_t tiles = static_cast<int64_t>((j.row1 - j.row0 + 63) / 64) * ((j.cols + 127) / 128);
   return j.k > 0 && j.k % 32 == 0 && j.k <= 512 && j.cols > 0 && tiles < 512 &&
          dense_planes_bytes(64, j.k) * static_cast<size_t>((j.row1 - j.row0 + 63) / 64 +
@@ -681,8 +767,24 @@ bool matmul_shape_on_planes(const DenseJob& j, size_t planes_bytes) {
          ((reinterpret_cast<uintptr_t>(j.a) | reinterpret_cast<uintptr_t>(j.bt)) & 15) == 0;
 }
 
+// matmul_direct reads its operands while other workgroups write outputs.
+static bool output_apart(const DenseJob& j) { return j.out != j.a && j.out != j.bt; }
+
+// matmul_direct up to this many tiles of 32 x 32, matmul_planes after split_dense beyond: 1008 tiles
+// (656 x 1536 outputs of K = 384) 19.3 and 20.5 us, 1152 (three times 1024 x 384) 23.2 and 19.3, 1536
+// (1024 x 1536) 27.3 and 21.3.
+constexpr int64_t kDirectTiles = 1024;
+
+static int64_t direct_tiles(const DenseJob& j) {
+  return static_cast<int64_t>((j.row1 - j.row0 + 31) / 32) * ((j.cols + 31) / 32);
+}
+
+bool matmul_reads_planes(const DenseJob& j, size_t planes_bytes) {
+  return split_shape(j, planes_bytes) && (3 * direct_tiles(j) > kDirectTiles || !output_apart(j));
+}
+
 bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
-  return scratch.planes && matmul_shape_on_planes(j, scratch.planes_bytes);
+  return split_shape(j, scratch.planes_bytes) && (scratch.planes || output_apart(j));
 }
 
 hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
@@ -695,10 +797,33 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
       return hipErrorInvalidValue;
   if (j.row1 <= j.row0) return hipSuccess;
   const int rows = j.row1 - j.row0;
+  PlanesArgs p{};
+  p.a = j.a;
+  p.row0 = j.row0;
+  p.row1 = j.row1;
+  p.k = j.k;
+  p.count = count;
+  int wtiles = 0, columns = 0;
+  int64_t tiles = 0;
+  bool direct = true;
+  for (int i = 0; i < count; ++i) {
+    p.set[i] = PlanesSet{jobs[i].bt, jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
+    wtiles += (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles
+    columns += (jobs[i].cols + 31) / 32;
+    tiles += direct_tiles(jobs[i]);
+    direct = direct && output_apart(jobs[i]);
+  }
+  const int xtiles = (rows + 31) / 32;
+  if (!scratch.planes || (direct && tiles <= kDirectTiles)) {
+    const dim3 grid(static_cast<unsigned>(xtiles), static_cast<unsigned>(columns));
+    if (gelu)
+      matmul_direct<true><<<grid, 128, 0, st>>>(p);
+    else
+      matmul_direct<false><<<grid, 128, 0, st>>>(p);
+    return hipGetLastError();
+  }
   // every job fits the scratch with three times its own weights, so three of equal width do
-  size_t bytes = dense_planes_bytes((rows + 31) / 32 * 32, j.k);
-  for (int i = 0; i < count; ++i) bytes += dense_planes_bytes((jobs[i].cols + 63) / 64 * 64, j.k);
-  if (bytes > scratch.planes_bytes) {
+  if (dense_planes_bytes(32 * (static_cast<int64_t>(xtiles) + wtiles), j.k) > scratch.planes_bytes) {
     for (int i = 0; i < count; ++i) {
       const hipError_t e = launch_matmul_planes(jobs + i, 1, gelu, scratch, st);
       if (e != hipSuccess) return e;
@@ -706,36 +831,22 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
     return hipSuccess;
   }
   SplitArgs s{};
-  PlanesArgs p{};
-  s.k = p.k = j.k;
+  s.k = j.k;
   s.planes = static_cast<uint16_t*>(scratch.planes);
-  p.x = s.planes;
-  p.a = j.a;
-  p.row0 = j.row0;
-  p.row1 = j.row1;
-  p.count = count;
   s.count = count + 1;
-  const int xtiles = (rows + 31) / 32;
   s.src[0] = j.a;
   s.row0[0] = j.row0;
   s.rows[0] = rows;
   s.tiles[0] = xtiles;
+  p.x = s.planes;
   p.w = s.planes + static_cast<size_t>(xtiles) * (j.k / 16) * kDenseStep;
-  int wtiles = 0;
   for (int i = 0; i < count; ++i) {
     s.src[i + 1] = jobs[i].bt;
     s.rows[i + 1] = jobs[i].cols;
-    s.tiles[i + 1] = (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles
-    p.set[i] = PlanesSet{jobs[i].bt, jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
-    wtiles += s.tiles[i + 1];
+    s.tiles[i + 1] = (jobs[i].cols + 63) / 64 * 2;
   }
   split_dense<<<dim3(static_cast<unsigned>(xtiles + wtiles), (j.k + 63) / 64), 256, 0, st>>>(s);
-  // under 128 tiles the CUs are not full: both halves of K at once (656 x 384 outputs 8.5 us, 10.1 in
-  // turn; 656 x 1152, 198 tiles, 16.1 and 12.3)
-  if (static_cast<int64_t>((rows + 63) / 64) * (wtiles / 2) < 128)
-    run_planes<2>(p, gelu, st);
-  else
-    run_planes<1>(p, gelu, st);
+  run_planes(p, gelu, st);
   return hipGetLastError();
 }
 

@@ -728,7 +728,7 @@ bool prepare(Runtime* rt, const Op& op) {
     return ensure_rope(rt, p.seq, p.dim, p.theta);
   tessery::DenseJob dense;
   if (dense_job(op, &dense)) {
-    if (tessery::matmul_shape_on_planes(dense, kDensePlanesBytes))
+    if (tessery::matmul_reads_planes(dense, kDensePlanesBytes))
       (void)have_scratch(&rt->dense_planes, kDensePlanesBytes);
     return have_scratch(&rt->dense_scratch, sums_bytes);
   }

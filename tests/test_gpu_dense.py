@@ -397,12 +397,15 @@ def test_plan_replay_graphs_match_eager(monkeypatch, graphs):
                                rtol=5e-5)
 
 
-# Rows and columns at the edges of the 64 x 64 tiles, under and over 128 of them (both halves of K at
-# once, or in turn), K of 1, 2, 3, 5, 12 and 16 chunks (empty and uneven halves); then, past K = 512,
-# split K at few tiles (from 8 chunks) and the shapes that stay on the fp32 kernel.
+# Rows and columns at the edges of the 32 x 32 tiles of the direct kernel and, beyond 1024 of those, of
+# the 64 x 64 ones of operands split beforehand; K of 1, 2, 3, 5, 12 and 16 chunks (empty and uneven
+# halves); then, past K = 512, split K at few tiles (from 8 chunks) and the shapes that stay on the
+# fp32 kernel.
 @pytest.mark.parametrize("rows,cols,k", [(1, 1, 32), (31, 33, 64), (64, 64, 96), (65, 129, 160),
                                          (33, 384, 384), (543, 1152, 384), (1000, 384, 384),
-                                         (129, 4160, 512), (16, 128, 544), (65, 384, 1536),
+                                         (129, 4160, 512), (1025, 1056, 96), (1200, 1100, 32),
+                                         (2049, 520, 512), (1057, 1090, 160), (1024, 1024, 64),
+                                         (16, 128, 544), (65, 384, 1536),
                                          (543, 384, 1536), (1, 256, 1568), (20, 100, 1536)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
@@ -430,10 +433,11 @@ def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
     assert np.all(err <= bound), float((err / bound).max())
 
 
-@pytest.mark.parametrize("rows", [7, 41, 543, 656])
+@pytest.mark.parametrize("rows", [7, 41, 543, 656, 1000, 1030])
 def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
     """Three projections of one input queued in one command run as one launch, their row ranges
-    joined; each output holds the bits of a command of its own."""
+    joined; each output holds the bits of a command of its own (from about 900 rows, on operands split
+    beforehand together and on the direct kernel alone)."""
     rng = np.random.default_rng(rows)
     x = rng.normal(size=(rows, 384)).astype(np.float32)
     sets = [(rng.normal(size=(384, 384)).astype(np.float32), rng.normal(size=384).astype(np.float32))
@@ -460,8 +464,8 @@ def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
         np.testing.assert_allclose(together, ref.linear(x, w, b), atol=2e-4, rtol=5e-5)
 
 
-# the split-operand kernel with both halves of K at once and in turn, and split K at few tiles
-@pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (656, 1152, 512),
+# the direct kernel, the one of operands split beforehand, and split K at few tiles
+@pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (656, 1152, 512), (1100, 1152, 512),
                                          (65, 384, 1536), (1, 256, 1568)])
 def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
     """Operands whose second and third bf16 terms are near their largest (2^-7 and 2^-15 of the
@@ -479,7 +483,8 @@ def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
     assert np.all(np.abs(got - want) <= 3.5e-7 * want), float(np.abs(got / want - 1).max())
 
 
-@pytest.mark.parametrize("rows,cols,k", [(33, 70, 64), (656, 1152, 384), (65, 384, 1536)])
+@pytest.mark.parametrize("rows,cols,k", [(33, 70, 64), (656, 1152, 384), (1100, 1152, 384),
+                                         (65, 384, 1536)])
 @pytest.mark.parametrize("gelu", [False, True])
 def test_non_finite_operands_give_what_fp32_gives(runtime, rows, cols, k, gelu):
     """Infinities and NaN in x, W and the bias: what sums of fp32 products give (infinities where no

@@ -318,7 +318,8 @@ def test_launcher_limits_are_rejected_at_dispatch(runtime, case):
             b.close()
 
 
-@pytest.mark.parametrize("route,rows,k,mib", [("matmul_f32", 5, 1536, 32), ("matmul_f32", 5, 384, 136),
+@pytest.mark.parametrize("route,rows,k,mib", [("matmul_f32", 5, 1536, 32), ("matmul_f32", 5, 384, 32),
+                                              ("matmul_f32", 4096, 384, 136),
                                               ("linear4", 5, 128, 40), ("linear4", 1024, 128, 32)])
 def test_projections_take_the_scratch_they_run_on(runtime, route, rows, k, mib):
     """A runtime's first projection takes the device memory its own kernel works in: 32 MiB of partial
