@@ -298,6 +298,8 @@ hipError_t launch_rms_norm_rope_f32(const NormRopeRows* sets, int count, const f
     const int slots = dim <= 128 ? (sets[i].rows + 1) / 2 : sets[i].rows;
     blocks[i] = static_cast<unsigned>((slots + 3) / 4);
   }
+  // each set is within a launch's 2^32 work items, two may not be
+  if ((static_cast<uint64_t>(blocks[0]) + blocks[1]) * 256 >= (1ull << 32)) return hipErrorNotReady;
   const NormRopeRows& last = sets[count - 1];
   if (dim <= 128)
     rms_norm_rope_f32<true><<<blocks[0] + blocks[1], 256, 0, st>>>(sets[0], last, blocks[0], cos_tab,

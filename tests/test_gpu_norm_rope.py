@@ -211,3 +211,32 @@ def test_add_then_rms_norm_fused_in_one_command(runtime, rows, cols, in_place):
     np.testing.assert_array_equal(outs[0][1], outs[1][1])
     want = ref.rms_norm(x.astype(np.float64) + r, bf16_values(w), 1e-6)
     np.testing.assert_allclose(outs[0][1], want, atol=2e-6, rtol=2e-6)
+
+
+def test_q_and_k_norms_beyond_one_launch(runtime):
+    """q and k rows that each fill a launch's 2^32 work items: too many for the joint launch of both,
+    they run as two. Every 16380 rows are the same and hold the bits of those rows alone."""
+    dim, heads, seq, copies = 8, 4, 4095, 4097
+    rows = heads * seq * copies
+    assert rows == (1 << 26) - 4
+    rng = np.random.default_rng(0)
+    blocks = [rng.normal(size=heads * seq * dim).astype(np.float32) for _ in range(2)]
+    gammas = [runtime.upload(workloads.bf16_words(rng.uniform(0.5, 1.5, dim))) for _ in range(2)]
+
+    def norm_rope(bufs, rows):
+        with runtime.command():
+            for buf, gamma in zip(bufs, gammas):
+                runtime._dispatch("rms_norm", [buf, gamma, buf], threads=rows * 32, group_size=32,
+                                  cols=dim, eps=1e-6)
+                runtime._dispatch("rope", [buf], threads=rows * dim // 2, n=rows * dim // 2,
+                                  heads=heads, seq=seq, dim=dim, theta=1e6)
+
+    small = [runtime.upload(b) for b in blocks]
+    norm_rope(small, heads * seq)
+    large = [runtime.upload(np.tile(b, copies)) for b in blocks]
+    norm_rope(large, rows)
+    for a, b in zip(small, large):
+        want = runtime.read(a, blocks[0].shape)
+        assert (runtime.read(b, (copies, want.size)) == want).all()
+    for b in [*small, *large, *gammas]:
+        b.close()
