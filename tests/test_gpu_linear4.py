@@ -310,3 +310,75 @@ def test_large_batch_beyond_the_fp16_kernels_k(runtime, k):
     err = np.abs(got - x.astype(np.float64) @ w.T)
     bound = 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
     assert np.all(err <= bound), float((err / bound).max())
+
+
+@pytest.mark.parametrize("m", [1024, 1029, 4096])
+@pytest.mark.parametrize("chain", ["norm", "add", "gated", "overwritten", "dense", "longer"])
+def test_row_scales_left_for_large_projections_keep_their_bits(runtime, m, chain):
+    """From 1024 rows a norm, and the first projection of an input, leave the row scales of that input
+    for the projections after them. Queued in one command, every buffer holds the bits of a command
+    for each launch: q, k and v after a norm, alone or with the add before it, or over more rows than
+    they project; gate, up, silu_gate, down; with their input written anew in between; with a dense
+    projection in between, which keeps its partial sums where the scales are. Rows from 2^-20 to 2^10
+    with an eps of 1e-2, so that the normalized rows, and their scales, differ as much."""
+    k, rows = 576, m + 71 if chain == "longer" else m
+    rng = np.random.default_rng(m)
+    x, r = [rng.normal(size=(rows, k)).astype(np.float32)
+            * np.exp2(rng.integers(-20, 11, (rows, 1))).astype(np.float32) for _ in range(2)]
+    z = rng.normal(size=(m, 128)).astype(np.float32) * np.exp2(rng.integers(-8, 9, (m, 1))).astype(np.float32)
+    dense = [rng.normal(size=s).astype(np.float32) for s in ((65, 1536), (384, 1536))]
+    gamma = bf16_words(rng.uniform(0.5, 1.5, k))
+
+    def weights(n, width):
+        return [ref.pack(rng.integers(0, 16, size=(n, width), dtype=np.uint32)),
+                bf16_words(rng.uniform(0.01, 0.2, size=(n, width // 64)) / 8),
+                bf16_words(rng.uniform(-1, 0.1, size=(n, width // 64)) / 8)]
+
+    widths = {"gated": [(640, k), (640, k), (k, 640)], "overwritten": [(256, k), (k, 128), (128, k)]}
+    sets = [weights(*s) for s in widths.get(chain, [(256, k), (128, k), (128, k)])]
+    results = []
+    for separate in (False, True):
+        xb, rb, zb, gb = [runtime.upload(a) for a in (x, r, z, gamma)]
+        wb = [[runtime.upload(a) for a in w] for w in sets]
+        db = [runtime.upload(a) for a in dense] + [runtime.buffer(65 * 384 * 4)]
+        h = runtime.buffer(x.nbytes)
+        outs = [runtime.buffer(m * w[0].shape[0] * 4) for w in sets]
+
+        def project(i, src, dst):
+            n, words = sets[i][0].shape
+            return lambda: runtime._linear4([src, *wb[i], dst], rows=m, cols=n, k=8 * words)
+
+        steps = [lambda: runtime._dispatch("rms_norm", [xb, gb, h], threads=rows * 32, group_size=32,
+                                           cols=k, eps=1e-2)]
+        if chain == "add":
+            steps.insert(0, lambda: runtime._dispatch("add", [xb, rb, xb], threads=x.size, n=x.size))
+        if chain == "gated":
+            steps += [project(0, h, outs[0]), project(1, h, outs[1]),
+                      lambda: runtime._dispatch("silu_gate", outs[:2], threads=m * 640, n=m * 640),
+                      project(2, outs[0], outs[2])]
+        elif chain == "overwritten":
+            steps += [project(0, h, outs[0]), project(1, zb, h), project(2, h, outs[2])]
+        else:
+            steps += [project(i, h, outs[i]) for i in range(3)]
+        if chain == "dense":
+            steps.insert(2, lambda: runtime._dispatch("matmul_f32", db, threads=68 // 4 * 384 * 32,
+                                                      group_size=32, rows=65, cols=384, k=1536))
+        if separate:
+            for step in steps:
+                with runtime.command():
+                    step()
+        else:
+            with runtime.command():
+                for step in steps:
+                    step()
+        results.append([runtime.read(h, x.shape), runtime.read(db[2], (65, 384)),
+                        *(runtime.read(o, (m, w[0].shape[0])) for o, w in zip(outs, sets))])
+        for b in [xb, rb, zb, gb, h, *db, *outs, *(b for w in wb for b in w)]:
+            b.close()
+    for together, alone in zip(*results):
+        np.testing.assert_array_equal(together, alone)
+    if chain != "gated":  # the last projection, of the input as it was by then
+        w = ref.dequantize(*sets[2], k)
+        hd = results[0][0][:m].astype(np.float64)
+        err = np.abs(results[0][4] - hd @ w.T)
+        assert np.all(err <= 2e-6 * (np.abs(hd) @ np.abs(w).T) + 1e-37)

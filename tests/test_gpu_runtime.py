@@ -357,3 +357,89 @@ def test_projections_take_the_scratch_they_run_on(runtime, route, rows, k, mib):
     with HipRuntime() as fresh:
         # small buffers share allocator blocks of up to 2 MiB with the scratch
         assert abs(project(fresh) - (mib << 20)) <= 4 << 20
+
+
+def attentions(runtime, count):
+    """A plan's worth of `count` attention launches over one set of inputs, its outputs and what they
+    should hold."""
+    rng = np.random.default_rng(count)
+    q = rng.normal(size=(1, 64, 2, 32)).astype(np.float32)
+    k, v = [rng.normal(size=(1, 64, 2, 32)).astype(np.float32) for _ in range(2)]
+    lengths = np.array([40], np.uint32)
+    bufs = [runtime.upload(a) for a in (q, k, v, lengths)]
+
+    def plan(key, outs):
+        with runtime._execution_plan(key, bufs + outs) as replayed:
+            if not replayed:
+                for out in outs:
+                    runtime._attention(bufs + [out], tokens=64, seq=64, heads=2, kv_heads=2, dim=32)
+
+    def check(outs):
+        first = runtime.read(outs[0], q.shape)
+        check_f32(first, ref.attention(q, k, v, lengths, bidirectional=False))
+        for out in outs[1:]:
+            np.testing.assert_array_equal(runtime.read(out, q.shape), first)
+        for out in outs:
+            runtime.write(out, np.full(q.shape, np.nan, np.float32))
+
+    return bufs, plan, check, lambda: [runtime.buffer(q.nbytes) for _ in range(count)]
+
+
+@pytest.mark.parametrize("count,graph", [(1, 0), (5, 0), (6, 1), (7, 1)])
+def test_plans_of_six_launches_replay_as_graphs(runtime, count, graph):
+    bufs, plan, check, new = attentions(runtime, count)
+    outs = new()
+    with runtime._workspace():
+        for _ in range(4):
+            with runtime.command():
+                plan(("a", count), outs)
+            check(outs)
+    diag = runtime.diagnostics()
+    assert (diag["plan_hits"], diag["graph_builds"], diag["graph_launches"]) == (3, graph, 3 * graph)
+    for b in bufs + outs:
+        b.close()
+
+
+def test_graph_plan_evicted_while_its_replay_is_queued(runtime):
+    """A plan that has run as a graph, replayed and then evicted by later captures in the same command
+    (the cache holds 4 plans): its launches still run."""
+    bufs, plan, check, new = attentions(runtime, 6)
+    sets = [new() for _ in range(5)]
+    with runtime._workspace():
+        for _ in range(2):
+            with runtime.command():
+                plan(("a",), sets[0])
+            check(sets[0])
+        assert runtime.diagnostics()["graph_launches"] == 1
+        with runtime.command():
+            plan(("a",), sets[0])
+            for i in range(4):
+                plan(("b", i), sets[1 + i])
+        assert runtime.diagnostics()["plan_hits"] == 2
+        for outs in sets:
+            check(outs)
+        with runtime.command():
+            plan(("b", 3), sets[4])
+        check(sets[4])
+        assert runtime.diagnostics()["graph_launches"] == 2
+    for b in [*bufs, *(b for outs in sets for b in outs)]:
+        b.close()
+
+
+def test_graph_plan_over_more_bindings_than_it_keeps(runtime):
+    """A plan keeps the graphs of its last four bindings: a fifth takes the place of the one used least
+    recently, which is built anew when it comes back. Every replay writes its own outputs."""
+    bufs, plan, check, new = attentions(runtime, 6)
+    sets = [new() for _ in range(5)]
+    with runtime._workspace():
+        with runtime.command():
+            plan(("a",), sets[0])
+        check(sets[0])
+        for i, builds in ((0, 1), (1, 2), (2, 3), (3, 4), (0, 4), (4, 5), (0, 5), (1, 6), (4, 6)):
+            with runtime.command():
+                plan(("a",), sets[i])
+            check(sets[i])
+            assert runtime.diagnostics()["graph_builds"] == builds, i
+    assert runtime.diagnostics()["graph_launches"] == 9
+    for b in [*bufs, *(b for outs in sets for b in outs)]:
+        b.close()
