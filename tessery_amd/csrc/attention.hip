@@ -2080,8 +2080,10 @@ static hipError_t launch_attention_f32x3(const AttnArgs& a, bool exact, hipStrea
     default:
       // the sums of P V apart (SEP) take two workgroups per CU where long rows need the three that
       // one sum leaves room for: 67 against 83 us at 8 x 512
-      if (exact || a.S < 64)
+      if (exact)
         attn_f32x3<128, true, true><<<grid, 256, 0, st>>>(x);
+      else if (a.S < 64)
+        attn_f32x3<128, true, false><<<grid, 256, 0, st>>>(x);
       else
         attn_f32x3<128, false, false><<<grid, 256, 0, st>>>(x);
       break;
