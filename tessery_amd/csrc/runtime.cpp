@@ -161,6 +161,7 @@ struct Runtime {
   float* dense_scratch = nullptr;  // split-K partial sums of dense projections, row scales of uint4
   void* dense_planes = nullptr;    // split operands of fp32 projections
   void* planes[2] = {};  // planes of the activations uint4 projections read, and of their output
+  void* wide_planes = nullptr;  // of activations beyond those
   std::vector<Segment> segments;
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_end = nullptr;
@@ -589,8 +590,12 @@ constexpr size_t kDenseScratchFloats = size_t{8} << 20;  // 32 MiB
 // matmul_x3), which is 96 MiB where they are one column of tiles of K = 512.
 constexpr size_t kDensePlanesBytes = size_t{104} << 20;
 // Each of the two planes scratches: 1023 rows (more run on linear4_hilo) of 3072 inputs, Qwen3's
-// widest, in 18.4 MiB. Others go through it in row ranges.
+// widest, in 18.4 MiB.
 constexpr size_t kPlanesBytes = size_t{20} << 20;
+// Wider inputs: 1023 rows of 8192. What exceeds it goes through in row ranges, one after the other,
+// each too few tiles for the chip where the columns are few (1000 x 64 outputs of K = 8192: 100.4 us
+// in three ranges of 20 MiB, 39.1 in one; of K = 4096 43.2 and 23.3).
+constexpr size_t kWidePlanesBytes = size_t{49} << 20;
 
 const RopeTable* rope_of(Runtime* rt, const Params& p) {
   auto it = rt->rope.find(std::make_tuple(p.seq, p.dim, float_bits(p.theta)));
@@ -738,9 +743,13 @@ bool prepare(Runtime* rt, const Op& op) {
         have_scratch(&rt->dense_scratch, sums_bytes) &&
         !tessery::linear4_on_rows(job, rt->dense_scratch, kDenseScratchFloats))
       return true;
-  } else if (!gated4_jobs(op, gated)) {
+  } else if (gated4_jobs(op, gated)) {
+    job = gated[0];
+  } else {
     return true;
   }
+  if (tessery::planes_bytes(job.row1 - job.row0, job.k) > kPlanesBytes)
+    (void)have_scratch(&rt->wide_planes, kWidePlanesBytes);
   (void)have_scratch(&rt->planes[1], kPlanesBytes);
   return have_scratch(&rt->planes[0], kPlanesBytes);
 }
@@ -939,6 +948,7 @@ void mi_destroy(void* runtime) {
   if (rt->dense_planes) (void)hipFree(rt->dense_planes);
   for (void* p : rt->planes)
     if (p) (void)hipFree(p);
+  if (rt->wide_planes) (void)hipFree(rt->wide_planes);
   release_profile_events(rt);
   if (rt->ev_start) (void)hipEventDestroy(rt->ev_start);
   if (rt->ev_end) (void)hipEventDestroy(rt->ev_end);
@@ -1428,8 +1438,14 @@ hipError_t launch_next(Runtime* rt, size_t first, size_t last, size_t* taken, Pa
     if (untouched) pass->scaled = scaled;
     if (keep)
       pass->ready = {j.out, static_cast<uint64_t>(j.row1), static_cast<uint64_t>(j.cols), 1 - slot};
-    return tessery::launch_linear4_rows(p.jobs, p.count, p.gated, planes_scratch(rt, slot),
-                                        prepared, keep, rt->stream);
+    // too wide for a planes scratch: neither prepared nor kept
+    const bool wide =
+        rt->wide_planes && tessery::planes_bytes(j.row1 - j.row0, j.k) > kPlanesBytes;
+    return tessery::launch_linear4_rows(
+        p.jobs, p.count, p.gated,
+        wide ? tessery::PlanesScratch{rt->wide_planes, nullptr, kWidePlanesBytes}
+             : planes_scratch(rt, slot),
+        prepared, keep, rt->stream);
   }
   DenseProjection d;
   if (find_dense(rt, first, last, &d)) {

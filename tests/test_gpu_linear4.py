@@ -382,3 +382,20 @@ def test_row_scales_left_for_large_projections_keep_their_bits(runtime, m, chain
         hd = results[0][0][:m].astype(np.float64)
         err = np.abs(results[0][4] - hd @ w.T)
         assert np.all(err <= 2e-6 * (np.abs(hd) @ np.abs(w).T) + 1e-37)
+
+
+@pytest.mark.parametrize("m,n,k", [(1000, 64, 8192), (1023, 40, 4096), (1056, 72, 8192)])
+def test_wide_inputs_beyond_one_planes_scratch_keep_their_bits(runtime, m, n, k):
+    """Inputs whose split form exceeds the scratch of the usual ones (one range in the wide scratch; the
+    last more than that holds): rows hold the bits of launches of their own, within 2e-6 of
+    sum_k |x| |w| of float64."""
+    x, packed, scales, biases = make(m, m, n, k)
+    got = project(runtime, [x, packed, scales, biases], m, n, k,
+                  out=np.full((m + 1, n), np.nan, np.float32))
+    assert np.isnan(got[m:]).all()
+    for rows in (slice(0, 96), slice(m - 50, m)):
+        alone = project(runtime, [x[rows], packed, scales, biases], len(x[rows]), n, k)
+        np.testing.assert_array_equal(got[:m][rows], alone)
+    w = ref.dequantize(packed, scales, biases, k)
+    err = np.abs(got[:m] - x.astype(np.float64) @ w.T)
+    assert np.all(err <= 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T))

@@ -320,11 +320,12 @@ def test_launcher_limits_are_rejected_at_dispatch(runtime, case):
 
 @pytest.mark.parametrize("route,rows,k,mib", [("matmul_f32", 5, 1536, 32), ("matmul_f32", 5, 384, 32),
                                               ("matmul_f32", 4096, 384, 136),
-                                              ("linear4", 5, 128, 40), ("linear4", 1024, 128, 32)])
+                                              ("linear4", 5, 128, 40), ("linear4", 1024, 128, 32),
+                                              ("linear4", 512, 8192, 89)])
 def test_projections_take_the_scratch_they_run_on(runtime, route, rows, k, mib):
     """A runtime's first projection takes the device memory its own kernel works in: 32 MiB of partial
     sums or row scales, 104 MiB of split operands only for the dense shapes that use them, 40 MiB of
-    split activations only for uint4 ones of under 1024 rows."""
+    split activations only for uint4 ones of under 1024 rows, 49 MiB more for wide ones."""
     import ctypes
 
     from tessery_amd import HipRuntime
