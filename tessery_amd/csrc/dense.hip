@@ -724,15 +724,16 @@ int dense_splits(int rows, int cols, int k, size_t scratch_floats) {
 // Workgroups along K for matmul_x3: 1 from 512 tiles of 64 x 128; from 64 tiles, enough splits of at
 // least two 32-wide chunks for about 768 workgroups; fewer tiles, for about 256 workgroups of at
 // least four chunks (656 x 384 outputs of K = 1536: 17.3 us with 7 to 12 splits, 20.8 with 4, 21.8
-// with 24, and 24.9 on matmul_f32); 0 (the fp32 kernel) where the partial sums do not fit the
+// with 24, and 24.9 on matmul_f32), below K = 1024 of two (64 x 384 outputs of K = 544: 10.0 us, 11.8
+// with four and 10.9 on matmul_f32); 0 (the fp32 kernel) where the partial sums do not fit the
 // scratch or K is short. Every split holds at least one chunk.
 constexpr int kX3WideTiles = 64;  // fewer take eight products, as precise as matmul_f32 in their place
 static int x3_split_count(int rows, int cols, int k, int tiles, size_t scratch_floats) {
   if (tiles >= 512) return 1;
   const int chunks32 = k / 32;
   if (tiles < 1 || chunks32 < (tiles < kX3WideTiles ? 8 : 4)) return 0;
-  int splits = tiles < kX3WideTiles ? std::min(chunks32 / 4, 256 / tiles)
-                          : std::min(chunks32 / 2, (768 + tiles - 1) / tiles);
+  int splits = tiles < kX3WideTiles ? std::min(chunks32 / (chunks32 < 32 ? 2 : 4), 256 / tiles)
+                                    : std::min(chunks32 / 2, (768 + tiles - 1) / tiles);
   const int per = (chunks32 + splits - 1) / splits;
   splits = (chunks32 + per - 1) / per;
   if (splits < 2 || static_cast<size_t>(splits) * rows * cols > scratch_floats) return 0;
@@ -770,10 +771,10 @@ static bool split_shape(const DenseJob& j, size_t planes_bytes) {
 // matmul_direct reads its operands while other workgroups write outputs.
 static bool output_apart(const DenseJob& j) { return j.out != j.a && j.out != j.bt; }
 
-// matmul_direct up to this many tiles of 32 x 32, matmul_planes after split_dense beyond: 1008 tiles
-// (656 x 1536 outputs of K = 384) 19.3 and 20.5 us, 1152 (three times 1024 x 384) 23.2 and 19.3, 1536
-// (1024 x 1536) 27.3 and 21.3.
-constexpr int64_t kDirectTiles = 1024;
+// matmul_direct up to this many tiles of 32 x 32, three a CU, matmul_planes after split_dense beyond: 768
+// tiles (512 x 1536 outputs of K = 384) 16.8 and 19.4 us, 800 (800 x 1024) 20.2 and 18.4, 1024 (1000 x
+// 1024) 20.7 and 18.8; of K = 512 19.5 and 22.2, 23.7 and 21.8, 24.3 and 22.4.
+constexpr int64_t kDirectTiles = 768;
 
 static int64_t direct_tiles(const DenseJob& j) {
   return static_cast<int64_t>((j.row1 - j.row0 + 31) / 32) * ((j.cols + 31) / 32);

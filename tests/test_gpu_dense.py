@@ -397,7 +397,7 @@ def test_plan_replay_graphs_match_eager(monkeypatch, graphs):
                                rtol=5e-5)
 
 
-# Rows and columns at the edges of the 32 x 32 tiles of the direct kernel and, beyond 1024 of those, of
+# Rows and columns at the edges of the 32 x 32 tiles of the direct kernel and, beyond 768 of those, of
 # the 64 x 64 ones of operands split beforehand; K of 1, 2, 3, 5, 12 and 16 chunks (empty and uneven
 # halves); then, past K = 512, split K at few tiles (from 8 chunks) and the shapes that stay on the
 # fp32 kernel.
@@ -405,7 +405,7 @@ def test_plan_replay_graphs_match_eager(monkeypatch, graphs):
                                          (33, 384, 384), (543, 1152, 384), (1000, 384, 384),
                                          (129, 4160, 512), (1025, 1056, 96), (1200, 1100, 32),
                                          (2049, 520, 512), (1057, 1090, 160), (1024, 1024, 64),
-                                         (16, 128, 544), (65, 384, 1536),
+                                         (16, 128, 544), (300, 128, 736), (65, 384, 1536),
                                          (543, 384, 1536), (1, 256, 1568), (20, 100, 1536)])
 @pytest.mark.parametrize("bias", [False, True])
 def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
@@ -436,7 +436,7 @@ def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
 @pytest.mark.parametrize("rows", [7, 41, 543, 656, 1000, 1030])
 def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
     """Three projections of one input queued in one command run as one launch, their row ranges
-    joined; each output holds the bits of a command of its own (from about 900 rows, on operands split
+    joined; each output holds the bits of a command of its own (from about 700 rows, on operands split
     beforehand together and on the direct kernel alone)."""
     rng = np.random.default_rng(rows)
     x = rng.normal(size=(rows, 384)).astype(np.float32)
