@@ -310,11 +310,11 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
 // no partial sums, and q, k and v in one launch. Measured, q, k and v of 1024 rows of 384: 19.3 us, 47.5
 // as three split-K launches with their reductions; of 4096: 36.8 us, 72.0 on matmul_x3.
 //
-// Eight products, all but that of the two smallest terms (below 2^-30 of the whole): nothing is lost
-// against fp32 products. K order: two halves, each with its leading products in one sum and the seven
-// smaller ones in another (only the leading ones round at the magnitude of the result), added at
-// the end. It is the same for every tile shape, so a row's bits depend on no other row and on no
-// projection beside it.
+// Eight products (EXACT), all but that of the two smallest terms (below 2^-30 of the whole): nothing is
+// lost against fp32 products. Shapes for which matmul_x3 takes six (it splits K where this kernel
+// does not) take six here too: 3% of a forward of 4096 tokens. K order: two halves, each with its leading products in one sum and the seven
+// smaller ones (five) in another (only the leading ones round at the magnitude of the result), added at
+// the end. It is the same for every tile shape, so a row's bits depend on no projection beside it.
 constexpr int kDenseStep = 3 * 64 * 8;  // bf16 words of a row tile's k-step
 
 struct SplitArgs {
@@ -392,9 +392,18 @@ __device__ __forceinline__ void store_halves(const PlanesArgs& a, int which, int
   }
 }
 
-// The products of two operands' terms that are taken, the smallest first; the last one leads.
-__device__ constexpr int kTerms[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2},
-                                         {1, 2}, {1, 0}, {0, 1}, {0, 0}};
+// The products of two operands' terms that are taken: the smaller ones, then the leading one.
+template <bool EXACT>
+struct Terms;
+template <>
+struct Terms<true> {
+  static constexpr int n = 8, at[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2},
+                                          {1, 2}, {1, 0}, {0, 1}, {0, 0}};
+};
+template <>
+struct Terms<false> {
+  static constexpr int n = 6, at[6][2] = {{2, 0}, {1, 1}, {0, 2}, {1, 0}, {0, 1}, {0, 0}};
+};
 
 // Tile 64 x 64, 4 wavefronts of 32 x 32 each. Two LDS stages of a 32-input chunk. While a chunk's
 // products run, its wavefront reads the operands of the next one from LDS and copies those of the
@@ -404,9 +413,10 @@ __device__ constexpr int kTerms[8][2] = {{2, 0}, {1, 1}, {2, 1}, {0, 2},
 // which ask L2 for less, or more stages leave too few wavefronts on a CU to hide either: 16384 x
 // 1152 outputs 97 and 194 us, 130 with three stages, against 94. Workgroups are numbered so that
 // an XCD takes all columns of a row tile in turn, from its own L2.
-template <bool GELU>
+template <bool GELU, bool EXACT>
 __global__ __launch_bounds__(256, 3) void matmul_planes(PlanesArgs a, int row_tiles,
                                                         int col_tiles) {
+  using T = Terms<EXACT>;
   constexpr int STAGE = 24 * 512;  // bf16 words: 12 KiB of x, then 12 KiB of weights
   constexpr int COPIES = 6, READS = 12;
   __shared__ __attribute__((aligned(1024))) uint16_t mem[2 * STAGE];
@@ -467,11 +477,11 @@ __global__ __launch_bounds__(256, 3) void matmul_planes(PlanesArgs a, int row_ti
     stage_barrier();
     const bool more = step + 2 < chunks;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 2 * T::n; ++i) {
       const int ks = i & 1, t = i >> 1;
-      floatx16& c = t < 7 ? lo : hi;
-      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][kTerms[t][0]], now.y[ks][kTerms[t][1]],
-                                                  c, 0, 0, 0);
+      floatx16& c = t < T::n - 1 ? lo : hi;
+      c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(now.x[ks][T::at[t][0]], now.y[ks][T::at[t][1]], c,
+                                                  0, 0, 0);
       if (i < READS) read(next, i, buf ^ 1);  // stale data after the last chunk, unused
       if (more && i < 2 * COPIES && (i & 1)) copy(i >> 1, buf, step + 2);
       __builtin_amdgcn_sched_barrier(0);
@@ -503,8 +513,9 @@ __global__ __launch_bounds__(256, 3) void matmul_planes(PlanesArgs a, int row_ti
 // and matmul_planes, and matmul_f32 with its reduction: 24 x 384 outputs of K = 384 7.7, 11.6 and 8.8
 // us, 128 x 1536 8.3, 16.3 and 11.3, 64 x 512 of K = 512 9.1, 14.5 and 10.3; q, k and v of 128 rows
 // 8.5, 15.2 and 29.4.
-template <bool GELU>
+template <bool GELU, bool EXACT>
 __global__ __launch_bounds__(128) void matmul_direct(PlanesArgs a) {
+  using T = Terms<EXACT>;
   constexpr int DEPTH = 2;  // chunks loaded ahead
   __shared__ __attribute__((aligned(16))) float sums[4 * 64 * 4];
   int ct = blockIdx.y, which = 0;
@@ -554,11 +565,11 @@ __global__ __launch_bounds__(128) void matmul_direct(PlanesArgs a) {
   };
   auto multiply = [&](const Operands& o) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < 2 * T::n; ++i) {
       const int ks = i & 1, t = i >> 1;
-      floatx16& sum = t < 7 ? lo : hi;
-      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.x[ks][kTerms[t][0]], o.w[ks][kTerms[t][1]],
-                                                    sum, 0, 0, 0);
+      floatx16& sum = t < T::n - 1 ? lo : hi;
+      sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(o.x[ks][T::at[t][0]], o.w[ks][T::at[t][1]], sum,
+                                                    0, 0, 0);
     }
   };
   if (begin < end) {
@@ -576,9 +587,9 @@ __global__ __launch_bounds__(128) void matmul_direct(PlanesArgs a) {
         multiply(now[i & 1]);
         split(now[(i + 1) & 1], ring[(i + 1) % DEPTH]);
 #pragma unroll
-        for (int m = 0; m < 16; ++m) {  // an MFMA, then the splitting that fits beside it
+        for (int m = 0; m < 2 * T::n; ++m) {  // an MFMA, then the splitting that fits beside it
           __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x2, 11, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, 176 / (2 * T::n), 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -740,6 +751,7 @@ static int x3_split_count(int rows, int cols, int k, int tiles, size_t scratch_f
   return splits;
 }
 
+template <bool EXACT>
 static void run_planes(const PlanesArgs& a, bool gelu, hipStream_t st) {
   const int row_tiles = (a.row1 - a.row0 + 63) / 64;
   int col_tiles = 0;
@@ -747,9 +759,20 @@ static void run_planes(const PlanesArgs& a, bool gelu, hipStream_t st) {
   const unsigned grid = 8u * static_cast<unsigned>((row_tiles + 7) / 8) *
                         static_cast<unsigned>(col_tiles);
   if (gelu)
-    matmul_planes<true><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
+    matmul_planes<true, EXACT><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
   else
-    matmul_planes<false><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
+    matmul_planes<false, EXACT><<<grid, 256, 0, st>>>(a, row_tiles, col_tiles);
+}
+
+template <bool EXACT>
+static void run_direct(const PlanesArgs& a, bool gelu, hipStream_t st) {
+  unsigned col_tiles = 0;
+  for (int i = 0; i < a.count; ++i) col_tiles += static_cast<unsigned>((a.set[i].cols + 31) / 32);
+  const dim3 grid(static_cast<unsigned>((a.row1 - a.row0 + 31) / 32), col_tiles);
+  if (gelu)
+    matmul_direct<true, EXACT><<<grid, 128, 0, st>>>(a);
+  else
+    matmul_direct<false, EXACT><<<grid, 128, 0, st>>>(a);
 }
 
 static size_t dense_planes_bytes(int64_t rows, int k) {
@@ -788,14 +811,25 @@ bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
   return split_shape(j, scratch.planes_bytes) && (scratch.planes || output_apart(j));
 }
 
+// The shapes that matmul_x3 takes on six products, K split (x3_split_count).
+static bool x3_takes_six(const DenseJob& j) {
+  return j.cols % 128 == 0 && j.k >= 128 &&
+         static_cast<int64_t>((j.row1 - j.row0 + kX3Rows - 1) / kX3Rows) * (j.cols / 128) >=
+             kX3WideTiles;
+}
+
+bool matmul_joins(const DenseJob& a, const DenseJob& b, const DenseScratch& scratch) {
+  return b.a == a.a && b.row0 == a.row0 && b.row1 == a.row1 && b.k == a.k &&
+         matmul_on_planes(a, scratch) && matmul_on_planes(b, scratch) &&
+         x3_takes_six(a) == x3_takes_six(b);
+}
+
 hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
                                 const DenseScratch& scratch, hipStream_t st) {
   if (count < 1 || count > 3) return hipErrorInvalidValue;
   const DenseJob& j = jobs[0];
   for (int i = 0; i < count; ++i)
-    if (jobs[i].a != j.a || jobs[i].row0 != j.row0 || jobs[i].row1 != j.row1 ||
-        jobs[i].k != j.k || !matmul_on_planes(jobs[i], scratch))
-      return hipErrorInvalidValue;
+    if (!matmul_joins(j, jobs[i], scratch)) return hipErrorInvalidValue;
   if (j.row1 <= j.row0) return hipSuccess;
   const int rows = j.row1 - j.row0;
   PlanesArgs p{};
@@ -804,23 +838,19 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
   p.row1 = j.row1;
   p.k = j.k;
   p.count = count;
-  int wtiles = 0, columns = 0;
+  int wtiles = 0;
   int64_t tiles = 0;
   bool direct = true;
+  const bool exact = !x3_takes_six(j);
   for (int i = 0; i < count; ++i) {
     p.set[i] = PlanesSet{jobs[i].bt, jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
     wtiles += (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles
-    columns += (jobs[i].cols + 31) / 32;
     tiles += direct_tiles(jobs[i]);
     direct = direct && output_apart(jobs[i]);
   }
   const int xtiles = (rows + 31) / 32;
   if (!scratch.planes || (direct && tiles <= kDirectTiles)) {
-    const dim3 grid(static_cast<unsigned>(xtiles), static_cast<unsigned>(columns));
-    if (gelu)
-      matmul_direct<true><<<grid, 128, 0, st>>>(p);
-    else
-      matmul_direct<false><<<grid, 128, 0, st>>>(p);
+    exact ? run_direct<true>(p, gelu, st) : run_direct<false>(p, gelu, st);
     return hipGetLastError();
   }
   // every job fits the scratch with three times its own weights, so three of equal width do
@@ -847,7 +877,7 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
     s.tiles[i + 1] = (jobs[i].cols + 63) / 64 * 2;
   }
   split_dense<<<dim3(static_cast<unsigned>(xtiles + wtiles), (j.k + 63) / 64), 256, 0, st>>>(s);
-  run_planes(p, gelu, st);
+  exact ? run_planes<true>(p, gelu, st) : run_planes<false>(p, gelu, st);
   return hipGetLastError();
 }
 

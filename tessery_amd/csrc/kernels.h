@@ -173,9 +173,11 @@ hipError_t launch_matmul_f32(const DenseJob& job, bool gelu, const DenseScratch&
 // Whether the job, alone or with two more like it, is one that planes_bytes of split operands serve best.
 bool matmul_reads_planes(const DenseJob& job, size_t planes_bytes);
 // Whether launch_matmul_f32 runs the job on the split-bf16 kernels of K <= 512 (scratch.planes may be
-// null), whose results depend neither on the rows of the launch nor on the projections beside it.
+// null), whose results do not depend on the projections beside it.
 bool matmul_on_planes(const DenseJob& job, const DenseScratch& scratch);
-// One to three such projections of the same rows of one a, with the bits of separate launches.
+// Whether b may share a's launch_matmul_planes: the same rows of one x and the same products.
+bool matmul_joins(const DenseJob& a, const DenseJob& b, const DenseScratch& scratch);
+// One to three such projections, with the bits of separate launches.
 hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
                                 const DenseScratch& scratch, hipStream_t st);
 // x[i] += bias[i % cols] (kernels.metal:376-379).

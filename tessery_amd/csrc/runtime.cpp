@@ -1364,9 +1364,8 @@ bool find_dense(Runtime* rt, size_t first, size_t last, DenseProjection* p) {
   while (p->count < 3 && p->end < last && tessery::matmul_on_planes(lead, scratch)) {
     tessery::DenseJob j;
     size_t end;
-    if (!dense_run(rt, p->end, last, &j, &end) || !tessery::matmul_on_planes(j, scratch) ||
-        j.a != lead.a || j.k != lead.k ||
-        j.row0 != lead.row0 || j.row1 != lead.row1 || j.out == j.a)
+    if (!dense_run(rt, p->end, last, &j, &end) || !tessery::matmul_joins(lead, j, scratch) ||
+        j.out == j.a)
       break;
     // no output is an input or output of another projection of the launch
     bool apart = true;

@@ -433,7 +433,7 @@ def test_split_operand_projection_at_its_edges(runtime, rows, cols, k, bias):
     assert np.all(err <= bound), float((err / bound).max())
 
 
-@pytest.mark.parametrize("rows", [7, 41, 543, 656, 1000, 1030])
+@pytest.mark.parametrize("rows", [7, 41, 543, 656, 1000, 1030, 1400])
 def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
     """Three projections of one input queued in one command run as one launch, their row ranges
     joined; each output holds the bits of a command of its own (from about 700 rows, on operands split
@@ -464,8 +464,9 @@ def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
         np.testing.assert_allclose(together, ref.linear(x, w, b), atol=2e-4, rtol=5e-5)
 
 
-# the direct kernel, the one of operands split beforehand, and split K at few tiles
-@pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (656, 1152, 512), (1100, 1152, 512),
+# the direct kernel, the one of operands split beforehand, and split K at few tiles: the shapes that fp32
+# MFMA served (from 64 tiles of 64 x 128 on, whole columns of them take six products, as ever)
+@pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (600, 1120, 512), (1100, 1160, 512),
                                          (65, 384, 1536), (1, 256, 1568)])
 def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
     """Operands whose second and third bf16 terms are near their largest (2^-7 and 2^-15 of the
