@@ -1983,9 +1983,9 @@ hipError_t launch_attention_scalar(const AttnArgs& a, hipStream_t st) {
   const unsigned grid = static_cast<unsigned>(a.B * a.S * a.H);
   if (!grid) return hipSuccess;
   // fp32 rows of a head size that attn_f32x3 tiles (32, 64, 128) run there from 16 keys on:
-  // attn_scalar's keys are a serial chain of wave reductions, about 1.25 us each whatever the
-  // batch (24 tokens of 16 heads 30.9 against 8.0 us, 16 x 41 tokens of 12 heads 39.6 against
-  // 9.1 us per launch). Under 16 keys the chain is as short as the tile's latency.
+  // attn_scalar's keys are a serial chain of wave reductions, 0.7 us each and more with the batch
+  // (24 tokens of 16 heads 19.0 against 7.4 us per launch, 16 x 40 tokens of 12 heads 28.8 against
+  // 5.2; 16 keys 13.3 and 6.0). Under 16 keys the chain is as short as the tile's latency.
   if (a.S >= kX3MinKeys && !a.in_f16 && !a.out_f16 &&
       attention_f32x3_fits(a.B, a.S, a.H, a.KV, a.D) &&
       attention_f32_fits(a.B, a.S, a.H, a.KV))

@@ -212,10 +212,12 @@ struct Plan {
 };
 
 constexpr size_t kPlanGraphs = 4;
-// A plan of fewer launches is replayed launch by launch: starting a graph costs more than its
-// launches save. Measured per replay, as a graph and directly: 5 launches of short attention 55.9 and
-// 50.0 us, of a 32 x 464 batch 242.5 and 234.5, 4 of projection and attention 162 and 155; but 10 of a
-// decoder layer 87.8 and 96.5, 9 (13 kernels) of an encoder layer 122.2 and 125.4.
+// A plan of fewer launches is replayed launch by launch: up to five launches start at once, the sixth
+// costs 10 to 17 us more, and from there on a graph costs less. Measured per replay, as a graph and
+// directly: attention of one 24-token query 4 launches 58.8 and 45.6 us, 5 62.0 and 51.5, 6 66.6 and
+// 68.8, 7 73.4 and 76.9, 9 89.0 and 94.3; projection and attention of 24 tokens 4 launches 84.7 and
+// 72.6, 6 109.6 and 111.5; of a 32 x 464 batch, attention 5 launches 490.6 and 485.6, 6 610.7 and 609.9;
+// 10 launches of a decoder layer 87.8 and 96.5.
 constexpr size_t kGraphLaunches = 6;
 
 inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
