@@ -399,3 +399,18 @@ def test_wide_inputs_beyond_one_planes_scratch_keep_their_bits(runtime, m, n, k)
     w = ref.dequantize(packed, scales, biases, k)
     err = np.abs(got[:m] - x.astype(np.float64) @ w.T)
     assert np.all(err <= 2e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T))
+
+
+@pytest.mark.parametrize("m", [24, 300, 700])
+def test_groups_without_scale(runtime, m):
+    """Scale 0, with and without a bias (a group of equal or zero weights): z is 0 or 15, and the bias
+    alone counts."""
+    n, k = 1056, 448
+    x, packed, scales, biases = make(m, m, n, k)
+    scales[::2, 1:4] = 0
+    scales[1::3, 2] = 0x8000
+    biases[::4, 1:3] = 0
+    got = project(runtime, [x, packed, scales, biases], m, n, k)
+    w = ref.dequantize(packed, scales, biases, k)
+    err = np.abs(got - x.astype(np.float64) @ w.T)
+    assert np.all(err <= 1e-6 * (np.abs(x).astype(np.float64) @ np.abs(w).T))
