@@ -811,17 +811,17 @@ bool matmul_on_planes(const DenseJob& j, const DenseScratch& scratch) {
   return split_shape(j, scratch.planes_bytes) && (scratch.planes || output_apart(j));
 }
 
-// The shapes that matmul_x3 takes on six products, K split (x3_split_count).
-static bool x3_takes_six(const DenseJob& j) {
-  return j.cols % 128 == 0 && j.k >= 128 &&
-         static_cast<int64_t>((j.row1 - j.row0 + kX3Rows - 1) / kX3Rows) * (j.cols / 128) >=
-             kX3WideTiles;
+// The shapes (under 512 tiles) that matmul_x3 would take on six products, K split.
+static bool x3_takes_six(const DenseJob& j, const DenseScratch& scratch) {
+  const int rows = j.row1 - j.row0, tiles = ((rows + kX3Rows - 1) / kX3Rows) * (j.cols / 128);
+  return j.cols % 128 == 0 && tiles >= kX3WideTiles &&
+         x3_split_count(rows, j.cols, j.k, tiles, scratch.sums_floats) > 0;
 }
 
 bool matmul_joins(const DenseJob& a, const DenseJob& b, const DenseScratch& scratch) {
   return b.a == a.a && b.row0 == a.row0 && b.row1 == a.row1 && b.k == a.k &&
          matmul_on_planes(a, scratch) && matmul_on_planes(b, scratch) &&
-         x3_takes_six(a) == x3_takes_six(b);
+         x3_takes_six(a, scratch) == x3_takes_six(b, scratch);
 }
 
 hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
@@ -841,7 +841,7 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
   int wtiles = 0;
   int64_t tiles = 0;
   bool direct = true;
-  const bool exact = !x3_takes_six(j);
+  const bool exact = !x3_takes_six(j, scratch);
   for (int i = 0; i < count; ++i) {
     p.set[i] = PlanesSet{jobs[i].bt, jobs[i].bias, jobs[i].out, jobs[i].cols, wtiles};
     wtiles += (jobs[i].cols + 63) / 64 * 2;  // whole 64-column tiles

@@ -465,9 +465,10 @@ def test_dense_projections_beside_each_other_keep_their_bits(runtime, rows):
 
 
 # the direct kernel, the one of operands split beforehand, and split K at few tiles: the shapes that fp32
-# MFMA served (from 64 tiles of 64 x 128 on, whole columns of them take six products, as ever)
+# MFMA served (from 64 tiles of 64 x 128 on, whole columns of them take six products, as ever, but where
+# the partial sums of a split K exceed the scratch: the last one)
 @pytest.mark.parametrize("rows,cols,k", [(33, 64, 64), (65, 384, 384), (600, 1120, 512), (1100, 1160, 512),
-                                         (65, 384, 1536), (1, 256, 1568)])
+                                         (65, 384, 1536), (1, 256, 1568), (1856, 1536, 384)])
 def test_split_products_keep_what_fp32_products_keep(runtime, rows, cols, k):
     """Operands whose second and third bf16 terms are near their largest (2^-7 and 2^-15 of the
     first), all of one sign: the products of those terms add up to 2^-21 of the result, and only the
