@@ -165,20 +165,20 @@ __global__ __launch_bounds__(256) void matmul_f32(const float* __restrict__ a,
     }
 }
 
-// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are split
-// exactly into three bf16 planes each (split3x8) and every fp32 product is taken as the six terms
-// b_i c_j with i + j <= 4, or (EXACT) the eight with i + j <= 5, on v_mfma_f32_32x32x16_bf16 in fp32
-// (the bf16 rate is 16x the fp32 one, so six products cost well under half the fp32 instructions;
-// what they leave out is at most 2^-21 of the product, eight 2^-30, and EXACT sums the leading products
-// apart from the others, so that only they round at the magnitude of the result). Tile 64 rows x 128 columns; wavefront w
-// owns rows 32 (w >> 1) .. +31 and columns 64 (w & 1) .. +63 (two 32x32 tiles). Per 32-wide K chunk
-// every thread loads 8 floats of one x row and 16 of one weight row into registers (one chunk
-// ahead), splits them after the barrier that retires the previous chunk's reads, and stores the
-// three planes to LDS as rows of 64 bytes (four 16-byte chunks, chunk c of row r at
-// c ^ ((r >> 1) & 3): conflict-free for the 16-lane reads and the 8-lane writes on gfx950). As in
-// matmul_f32, each 32-wide chunk's products form a partial sum added to the total (the chunk32
-// order), and the bias and GELU are applied the same way. Rows past row1 read row0 and are never
-// stored.
+// matmul_x3<BIAS, GELU>: the same product on bf16 MFMA (K % 32 == 0, N % 128 == 0): a and bt are
+// split exactly into three bf16 planes each (split3x8) and every fp32 product is taken as the six
+// terms b_i c_j with i + j <= 4, or (EXACT) the eight with i + j <= 5, on v_mfma_f32_32x32x16_bf16
+// in fp32 (the bf16 rate is 16x the fp32 one, so six products cost well under half the fp32
+// instructions; what they leave out is at most 2^-21 of the product, eight 2^-30, and EXACT sums
+// the leading products apart from the others, so that only they round at the magnitude of the
+// result). Tile 64 rows x 128 columns; wavefront w owns rows 32 (w >> 1) .. +31 and columns 64 (w &
+// 1) .. +63 (two 32x32 tiles). Per 32-wide K chunk every thread loads 8 floats of one x row and 16
+// of one weight row into registers (one chunk ahead), splits them after the barrier that retires
+// the previous chunk's reads, and stores the three planes to LDS as rows of 64 bytes (four 16-byte
+// chunks, chunk c of row r at c ^ ((r >> 1) & 3): conflict-free for the 16-lane reads and the
+// 8-lane writes on gfx950). As in matmul_f32, each 32-wide chunk's products form a partial sum
+// added to the total (the chunk32 order), and the bias and GELU are applied the same way. Rows past
+// row1 read row0 and are never stored.
 constexpr int kX3Rows = 64;
 
 __device__ __forceinline__ int x3sw(int row) { return (row >> 1) & 3; }
@@ -307,14 +307,15 @@ __global__ __launch_bounds__(256, 3) void matmul_x3(const float* __restrict__ a,
 // [row tile of 32][k-step of 16][term][lane][8], lane = row % 32 + 32 h holding inputs
 // 16 step + 8 h .. + 7. matmul_planes then only copies operands to LDS (global_load_lds_dwordx4:
 // whole KiB pieces, read back by lane, no bank conflicts) and multiplies, all of K in one workgroup:
-// no partial sums, and q, k and v in one launch. Measured, q, k and v of 1024 rows of 384: 19.3 us, 47.5
-// as three split-K launches with their reductions; of 4096: 36.8 us, 72.0 on matmul_x3.
+// no partial sums, and q, k and v in one launch. Measured, q, k and v of 1024 rows of 384: 19.3 us,
+// 47.5 as three split-K launches with their reductions; of 4096: 36.8 us, 72.0 on matmul_x3.
 //
-// Eight products (EXACT), all but that of the two smallest terms (below 2^-30 of the whole): nothing is
-// lost against fp32 products. Shapes for which matmul_x3 takes six (it splits K where this kernel
-// does not) take six here too: 3% of a forward of 4096 tokens. K order: two halves, each with its leading products in one sum and the seven
-// smaller ones (five) in another (only the leading ones round at the magnitude of the result), added at
-// the end. It is the same for every tile shape, so a row's bits depend on no projection beside it.
+// Eight products (EXACT), all but that of the two smallest terms (below 2^-30 of the whole): nothing
+// is lost against fp32 products. Shapes that matmul_x3 would take on six products, K split, take six
+// here too (eight cost a forward of 4096 tokens 3%). K order: two halves, each with its leading
+// products in one sum and the smaller ones in another (only the leading ones round at the magnitude
+// of the result), added at the end. It is the same for every tile shape, so a row's bits depend on
+// no projection beside it.
 constexpr int kDenseStep = 3 * 64 * 8;  // bf16 words of a row tile's k-step
 
 struct SplitArgs {
@@ -408,9 +409,8 @@ struct Terms<false> {
 // Tile 64 x 64, 4 wavefronts of 32 x 32 each. Two LDS stages of a 32-input chunk. While a chunk's
 // products run, its wavefront reads the operands of the next one from LDS and copies those of the
 // one after, one instruction between two products (issued together they cost as much as the
-// products). Bound: few tiles, the issue and latency of a chunk's copies; many, L2 (13 TB/s at 16384
-// rows). Tiles of 64 x 128 and 128 x 128,
-// which ask L2 for less, or more stages leave too few wavefronts on a CU to hide either: 16384 x
+// products). Bound: L2 (13 TB/s for q, k and v of 4096 rows). Tiles of 64 x 128 and 128 x 128, which
+// ask it for less, or more stages leave too few wavefronts on a CU to hide a chunk's latency: 16384 x
 // 1152 outputs 97 and 194 us, 130 with three stages, against 94. Workgroups are numbered so that
 // an XCD takes all columns of a row tile in turn, from its own L2.
 template <bool GELU, bool EXACT>
@@ -881,6 +881,21 @@ hipError_t launch_matmul_planes(const DenseJob* jobs, int count, bool gelu,
   return hipGetLastError();
 }
 
+// again: results that aren't finite are made again (split operands in place of fp32 MFMA).
+static void run_reduce(const DenseJob& j, bool gelu, const float* part, int splits, bool again,
+                       hipStream_t st) {
+  const int rows = j.row1 - j.row0;
+  const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * j.cols + 255) / 256);
+  const float* const a = again ? j.a : nullptr;
+  auto run = [&](auto kernel) {
+    kernel<<<blocks, 256, 0, st>>>(part, j.bias, j.out, j.row0, rows, j.cols, splits, a, j.bt, j.k);
+  };
+  if (j.bias)
+    gelu ? run(dense_reduce<true, true>) : run(dense_reduce<true, false>);
+  else
+    gelu ? run(dense_reduce<false, true>) : run(dense_reduce<false, false>);
+}
+
 hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& dense,
                              hipStream_t st) {
   if (j.row1 <= j.row0 || j.cols <= 0) return hipSuccess;
@@ -902,12 +917,14 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
   if (x3_splits == 1) {
     dim3 grid((rows + kX3Rows - 1) / kX3Rows, cols / 128);
     if (bias && gelu)
-      matmul_x3<true, true, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
+      matmul_x3<true, true, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols,
+                                                             k, 0);
     else if (bias)
-      matmul_x3<true, false, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols, k, 0);
+      matmul_x3<true, false, false, false><<<grid, 256, 0, st>>>(a, bt, bias, out, row0, row1, cols,
+                                                             k, 0);
     else if (gelu)
-      matmul_x3<false, true, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols, k,
-                                                          0);
+      matmul_x3<false, true, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols,
+                                                             k, 0);
     else
       matmul_x3<false, false, false, false><<<grid, 256, 0, st>>>(a, bt, nullptr, out, row0, row1, cols,
                                                            k, 0);
@@ -922,20 +939,7 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
     else
       matmul_x3<false, false, true, false><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0,
                                                                  row1, cols, k, per);
-    const float* const again = x3_tiles < kX3WideTiles ? a : nullptr;
-    const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * cols + 255) / 256);
-    if (bias && gelu)
-      dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols,
-                                                       x3_splits, again, bt, k);
-    else if (bias)
-      dense_reduce<true, false><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols,
-                                                       x3_splits, again, bt, k);
-    else if (gelu)
-      dense_reduce<false, true><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols,
-                                                       x3_splits, again, bt, k);
-    else
-      dense_reduce<false, false><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols,
-                                                       x3_splits, again, bt, k);
+    run_reduce(j, gelu, scratch, x3_splits, x3_tiles < kX3WideTiles, st);
     return hipGetLastError();
   }
   const int splits = scratch ? dense_splits(rows, cols, k, scratch_floats) : 1;
@@ -945,19 +949,7 @@ hipError_t launch_matmul_f32(const DenseJob& j, bool gelu, const DenseScratch& d
     dim3 grid((rows + kDenseRows - 1) / kDenseRows, (cols + 127) / 128, splits);
     matmul_f32<false, false, true><<<grid, 256, 0, st>>>(a, bt, nullptr, scratch, row0, row1,
                                                          cols, k, per);
-    const unsigned blocks = static_cast<unsigned>((static_cast<size_t>(rows) * cols + 255) / 256);
-    if (bias && gelu)
-      dense_reduce<true, true><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits, nullptr, nullptr,
-                                                       0);
-    else if (bias)
-      dense_reduce<true, false><<<blocks, 256, 0, st>>>(scratch, bias, out, row0, rows, cols, splits, nullptr, nullptr,
-                                                       0);
-    else if (gelu)
-      dense_reduce<false, true><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits, nullptr, nullptr,
-                                                       0);
-    else
-      dense_reduce<false, false><<<blocks, 256, 0, st>>>(scratch, nullptr, out, row0, rows, cols, splits, nullptr, nullptr,
-                                                       0);
+    run_reduce(j, gelu, scratch, splits, false, st);
     return hipGetLastError();
   }
   dim3 grid((rows + kDenseRows - 1) / kDenseRows, (cols + 127) / 128);
